@@ -10,8 +10,8 @@
 // and LayerNorm epilogues then work on 16-byte (fp32) / 8-byte (fp16)
 // vectors along the row.
 //
-// Block tile BM x BN (256x256 with 8 waves, 128x128 with 4, 64x64 with 1),
-// K-step BK with STAGES LDS buffers.  When K is a multiple of BK the K-tiles
+// Block tile BM x BN (256x256 with 8 waves, 128x128 with 4 or 8, 128x64 with 8,
+// 64x64 with 4; gemm_dispatch picks), K-step BK with STAGES LDS buffers.  When K is a multiple of BK the K-tiles
 // are copied global -> LDS with global_load_lds_dwordx4 (no register
 // staging), STAGES-1 tiles in flight, one vmcnt wait + barrier per K-step;
 // otherwise a register-staged path with zero fill handles the K tail.  LDS
@@ -19,8 +19,8 @@
 // the copies are bank-conflict free on gfx950's 64-bank LDS.  Block ids are
 // remapped so that the tiles of one XCD (workgroups are dealt round-robin
 // over the 8 XCDs) form a compact group of output tiles sharing A rows and
-// W rows in that XCD's L2.  Whole 256x256 tiles (M, N multiples of 256, K of
-// 128) run the ping-pong K loop instead (Mainloop::run_pingpong): the two
+// W rows in that XCD's L2.  256x256 tiles (M and N at least 256, K a multiple
+// of 128) run the ping-pong K loop instead (Mainloop::run_pingpong): the two
 // waves of each SIMD alternate between a phase of LDS reads and copies and a
 // phase of MFMAs only, so one of them always feeds the matrix core.
 #include "tk_attn_tile.hpp"
@@ -98,6 +98,7 @@ __device__ __forceinline__ void wait_lgkm0() {
 // Raw buffer resource for buffer_load ... lds: base address, no stride, no
 // range limit (the callers copy whole tiles only), gfx9 data format word.
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ i32x4 raw_buffer_rsrc(const void* base) {
   const uint64_t b = (uint64_t)base;
   return i32x4{(int32_t)__builtin_amdgcn_readfirstlane((uint32_t)b),
@@ -597,11 +598,15 @@ struct Mainloop {
 // Tile configuration: block tile BM x BN, wave grid WAVES_M x WAVES_N, and
 // for the direct-copy path the K step and number of LDS stages.  The staged
 // (K-tail) path always runs K step 64 with two stages.
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int BK_, int STAGES_, bool PP_ = false>
+// SHIFT (ping-pong tiles only): M and N need not be multiples of the tile; see
+// gemm_kernel.
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int BK_, int STAGES_, bool PP_ = false, bool SHIFT_ = false>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int BK = BK_, STAGES = STAGES_;
   static constexpr bool PP = PP_;
+  static constexpr bool SHIFT = SHIFT_;
+  static_assert(PP_ || !SHIFT_, "shifted edge tiles: ping-pong loop");
   static constexpr int NT = 64 * WAVES_M_ * WAVES_N_;
   template <bool DIRECT>
   using ML = Mainloop<BM, BN, WAVES_M, WAVES_N, DIRECT ? BK : 64, DIRECT ? STAGES : 2, DIRECT, 0, PP && DIRECT>;
@@ -632,9 +637,11 @@ constexpr int kEpiResidRows = 3;
 // rounding.  The caller has made the main-loop LDS free (every read of the
 // K-tile stages complete).  WHOLE: the tile lies inside M x N, the output rows
 // take 16-byte stores and a given bias 16-byte loads (no bounds tests).
-template <class ML, int WAVES_M, int EPI, bool WHOLE>
+// SHIFT: rows below m_lo and columns below n_lo belong to another tile and are
+// not stored.
+template <class ML, int WAVES_M, int EPI, bool WHOLE, bool SHIFT>
 __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
-                                               int n0, f16* smem) {
+                                               int n0, f16* smem, int m_lo, int n_lo) {
   constexpr int WM = ML::WM, WN = ML::WN, FM = ML::FM, FN = ML::FN, NW = ML::NW;
   constexpr int ROWB = WN * 2;
   constexpr int CPR = ROWB / 16;
@@ -691,7 +698,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
       const int row = idx / CPR, ch = idx % CPR;
       const int m = mw + jb * 32 + row;
       const int n = nw + ch * EPC;
-      if (WHOLE || (m < p.M && n < p.N)) {
+      if (SHIFT ? (m >= m_lo && n >= n_lo) : (WHOLE || (m < p.M && n < p.N))) {
         const f16x8 d = *reinterpret_cast<const f16x8*>(region + epi_off<CPR>(row, ch));
         f16* cr = reinterpret_cast<f16*>(p.c) + (int64_t)m * p.ldc + n;
         if (WHOLE || (p.vec && n + 7 < p.N)) {
@@ -715,10 +722,22 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
 // make the compiler's wait for it also wait for those (the vector memory
 // counter retires in order).  Then the prefetch, then the passes with their
 // kPfStores output stores, all of which may stay in flight into the next tile.
+// SHIFT: rows below m_lo and columns below n_lo are not stored; their stores
+// are issued all the same (the count of instructions in flight must not
+// depend on the tile), to an offset past the buffer's range, which drops them.
 constexpr int kPfStores = 16;
-template <class ML, int WAVES_M, int EPI>
+constexpr uint32_t kDropOffset = 0x80000000u;  // past every range that tile_store_rsrc gives
+
+// Buffer over output tile rows: offsets below 2^31 (the dispatch checks that a
+// tile's rows fit) are stored, kDropOffset is out of range.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_store_rsrc(void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
+}
+
+template <class ML, int WAVES_M, int EPI, bool SHIFT>
 __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
-                                                  int n0, f16* smem, bool has_next, int next_m0, int next_n0) {
+                                                  int n0, f16* smem, bool has_next, int next_m0, int next_n0,
+                                                  int m_lo, int n_lo) {
   constexpr int WM = ML::WM, WN = ML::WN, FM = ML::FM, FN = ML::FN;
   constexpr int ROWB = WN * 2;
   constexpr int CPR = ROWB / 16;
@@ -772,7 +791,14 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
       const int m = mw + jb * 32 + row;
       const int n = nw + ch * EPC;
       const f16x8 d = *reinterpret_cast<const f16x8*>(region + epi_off<CPR>(row, ch));
-      *reinterpret_cast<f16x8*>(reinterpret_cast<f16*>(p.c) + (int64_t)m * p.ldc + n) = d;
+      if constexpr (SHIFT) {
+        const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 2) + (uint32_t)(n - n0) * 2;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d),
+                                               tile_store_rsrc(reinterpret_cast<f16*>(p.c) + (int64_t)m0 * p.ldc + n0),
+                                               m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
+      } else {
+        *reinterpret_cast<f16x8*>(reinterpret_cast<f16*>(p.c) + (int64_t)m * p.ldc + n) = d;
+      }
     }
     asm volatile("" ::: "memory");
   }
@@ -793,9 +819,9 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
 // given) the pass's JC * 32 validity bytes are loaded once, one per lane, and
 // their ballot is a wave-uniform bit mask; a lane tests its row's bit, and
 // an invalid row is written as resid (TK_ROWS_KEEP_RESID) or 0.
-template <class ML, int WAVES_M, int JB, int JC, bool ROWS, bool WHOLE>
+template <class ML, int WAVES_M, int JB, int JC, bool ROWS, bool WHOLE, bool SHIFT>
 __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int mw, int nw,
-                                           char* region) {
+                                           char* region, int m_lo, int n_lo) {
   constexpr int FN = ML::FN;
   constexpr int CPR = ML::WN * 4 / 16;  // 16-byte chunks per staged row
   constexpr int RPI = 64 / CPR;         // staged rows per read-back step of the wave
@@ -833,7 +859,7 @@ __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc
     for (int it = 0; it < G; ++it) {
       const int row = (g * G + it) * RPI + row0;
       const int m = mb + row;
-      if (WHOLE || (m < p.M && n < p.N)) {
+      if (SHIFT ? (m >= m_lo && n >= n_lo) : (WHOLE || (m < p.M && n < p.N))) {
         const f32x4 d = *reinterpret_cast<const f32x4*>(region + epi_off<CPR>(row, ch));
         float* cr = reinterpret_cast<float*>(p.c) + (int64_t)m * p.ldc + n;
         const bool valid = !ROWS || ((rows_ok >> row) & 1ull);
@@ -883,9 +909,9 @@ __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc
 // fp32 residual epilogue: one resid_pass per group of JC accumulator blocks
 // (two groups when the staging region holds one 32-row block per wave).  The
 // caller has made the main-loop LDS free.
-template <class ML, int WAVES_M, bool ROWS, bool WHOLE>
+template <class ML, int WAVES_M, bool ROWS, bool WHOLE, bool SHIFT>
 __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
-                                                 int n0, f16* smem) {
+                                                 int n0, f16* smem, int m_lo, int n_lo) {
   constexpr int FM = ML::FM, NW = ML::NW;
   constexpr int ROWB = ML::WN * 4;
   constexpr int LDS_BYTES = ML::LDS_HALVES * 2;
@@ -895,8 +921,8 @@ __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16
   const int mw = m0 + (wave % WAVES_M) * ML::WM;
   const int nw = n0 + (wave / WAVES_M) * ML::WN;
   char* region = reinterpret_cast<char*>(smem) + wave * (JC * 32 * ROWB);
-  resid_pass<ML, WAVES_M, 0, JC, ROWS, WHOLE>(p, acc, mw, nw, region);
-  if constexpr (JC < FM) resid_pass<ML, WAVES_M, JC, JC, ROWS, WHOLE>(p, acc, mw, nw, region);
+  resid_pass<ML, WAVES_M, 0, JC, ROWS, WHOLE, SHIFT>(p, acc, mw, nw, region, m_lo, n_lo);
+  if constexpr (JC < FM) resid_pass<ML, WAVES_M, JC, JC, ROWS, WHOLE, SHIFT>(p, acc, mw, nw, region, m_lo, n_lo);
 }
 
 // The fp32 residual epilogue (dense rows) of the persistent ping-pong kernel,
@@ -913,9 +939,10 @@ __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16
 // instructions are the output stores of passes 2 and 3, which may stay in
 // flight into the next tile.  Per element the sum is resid + (acc + bias),
 // as in resid_pass, so the outputs are bit-identical to gemm_kernel's.
-template <class ML, int WAVES_M>
+template <class ML, int WAVES_M, bool SHIFT>
 __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
-                                                    int n0, f16* smem, bool has_next, int next_m0, int next_n0) {
+                                                    int n0, f16* smem, bool has_next, int next_m0, int next_n0,
+                                                    int m_lo, int n_lo) {
   constexpr int FM = ML::FM, FN = ML::FN;
   constexpr int CPR = 16;          // 16-byte chunks per staged row (64 fp32)
   constexpr int RPI = 64 / CPR;    // rows per read-back step
@@ -966,7 +993,15 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = rk[it][e] + (d[e] + b[e]);
-      *reinterpret_cast<f32x4*>(cbase + (int64_t)row * p.ldc + ch * 4) = o;
+      if constexpr (SHIFT) {
+        const int m = mw + (k >> 1) * 32 + row, n = nw + (k & 1) * 64 + ch * 4;
+        const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 4) + (uint32_t)(n - n0) * 4;
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(u32x4, o), tile_store_rsrc(reinterpret_cast<float*>(p.c) + (int64_t)m0 * p.ldc + n0),
+            m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
+      } else {
+        *reinterpret_cast<f32x4*>(cbase + (int64_t)row * p.ldc + ch * 4) = o;
+      }
     }
   };
   fetch(0, r[0]);
@@ -983,6 +1018,21 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
   }
 }
 
+// T::SHIFT: M and N are at least one tile but need not be multiples of it.
+// The last tile row (column) is moved up (left) to end at M (N), so every load
+// stays in range without a test; the rows and columns that the tile before
+// it owns are computed again and not stored (with an in-place residual their
+// residual may be read before or after the owner's update; the value is
+// dropped).
+template <class T>
+__device__ __forceinline__ int tile_m0(const GemmArgs& p, int tm) {
+  return T::SHIFT ? min(tm * T::BM, p.M - T::BM) : tm * T::BM;
+}
+template <class T>
+__device__ __forceinline__ int tile_n0(const GemmArgs& p, int tn) {
+  return T::SHIFT ? min(tn * T::BN, p.N - T::BN) : tn * T::BN;
+}
+
 template <class T, int EPI, bool DIRECT>
 __global__ __launch_bounds__(T::NT) void gemm_kernel(GemmArgs p) {
   constexpr int BM = T::BM, BN = T::BN;
@@ -993,7 +1043,8 @@ __global__ __launch_bounds__(T::NT) void gemm_kernel(GemmArgs p) {
   int tm, tn;
   tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
   f32x16 acc[ML::FN][ML::FM];
-  ML::run(p, tm * BM, tn * BN, smem, acc);
+  const int m0 = tile_m0<T>(p, tm), n0 = tile_n0<T>(p, tn);
+  ML::run(p, m0, n0, smem, acc);
   // The epilogues stage each wave's results in its own part of the main-loop
   // LDS.  The two-stage loop needs a barrier first (other waves may still read
   // the last K-tile); after the ping-pong loop every read of the stages has
@@ -1001,9 +1052,10 @@ __global__ __launch_bounds__(T::NT) void gemm_kernel(GemmArgs p) {
   // while group 1 issues the last K-tile's MFMAs.
   if constexpr (!ML::PINGPONG) __syncthreads();
   if constexpr (EPI == TK_EPI_BIAS_RESID || EPI == kEpiResidRows)
-    store_tile_resid<ML, T::WAVES_M, EPI == kEpiResidRows, ML::PINGPONG>(p, acc, tm * BM, tn * BN, smem);
+    store_tile_resid<ML, T::WAVES_M, EPI == kEpiResidRows, ML::PINGPONG, T::SHIFT>(p, acc, m0, n0, smem, tm * BM,
+                                                                                   tn * BN);
   else
-    store_tile_lds<ML, T::WAVES_M, EPI, ML::PINGPONG>(p, acc, tm * BM, tn * BN, smem);
+    store_tile_lds<ML, T::WAVES_M, EPI, ML::PINGPONG, T::SHIFT>(p, acc, m0, n0, smem, tm * BM, tn * BN);
 }
 
 // Persistent ping-pong GEMM (whole 256 x 256 tiles; fp16 epilogues and the
@@ -1021,7 +1073,7 @@ __global__ __launch_bounds__(T::NT) void gemm_pf_kernel(GemmArgs p) {
   static_assert(ML::PINGPONG && (EPI == TK_EPI_BIAS || EPI == TK_EPI_BIAS_GELU || EPI == TK_EPI_BIAS_RESID),
                 "bias, GELU or dense residual epilogue, ping-pong loop");
   __shared__ __attribute__((aligned(16))) f16 smem[ML::LDS_HALVES];
-  const int tiles_m = p.M / BM, tiles_n = p.N / BN;
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
   const int tiles = tiles_m * tiles_n;
   bool prefetched = false;
   for (int id = blockIdx.x; id < tiles; id += gridDim.x) {
@@ -1030,13 +1082,16 @@ __global__ __launch_bounds__(T::NT) void gemm_pf_kernel(GemmArgs p) {
     const int next = id + (int)gridDim.x;
     int ntm = 0, ntn = 0;
     if (next < tiles) tile_of_block(next, tiles_m, tiles_n, ntm, ntn);
+    const int m0 = tile_m0<T>(p, tm), n0 = tile_n0<T>(p, tn);
+    const int nm0 = tile_m0<T>(p, ntm), nn0 = tile_n0<T>(p, ntn);
     f32x16 acc[ML::FN][ML::FM];
     ML::zero(acc);
-    ML::template run_pingpong<kPfStores>(p, tm * BM, tn * BN, smem, acc, prefetched);
+    ML::template run_pingpong<kPfStores>(p, m0, n0, smem, acc, prefetched);
     if constexpr (EPI == TK_EPI_BIAS_RESID)
-      store_tile_resid_pf<ML, T::WAVES_M>(p, acc, tm * BM, tn * BN, smem, next < tiles, ntm * BM, ntn * BN);
+      store_tile_resid_pf<ML, T::WAVES_M, T::SHIFT>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM, tn * BN);
     else
-      store_tile_lds_pf<ML, T::WAVES_M, EPI>(p, acc, tm * BM, tn * BN, smem, next < tiles, ntm * BM, ntn * BN);
+      store_tile_lds_pf<ML, T::WAVES_M, EPI, T::SHIFT>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM,
+                                                       tn * BN);
     wait_lgkm0();
     phase_barrier();
     prefetched = next < tiles;
@@ -1169,22 +1224,21 @@ __global__ __launch_bounds__(T::NT) void gemm_ln_kernel(GemmArgs p) {
     }
 }
 
-template <class T, int EPI>
+template <class T, int EPI, bool DIRECT>
 int launch_gemm(const GemmArgs& p, hipStream_t st) {
   const int64_t tiles = (int64_t)((p.M + T::BM - 1) / T::BM) * ((p.N + T::BN - 1) / T::BN);
-  // The direct global->LDS copy needs whole K tiles of 16-byte row chunks.
-  if (p.K % T::BK == 0 && p.kvec) {
-    hipLaunchKernelGGL((gemm_kernel<T, EPI, true>), dim3((unsigned)tiles), dim3(T::NT), 0, st, p);
-  } else {
-    hipLaunchKernelGGL((gemm_kernel<T, EPI, false>), dim3((unsigned)tiles), dim3(T::NT), 0, st, p);
-  }
+  hipLaunchKernelGGL((gemm_kernel<T, EPI, DIRECT>), dim3((unsigned)tiles), dim3(T::NT), 0, st, p);
   return check_launch("tk_gemm");
 }
 
 using TileBig = Tile<256, 256, 4, 2, 64, 2>;   // 8 waves of 64 x 128
 using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop (whole tiles)
+using TileBigPPS = Tile<256, 256, 4, 2, 64, 2, true, true>;  // ping-pong, shifted edge tiles
 using TileMid = Tile<128, 128, 2, 2, 64, 2>;   // 4 waves of 64 x 64, 2 blocks per CU
-using TileSmall = Tile<64, 64, 1, 1, 64, 2>;   // 1 wave
+using TileMid3 = Tile<128, 128, 4, 2, 64, 3>;  // 8 waves of 32 x 64, 1 block per CU (96 KB LDS)
+using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
+using TileTall3 = Tile<128, 64, 4, 2, 64, 3>;  // the same, two K-tiles in flight
+using TileSmall = Tile<64, 64, 2, 2, 64, 3>;   // 4 waves of 32 x 32, 3 blocks per CU
 
 #ifndef TK_GEMM_PF
 #define TK_GEMM_PF 1
@@ -1192,39 +1246,77 @@ using TileSmall = Tile<64, 64, 1, 1, 64, 2>;   // 1 wave
 constexpr bool kGemmPf = TK_GEMM_PF;
 constexpr int kPfGrid = 256;  // one persistent workgroup per CU
 
+template <class T, int EPI>
+int launch_pingpong(const GemmArgs& p, int64_t tiles, hipStream_t st) {
+  if constexpr (EPI == TK_EPI_BIAS || EPI == TK_EPI_BIAS_GELU || EPI == TK_EPI_BIAS_RESID) {
+    if (kGemmPf && tiles > kPfGrid) {  // some workgroup runs two or more tiles
+      hipLaunchKernelGGL((gemm_pf_kernel<T, EPI>), dim3((unsigned)kPfGrid), dim3(T::NT), 0, st, p);
+      return check_launch("tk_gemm");
+    }
+  }
+  return launch_gemm<T, EPI, true>(p, st);
+}
+
+// Every figure: MI355X, us per launch, operands rotated through four buffers,
+// all tiles timed on 200 shapes (M 16 .. 30000, N 384 .. 6144, K 256 .. 4096,
+// the three epilogues).  Per accumulator the k order is the same for every
+// tile, so the choice never changes a result.
 template <int EPI>
 int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   const int64_t t256 = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
   const int64_t t128 = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
-  // Measured on MI355X (fp16, 256 CUs, every epilogue).
-  // Whole 256x256 tiles (the ping-pong loop has no row clamp and runs K-tiles
-  // in pairs) that fill at least one round of the CUs take the ping-pong loop,
-  // short K included: C4 forward 9.07 -> 8.62 ms, every 256x256 GEMM role 6-9 %
-  // faster than the two-stage loop; C3 out-projection (one round, K = 1024)
-  // 62.0 -> 54.4 us against the 128x128 tile; C2 FFN-up (two rounds, K = 512)
-  // unchanged.
-  // (its epilogues also assume vector-aligned output rows and bias).
-  if (t256 >= 256 && p.M % 256 == 0 && p.N % 256 == 0 && p.K > 0 && p.K % 128 == 0 && p.vec &&
-      (p.bias == nullptr || p.bias16)) {
-    if constexpr (EPI == TK_EPI_BIAS || EPI == TK_EPI_BIAS_GELU || EPI == TK_EPI_BIAS_RESID) {
-      if (kGemmPf && p.kvec && t256 > kPfGrid) {  // some workgroup runs two or more tiles
-        hipLaunchKernelGGL((gemm_pf_kernel<TileBigPP, EPI>), dim3((unsigned)kPfGrid), dim3(TileBigPP::NT), 0, st, p);
-        return check_launch("tk_gemm");
-      }
-    }
-    return launch_gemm<TileBigPP, EPI>(p, st);
+  const int64_t tall = (int64_t)((p.M + 127) / 128) * ((p.N + 63) / 64);
+  const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64);
+  // Share of the rounds of 256 tiles of 256 x 256 (one per CU) that is output:
+  // what a partial last round and partial edge tiles leave.
+  const int64_t rounds = (t256 + 255) / 256;
+  const double fill = (double)p.M * p.N / (65536.0 * 256.0 * (double)rounds);
+  // The direct global->LDS copy needs whole K tiles of 16-byte row chunks.
+  const bool direct = p.K % 64 == 0 && p.kvec;
+  // Ping-pong loop (256 x 256 tiles, K in pairs of 64, vector-aligned output
+  // rows and bias; no row clamp, so M and N of at least a tile, edge tiles
+  // shifted, whose stores take 32-bit offsets).  Against the best two-stage
+  // tile: M4662 N3072 K1024 (fill 0.85) 33.8 vs 36.0, M4662 N2304 K768 (0.63)
+  // 25.1 vs 26.4, M3000 N3072 K1024 (0.55) 28.2 vs 31.0, M12000 N1024 K4096
+  // (0.73) 105 vs 125; at 0.5 and below it loses (M8192 N1024 K4096 92 vs 83).
+  // With two rounds it pays from two thirds (M4662 N6144 K2048, 0.85: 110 vs
+  // 126; M6000 N4096 K1024, 0.72: 65.5 vs 68.6; M6000 N3072 K1024, 0.55: 53.6
+  // vs 53.1).  Below K = 512 the smaller tiles are as fast.
+  const bool pp_fits = direct && p.K > 0 && p.K % 128 == 0 && p.vec && (p.bias == nullptr || p.bias16) &&
+                       p.M >= 256 && p.N >= 256 && p.N % 8 == 0 && p.ldc < (1 << 20) && p.ldr < (1 << 20) &&
+                       p.lda < (1 << 24) && p.ldw < (1 << 24);
+  if (pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.52 : 0.66)) {
+    // Whole tiles need no store masks: the fp32 residual epilogue is 0.5-1.5 %
+    // faster without them (C4 out-projection 289.5 vs 291.2), the fp16 ones equal.
+    if (p.M % 256 == 0 && p.N % 256 == 0) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
+    return launch_pingpong<TileBigPPS, EPI>(p, t256, st);
   }
-  // Other shapes, with the two-stage loop: 256x256 tiles win when they fill
-  // whole rounds of the 256 CUs (or at least two rounds); with a partial last
-  // round (e.g. 384 tiles) the 128x128 tile, two blocks per CU, is 5-10 %
-  // faster, as it is for narrow and short outputs down to 128 of its tiles;
-  // below that the 64x64 tile keeps the CUs busy.  Short K (<= 1024) with at
-  // most two rounds of 256x256 tiles also runs 128x128 tiles (0.5-4 % faster);
-  // larger K or more rounds favour 256x256.
-  const bool short_k = p.K <= 1024 && t256 <= 512;
-  if (!short_k && t256 >= 256 && (t256 % 256 == 0 || t256 >= 512)) return launch_gemm<TileBig, EPI>(p, st);
-  if (t128 >= 128) return launch_gemm<TileMid, EPI>(p, st);
-  return launch_gemm<TileSmall, EPI>(p, st);
+  if (!direct) {  // register-staged operands
+    const bool short_k = p.K <= 1024 && t256 <= 512;
+    if (!short_k && t256 >= 256 && (t256 % 256 == 0 || t256 >= 512)) return launch_gemm<TileBig, EPI, false>(p, st);
+    if (t128 >= 128) return launch_gemm<TileMid, EPI, false>(p, st);
+    return launch_gemm<TileSmall, EPI, false>(p, st);
+  }
+  // Two-stage 256 x 256 tiles where the ping-pong loop cannot run (K an odd
+  // multiple of 64): they win later than it does (M12000 N4096 K1024, fill
+  // 0.98: 123.6 vs 133.6 on 128 x 128; M6000 N6144 K2048, 0.73: 171.6 vs 169.6).
+  if (p.K >= 512 && fill >= (rounds == 1 ? 0.62 : 0.8)) return launch_gemm<TileBig, EPI, true>(p, st);
+  // Up to one workgroup per CU the K loop is a chain of copy latencies: the
+  // smallest tile that keeps every workgroup resident, more waves on each and
+  // two K-tiles in flight.  Four-wave 64 x 64 tiles: M512 N1024 K4096 35.3
+  // (one wave, one K-tile in flight) -> 20.6, M128 N3072 K1024 12.5 -> 7.7.
+  if (t64 <= 256) return launch_gemm<TileSmall, EPI, true>(p, st);
+  // 128 x 64: M512 N4096 K1024 15.8 -> 10.1, M2048 N1024 K4096 41.2 -> 28.4.
+  if (tall <= 256) return launch_gemm<TileTall3, EPI, true>(p, st);
+  // Up to one 128 x 128 tile per CU: with a long K that tile with two K-tiles
+  // in flight (M3000 N1024 K4096 44.7 -> 38.9, M8192 N512 K2048 34.0 -> 28.1);
+  // else two or three 128 x 64 tiles per CU, whose waves cover one another's
+  // waits (M2048 N2048 K512 12.1 -> 11.1, M3000 N768 K768 13.4 -> 11.8).
+  if (t128 <= 256) return p.K >= 2048 ? launch_gemm<TileMid3, EPI, true>(p, st) : launch_gemm<TileTall2, EPI, true>(p, st);
+  // Up to 512 the same 128 x 64 tiles with a short K (M3000 N2048 K512 15.7 ->
+  // 14.8, M6000 N768 K256 10.0 -> 8.8); beyond, or with a longer K, 128 x 128.
+  if (t128 <= 512 && p.K <= 512) return launch_gemm<TileTall2, EPI, true>(p, st);
+  return launch_gemm<TileMid, EPI, true>(p, st);
 }
 
 template <class T>

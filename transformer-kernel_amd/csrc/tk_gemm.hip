@@ -598,15 +598,11 @@ struct Mainloop {
 // Tile configuration: block tile BM x BN, wave grid WAVES_M x WAVES_N, and
 // for the direct-copy path the K step and number of LDS stages.  The staged
 // (K-tail) path always runs K step 64 with two stages.
-// SHIFT (ping-pong tiles only): M and N need not be multiples of the tile; see
-// gemm_kernel.
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int BK_, int STAGES_, bool PP_ = false, bool SHIFT_ = false>
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int BK_, int STAGES_, bool PP_ = false>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int BK = BK_, STAGES = STAGES_;
   static constexpr bool PP = PP_;
-  static constexpr bool SHIFT = SHIFT_;
-  static_assert(PP_ || !SHIFT_, "shifted edge tiles: ping-pong loop");
   static constexpr int NT = 64 * WAVES_M_ * WAVES_N_;
   template <bool DIRECT>
   using ML = Mainloop<BM, BN, WAVES_M, WAVES_N, DIRECT ? BK : 64, DIRECT ? STAGES : 2, DIRECT, 0, PP && DIRECT>;
@@ -636,10 +632,10 @@ constexpr int kEpiResidRows = 3;
 // pieces of 32 rows.  Bias and GELU are applied in fp32 before the fp16
 // rounding.  The caller has made the main-loop LDS free (every read of the
 // K-tile stages complete).  WHOLE: the tile lies inside M x N, the output rows
-// take 16-byte stores and a given bias 16-byte loads (no bounds tests).
-// SHIFT: rows below m_lo and columns below n_lo belong to another tile and are
-// not stored.
-template <class ML, int WAVES_M, int EPI, bool WHOLE, bool SHIFT>
+// take 16-byte stores and a given bias 16-byte loads (no bounds tests); rows
+// below m_lo and columns below n_lo belong to another tile and are not stored
+// (tile_m0).
+template <class ML, int WAVES_M, int EPI, bool WHOLE>
 __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
                                                int n0, f16* smem, int m_lo, int n_lo) {
   constexpr int WM = ML::WM, WN = ML::WN, FM = ML::FM, FN = ML::FN, NW = ML::NW;
@@ -698,7 +694,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
       const int row = idx / CPR, ch = idx % CPR;
       const int m = mw + jb * 32 + row;
       const int n = nw + ch * EPC;
-      if (SHIFT ? (m >= m_lo && n >= n_lo) : (WHOLE || (m < p.M && n < p.N))) {
+      if (WHOLE ? (m >= m_lo && n >= n_lo) : (m < p.M && n < p.N)) {
         const f16x8 d = *reinterpret_cast<const f16x8*>(region + epi_off<CPR>(row, ch));
         f16* cr = reinterpret_cast<f16*>(p.c) + (int64_t)m * p.ldc + n;
         if (WHOLE || (p.vec && n + 7 < p.N)) {
@@ -722,7 +718,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
 // make the compiler's wait for it also wait for those (the vector memory
 // counter retires in order).  Then the prefetch, then the passes with their
 // kPfStores output stores, all of which may stay in flight into the next tile.
-// SHIFT: rows below m_lo and columns below n_lo are not stored; their stores
+// Rows below m_lo and columns below n_lo are not stored (tile_m0); their stores
 // are issued all the same (the count of instructions in flight must not
 // depend on the tile), to an offset past the buffer's range, which drops them.
 constexpr int kPfStores = 16;
@@ -734,7 +730,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_store_rsrc(void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
 }
 
-template <class ML, int WAVES_M, int EPI, bool SHIFT>
+template <class ML, int WAVES_M, int EPI>
 __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
                                                   int n0, f16* smem, bool has_next, int next_m0, int next_n0,
                                                   int m_lo, int n_lo) {
@@ -763,6 +759,7 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
 #pragma unroll
     for (int q = 0; q < 4; ++q) asm volatile("" ::"v"(bias[i][q]));  // the loads have returned here
   if (has_next) ML::pp_prefetch(p, next_m0, next_n0, smem);
+  const __amdgpu_buffer_rsrc_t rsrc = tile_store_rsrc(reinterpret_cast<f16*>(p.c) + (int64_t)m0 * p.ldc + n0);
 #pragma unroll
   for (int jb = 0; jb < FM; ++jb) {
 #pragma unroll
@@ -791,14 +788,9 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
       const int m = mw + jb * 32 + row;
       const int n = nw + ch * EPC;
       const f16x8 d = *reinterpret_cast<const f16x8*>(region + epi_off<CPR>(row, ch));
-      if constexpr (SHIFT) {
-        const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 2) + (uint32_t)(n - n0) * 2;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d),
-                                               tile_store_rsrc(reinterpret_cast<f16*>(p.c) + (int64_t)m0 * p.ldc + n0),
-                                               m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
-      } else {
-        *reinterpret_cast<f16x8*>(reinterpret_cast<f16*>(p.c) + (int64_t)m * p.ldc + n) = d;
-      }
+      const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 2) + (uint32_t)(n - n0) * 2;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d), rsrc,
+                                             m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
     }
     asm volatile("" ::: "memory");
   }
@@ -819,7 +811,7 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
 // given) the pass's JC * 32 validity bytes are loaded once, one per lane, and
 // their ballot is a wave-uniform bit mask; a lane tests its row's bit, and
 // an invalid row is written as resid (TK_ROWS_KEEP_RESID) or 0.
-template <class ML, int WAVES_M, int JB, int JC, bool ROWS, bool WHOLE, bool SHIFT>
+template <class ML, int WAVES_M, int JB, int JC, bool ROWS, bool WHOLE>
 __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int mw, int nw,
                                            char* region, int m_lo, int n_lo) {
   constexpr int FN = ML::FN;
@@ -859,7 +851,7 @@ __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc
     for (int it = 0; it < G; ++it) {
       const int row = (g * G + it) * RPI + row0;
       const int m = mb + row;
-      if (SHIFT ? (m >= m_lo && n >= n_lo) : (WHOLE || (m < p.M && n < p.N))) {
+      if (WHOLE ? (m >= m_lo && n >= n_lo) : (m < p.M && n < p.N)) {
         const f32x4 d = *reinterpret_cast<const f32x4*>(region + epi_off<CPR>(row, ch));
         float* cr = reinterpret_cast<float*>(p.c) + (int64_t)m * p.ldc + n;
         const bool valid = !ROWS || ((rows_ok >> row) & 1ull);
@@ -909,7 +901,7 @@ __device__ __forceinline__ void resid_pass(const GemmArgs& p, const f32x16 (&acc
 // fp32 residual epilogue: one resid_pass per group of JC accumulator blocks
 // (two groups when the staging region holds one 32-row block per wave).  The
 // caller has made the main-loop LDS free.
-template <class ML, int WAVES_M, bool ROWS, bool WHOLE, bool SHIFT>
+template <class ML, int WAVES_M, bool ROWS, bool WHOLE>
 __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
                                                  int n0, f16* smem, int m_lo, int n_lo) {
   constexpr int FM = ML::FM, NW = ML::NW;
@@ -921,8 +913,8 @@ __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16
   const int mw = m0 + (wave % WAVES_M) * ML::WM;
   const int nw = n0 + (wave / WAVES_M) * ML::WN;
   char* region = reinterpret_cast<char*>(smem) + wave * (JC * 32 * ROWB);
-  resid_pass<ML, WAVES_M, 0, JC, ROWS, WHOLE, SHIFT>(p, acc, mw, nw, region, m_lo, n_lo);
-  if constexpr (JC < FM) resid_pass<ML, WAVES_M, JC, JC, ROWS, WHOLE, SHIFT>(p, acc, mw, nw, region, m_lo, n_lo);
+  resid_pass<ML, WAVES_M, 0, JC, ROWS, WHOLE>(p, acc, mw, nw, region, m_lo, n_lo);
+  if constexpr (JC < FM) resid_pass<ML, WAVES_M, JC, JC, ROWS, WHOLE>(p, acc, mw, nw, region, m_lo, n_lo);
 }
 
 // The fp32 residual epilogue (dense rows) of the persistent ping-pong kernel,
@@ -939,7 +931,7 @@ __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16
 // instructions are the output stores of passes 2 and 3, which may stay in
 // flight into the next tile.  Per element the sum is resid + (acc + bias),
 // as in resid_pass, so the outputs are bit-identical to gemm_kernel's.
-template <class ML, int WAVES_M, bool SHIFT>
+template <class ML, int WAVES_M>
 __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
                                                     int n0, f16* smem, bool has_next, int next_m0, int next_n0,
                                                     int m_lo, int n_lo) {
@@ -964,6 +956,7 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
   for (int h = 0; h < 2; ++h) asm volatile("" ::"v"(bias[h]));  // the loads have returned here
   if (has_next) ML::pp_prefetch(p, next_m0, next_n0, smem);
   const uint32_t ldr = (uint32_t)p.ldr;
+  const __amdgpu_buffer_rsrc_t rsrc = tile_store_rsrc(reinterpret_cast<float*>(p.c) + (int64_t)m0 * p.ldc + n0);
   f32x4 r[2][NIT];
   auto fetch = [&](int k, f32x4 (&rk)[NIT]) {
     const float* rbase = p.resid + (int64_t)(mw + (k >> 1) * 32) * p.ldr + nw + (k & 1) * 64;
@@ -985,7 +978,6 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
   };
   auto combine = [&](int k, const f32x4 (&rk)[NIT]) {
     const f32x4 b = bias[k & 1];
-    float* cbase = reinterpret_cast<float*>(p.c) + (int64_t)(mw + (k >> 1) * 32) * p.ldc + nw + (k & 1) * 64;
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int row = it * RPI + row0;
@@ -993,15 +985,10 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = rk[it][e] + (d[e] + b[e]);
-      if constexpr (SHIFT) {
-        const int m = mw + (k >> 1) * 32 + row, n = nw + (k & 1) * 64 + ch * 4;
-        const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 4) + (uint32_t)(n - n0) * 4;
-        __builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(u32x4, o), tile_store_rsrc(reinterpret_cast<float*>(p.c) + (int64_t)m0 * p.ldc + n0),
-            m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
-      } else {
-        *reinterpret_cast<f32x4*>(cbase + (int64_t)row * p.ldc + ch * 4) = o;
-      }
+      const int m = mw + (k >> 1) * 32 + row, n = nw + (k & 1) * 64 + ch * 4;
+      const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 4) + (uint32_t)(n - n0) * 4;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rsrc,
+                                             m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
     }
   };
   fetch(0, r[0]);
@@ -1018,19 +1005,21 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
   }
 }
 
-// T::SHIFT: M and N are at least one tile but need not be multiples of it.
-// The last tile row (column) is moved up (left) to end at M (N), so every load
-// stays in range without a test; the rows and columns that the tile before
-// it owns are computed again and not stored (with an in-place residual their
-// residual may be read before or after the owner's update; the value is
-// dropped).
+// Ping-pong tiles: M and N are at least one tile but need not be multiples of
+// it.  The last tile row (column) is moved up (left) to end at M (N), so every
+// load stays in range without a test; the rows and columns that the tile
+// before it owns are computed again and not stored (with an in-place residual
+// their residual may be read before or after the owner's update; the value is
+// dropped).  Where M and N are whole tiles the masks cost nothing on the fp16
+// epilogues and up to 1 % on the fp32 residual one (M32768 N2048 K2048 289.5
+// -> 291.2 us), so there is no second variant without them.
 template <class T>
 __device__ __forceinline__ int tile_m0(const GemmArgs& p, int tm) {
-  return T::SHIFT ? min(tm * T::BM, p.M - T::BM) : tm * T::BM;
+  return T::PP ? min(tm * T::BM, p.M - T::BM) : tm * T::BM;
 }
 template <class T>
 __device__ __forceinline__ int tile_n0(const GemmArgs& p, int tn) {
-  return T::SHIFT ? min(tn * T::BN, p.N - T::BN) : tn * T::BN;
+  return T::PP ? min(tn * T::BN, p.N - T::BN) : tn * T::BN;
 }
 
 template <class T, int EPI, bool DIRECT>
@@ -1052,13 +1041,12 @@ __global__ __launch_bounds__(T::NT) void gemm_kernel(GemmArgs p) {
   // while group 1 issues the last K-tile's MFMAs.
   if constexpr (!ML::PINGPONG) __syncthreads();
   if constexpr (EPI == TK_EPI_BIAS_RESID || EPI == kEpiResidRows)
-    store_tile_resid<ML, T::WAVES_M, EPI == kEpiResidRows, ML::PINGPONG, T::SHIFT>(p, acc, m0, n0, smem, tm * BM,
-                                                                                   tn * BN);
+    store_tile_resid<ML, T::WAVES_M, EPI == kEpiResidRows, ML::PINGPONG>(p, acc, m0, n0, smem, tm * BM, tn * BN);
   else
-    store_tile_lds<ML, T::WAVES_M, EPI, ML::PINGPONG, T::SHIFT>(p, acc, m0, n0, smem, tm * BM, tn * BN);
+    store_tile_lds<ML, T::WAVES_M, EPI, ML::PINGPONG>(p, acc, m0, n0, smem, tm * BM, tn * BN);
 }
 
-// Persistent ping-pong GEMM (whole 256 x 256 tiles; fp16 epilogues and the
+// Persistent ping-pong GEMM (256 x 256 tiles; fp16 epilogues and the
 // dense fp32 residual epilogue): block b runs tiles b, b + gridDim.x, ...
 // (one XCD each, as tile_of_block expects).  Before a tile's output stores it
 // copies the next tile's first K-tile into stage 0, so the next K loop
@@ -1088,10 +1076,9 @@ __global__ __launch_bounds__(T::NT) void gemm_pf_kernel(GemmArgs p) {
     ML::zero(acc);
     ML::template run_pingpong<kPfStores>(p, m0, n0, smem, acc, prefetched);
     if constexpr (EPI == TK_EPI_BIAS_RESID)
-      store_tile_resid_pf<ML, T::WAVES_M, T::SHIFT>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM, tn * BN);
+      store_tile_resid_pf<ML, T::WAVES_M>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM, tn * BN);
     else
-      store_tile_lds_pf<ML, T::WAVES_M, EPI, T::SHIFT>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM,
-                                                       tn * BN);
+      store_tile_lds_pf<ML, T::WAVES_M, EPI>(p, acc, m0, n0, smem, next < tiles, nm0, nn0, tm * BM, tn * BN);
     wait_lgkm0();
     phase_barrier();
     prefetched = next < tiles;
@@ -1232,8 +1219,7 @@ int launch_gemm(const GemmArgs& p, hipStream_t st) {
 }
 
 using TileBig = Tile<256, 256, 4, 2, 64, 2>;   // 8 waves of 64 x 128
-using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop (whole tiles)
-using TileBigPPS = Tile<256, 256, 4, 2, 64, 2, true, true>;  // ping-pong, shifted edge tiles
+using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop
 using TileMid = Tile<128, 128, 2, 2, 64, 2>;   // 4 waves of 64 x 64, 2 blocks per CU
 using TileMid3 = Tile<128, 128, 4, 2, 64, 3>;  // 8 waves of 32 x 64, 1 block per CU (96 KB LDS)
 using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
@@ -1285,12 +1271,7 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   const bool pp_fits = direct && p.K > 0 && p.K % 128 == 0 && p.vec && (p.bias == nullptr || p.bias16) &&
                        p.M >= 256 && p.N >= 256 && p.N % 8 == 0 && p.ldc < (1 << 20) && p.ldr < (1 << 20) &&
                        p.lda < (1 << 24) && p.ldw < (1 << 24);
-  if (pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.52 : 0.66)) {
-    // Whole tiles need no store masks: the fp32 residual epilogue is 0.5-1.5 %
-    // faster without them (C4 out-projection 289.5 vs 291.2), the fp16 ones equal.
-    if (p.M % 256 == 0 && p.N % 256 == 0) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
-    return launch_pingpong<TileBigPPS, EPI>(p, t256, st);
-  }
+  if (pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.52 : 0.66)) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
   if (!direct) {  // register-staged operands
     const bool short_k = p.K <= 1024 && t256 <= 512;
     if (!short_k && t256 >= 256 && (t256 % 256 == 0 || t256 >= 512)) return launch_gemm<TileBig, EPI, false>(p, st);

@@ -284,6 +284,66 @@ int tk_qkv_attention_supported(int64_t batch, int64_t seq, int64_t heads,
 int tk_small_forward_supported(int64_t seq, int64_t d_model, int64_t heads,
                                int64_t head_dim_padded, int64_t ffn_dim);
 
+/*
+ * The layer loop of the forward: every launch of a dense or padded forward of
+ * any width, enqueued by one call with the arguments the entry points above
+ * take (no other work, so the results are those of the separate calls).
+ *
+ * tk_layer / tk_model hold device pointers to packed weights, laid out as
+ * the separate calls take them: w_qkv [3*heads*head_dim][d_model] (each
+ * head's rows zero-padded to head_dim), w_o [d_model][heads*head_dim], w_1
+ * [ffn][d_model], w_2 [d_model][ffn] f16; biases, norms f32.  The structs
+ * themselves are host memory, read during the call only.
+ */
+typedef struct tk_layer {
+  const float *n1_w, *n1_b;
+  const tk_half *w_qkv;
+  const float *b_qkv;
+  const tk_half *w_o;
+  const float *b_o;
+  const float *n2_w, *n2_b;
+  const tk_half *w_1;
+  const float *b_1;
+  const tk_half *w_2;
+  const float *b_2;
+  float n1_eps, n2_eps;
+} tk_layer;
+
+typedef struct tk_model {
+  int64_t d_model, heads, head_dim, ffn_dim, num_layers; /* head_dim as padded */
+  const tk_layer *layers;                                /* [num_layers] */
+  const float *nf_w, *nf_b;
+  float nf_eps;
+  float scale; /* 1/sqrt(unpadded head_dim) */
+  int causal;
+} tk_model;
+
+enum tk_forward_flags {
+  TK_FWD_FUSED_NORM = 1,   /* residual + LayerNorm in the GEMM epilogues where tk_gemm_ln_supported */
+  TK_FWD_QKV_ATTENTION = 2 /* tk_qkv_attention where it takes the shape (dense inputs) */
+};
+
+/* Bytes of the workspace that tk_forward needs; negative: a tk_status. */
+int64_t tk_forward_workspace(const tk_model *model, int64_t batch, int64_t seq, int dense, int flags);
+
+/* Launches of one forward, and the name of launch `step` (NULL past the end). */
+int64_t tk_forward_steps(const tk_model *model, int64_t batch, int64_t seq, int dense, int flags);
+const char *tk_forward_step_name(const tk_model *model, int64_t batch, int64_t seq, int dense, int flags,
+                                 int64_t step);
+
+/*
+ * x, out: [batch, seq, d_model] f32 (out may not alias x).  valid (nullable):
+ * [batch, seq] validity bytes, NULL = dense.  workspace: 256-byte aligned
+ * device memory of at least tk_forward_workspace bytes, this call's own until
+ * its launches have run.  Runs launches [first_step, first_step + num_steps);
+ * num_steps < 0: all that follow.
+ * Replaces the layer loop of OptimizedTransformer._run_layers_fused
+ * (src/optimized.py:488-554).
+ */
+int tk_forward(const tk_model *model, const float *x, float *out, int64_t batch, int64_t seq,
+               const uint8_t *valid, void *workspace, int64_t workspace_bytes, int flags,
+               int64_t first_step, int64_t num_steps, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

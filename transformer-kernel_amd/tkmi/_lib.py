@@ -20,7 +20,24 @@ TK_F32, TK_F16 = 0, 1
 TK_EPI_BIAS, TK_EPI_BIAS_GELU, TK_EPI_BIAS_RESID = 0, 1, 2
 TK_ROWS_KEEP_RESID, TK_ROWS_ZERO, TK_ROWS_ZERO_ALL = 1, 2, 3
 
+TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION = 1, 2
+
 _I64_3 = c_int64 * 3
+
+
+class Layer(ctypes.Structure):
+    """tk_layer of include/tkmi.h."""
+
+    _fields_ = [(n, c_void_p) for n in ("n1_w", "n1_b", "w_qkv", "b_qkv", "w_o", "b_o", "n2_w", "n2_b", "w_1", "b_1",
+                                        "w_2", "b_2")] + [("n1_eps", c_float), ("n2_eps", c_float)]
+
+
+class Model(ctypes.Structure):
+    """tk_model of include/tkmi.h."""
+
+    _fields_ = [(n, c_int64) for n in ("d_model", "heads", "head_dim", "ffn_dim", "num_layers")] + [
+        ("layers", POINTER(Layer)), ("nf_w", c_void_p), ("nf_b", c_void_p), ("nf_eps", c_float), ("scale", c_float),
+        ("causal", c_int)]
 
 # name -> (restype, argtypes); mirrors include/tkmi.h one to one.
 SIGNATURES = {
@@ -72,6 +89,14 @@ SIGNATURES = {
         + [c_void_p] * 14 + [c_float, c_float, c_float, c_float, c_void_p],
     ),
     "tk_small_forward_supported": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "tk_forward_workspace": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),
+    "tk_forward_steps": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),
+    "tk_forward_step_name": (ctypes.c_char_p, [c_void_p, c_int64, c_int64, c_int, c_int, c_int64]),
+    "tk_forward": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int64,
+         c_void_p],
+    ),
 }
 
 _lock = threading.Lock()

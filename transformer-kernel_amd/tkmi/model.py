@@ -12,7 +12,8 @@ Interface (src/optimized.py:85-157,200-232,393-408):
     module-level default.
 
 Per layer the forward launches five kernels (src/optimized.py:488-554 is the
-reference schedule it replaces):
+reference schedule it replaces), all of them from one call into the library
+(tk_forward; the schedule is written down in csrc/tk_model.hip):
 
   1. QKV GEMM       h[T,D] . Wqkv[3D,D]^T + b          -> qkv fp16 [T, 3D]
   2. attention      flash forward over strided q/k/v    -> ctx fp16 [B, S, H*hd]
@@ -39,7 +40,8 @@ from typing import List, Optional
 
 import torch
 
-from . import ops
+from . import _lib, ops
+from ._lib import TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION
 from .modules import BaselineTransformer
 
 __all__ = ["OptimizerSettings", "OptimizedTransformer", "configure", "active_settings"]
@@ -144,6 +146,7 @@ class OptimizedTransformer(BaselineTransformer):
         self._weight_cache_key: Optional[tuple] = None
         self._param_list: Optional[list] = None  # walking the module tree costs ~60 us per forward
         self._stacked: Optional[dict] = None
+        self._native: Optional[_lib.Model] = None
         self._small_ok: dict = {}  # seq -> tk_small_forward_supported
         self._dense_mask_ref: Optional[weakref.ReferenceType] = None
         self._dense_mask_value = False
@@ -152,6 +155,7 @@ class OptimizedTransformer(BaselineTransformer):
 
     def _apply(self, *args, **kwargs):
         result = super()._apply(*args, **kwargs)
+        self._native = None
         self._weight_cache = None
         self._weight_cache_key = None
         self._param_list = None
@@ -208,7 +212,30 @@ class OptimizedTransformer(BaselineTransformer):
         self._weight_cache = built
         self._weight_cache_key = key
         self._stacked = None
+        self._native = None
         return built
+
+    def _native_model(self) -> _lib.Model:
+        """Addresses of the packed weights as the library's host call takes them."""
+        built = self._weights()
+        if self._native is None:
+            layers = (_lib.Layer * len(built))()
+            for dst, lw in zip(layers, built):
+                for name, _ in _lib.Layer._fields_:
+                    val = getattr(lw, name)
+                    setattr(dst, name, val if name.endswith("_eps") else val.data_ptr())
+            nf_w, nf_b, nf_eps = self._final
+            self._native = _lib.Model(
+                d_model=self.d_model, heads=self.num_heads, head_dim=self.head_dim_padded,
+                ffn_dim=self.config.ffn_dim, num_layers=len(built), layers=layers, nf_w=nf_w.data_ptr(),
+                nf_b=nf_b.data_ptr(), nf_eps=nf_eps, scale=self.attn_scale, causal=int(self.config.causal))
+        return self._native
+
+    def __getstate__(self):
+        # The addresses belong to this object's packed weights: a copy makes its own.
+        state = self.__dict__.copy()
+        state["_native"] = None
+        return state
 
     def _stacked_weights(self) -> dict:
         """The per-layer packed weights stacked over layers (tk_small_forward's layout)."""
@@ -272,7 +299,6 @@ class OptimizedTransformer(BaselineTransformer):
         bsz, seq, d = x.shape
         t = bsz * seq
         nh, hd = self.num_heads, self.head_dim_padded
-        dp = nh * hd  # attention width; > d when the head dim is zero-padded
         weights = self._weights()
         fn_w, fn_b, fn_eps = self._final
         dev = x.device
@@ -287,60 +313,11 @@ class OptimizedTransformer(BaselineTransformer):
                               self.config.causal, self.attn_scale)
             return out
 
-        resid = torch.empty((t, d), dtype=torch.float32, device=dev)
-        h = torch.empty((t, d), dtype=torch.float16, device=dev)
-        # The fused QKV + attention kernel reads h as [T, heads * head_dim]:
-        # only for unpadded head dims (h is [T, d_model]).
-        fused_qa = (mask is None and self.settings.qkv_attention and hd == self.head_dim
-                    and ops.qkv_attention_supported(bsz, seq, nh, hd))
-        qkv = None if fused_qa else torch.empty((t, 3 * dp), dtype=torch.float16, device=dev)
-        ctx = torch.empty((t, dp), dtype=torch.float16, device=dev)
-        u = torch.empty((t, self.config.ffn_dim), dtype=torch.float16, device=dev)
-        out = torch.empty((t, d), dtype=torch.float32, device=dev)
-        fuse = (self.settings.fused_norm and d <= self.settings.fused_norm_max_d
-                and ops.gemm_ln_supported(d))
-
-        rows = mask.view(t) if mask is not None else None
-        ops.ln_fwd(xin, weights[0].n1_w, weights[0].n1_b, weights[0].n1_eps, torch.float16, out=h,
-                   name="ln_in")
-        src = xin  # residual stream input of the next add (the caller's x is never written)
-        if qkv is not None:
-            qkv5 = qkv.view(bsz, seq, 3, nh, hd)
-            q, k, v = qkv5.permute(2, 0, 3, 1, 4).unbind(0)  # [B, H, S, hd] strided views
-        ctx3 = ctx.view(bsz, seq, dp)
-        last = len(weights) - 1
-        for i, lw in enumerate(weights):
-            if fused_qa:
-                ops.qkv_attention(h, lw.w_qkv, lw.b_qkv, bsz, seq, nh, hd, self.attn_scale, self.config.causal,
-                                  out=ctx)
-            else:
-                ops.linear(h, lw.w_qkv, lw.b_qkv, out=qkv, name="qkv")
-                ops.flash_attention(q, k, v, self.attn_scale, self.config.causal, out=ctx3, key_valid=mask)
-            if fuse:
-                ops.linear_add_ln(ctx, lw.w_o, lw.b_o, src, lw.n2_w, lw.n2_b, lw.n2_eps,
-                                  sum_out=resid, h_out=h, name="out_proj_ln",
-                                  row_valid=rows, row_mode=ops.TK_ROWS_KEEP_RESID)
-            else:
-                ops.linear_residual(ctx, lw.w_o, lw.b_o, src, out=resid, name="out_proj_resid",
-                                    row_valid=rows, row_mode=ops.TK_ROWS_KEEP_RESID)
-                ops.ln_fwd(resid, lw.n2_w, lw.n2_b, lw.n2_eps, torch.float16, out=h, name="ln2")
-            src = resid
-            ops.linear(h, lw.w_1, lw.b_1, gelu=True, out=u, name="ffn_up_gelu")
-            if i < last:
-                nw, nb, neps = weights[i + 1].n1_w, weights[i + 1].n1_b, weights[i + 1].n1_eps
-                dst, keep_sum = h, True
-            else:
-                nw, nb, neps = fn_w, fn_b, fn_eps
-                dst, keep_sum = out, False  # final norm: the summed residual is dead
-            if fuse:
-                ops.linear_add_ln(u, lw.w_2, lw.b_2, resid, nw, nb, neps,
-                                  sum_out=resid if keep_sum else None, h_out=dst, name="ffn_down_ln",
-                                  row_valid=rows,
-                                  row_mode=ops.TK_ROWS_ZERO if keep_sum else ops.TK_ROWS_ZERO_ALL)
-            else:
-                ops.linear_residual(u, lw.w_2, lw.b_2, resid, out=resid, name="ffn_down_resid",
-                                    row_valid=rows, row_mode=ops.TK_ROWS_ZERO)
-                ops.ln_fwd(resid, nw, nb, neps, dst.dtype, out=dst,
-                           name="ln_next" if keep_sum else "ln_final",
-                           row_valid=None if keep_sum else rows)
-        return out.view(bsz, seq, d)
+        out = torch.empty((bsz, seq, d), dtype=torch.float32, device=dev)
+        flags = 0
+        if self.settings.fused_norm and d <= self.settings.fused_norm_max_d:
+            flags |= TK_FWD_FUSED_NORM
+        if self.settings.qkv_attention:
+            flags |= TK_FWD_QKV_ATTENTION
+        ops.transformer_forward(self._native_model(), xin.view(bsz, seq, d), out, mask, flags)
+        return out

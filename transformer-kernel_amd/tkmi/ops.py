@@ -15,6 +15,7 @@ raises.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 from typing import List, Optional, Tuple
 
 import torch
@@ -342,6 +343,32 @@ def small_forward(x, out, stacked: dict, final: tuple, n1_eps: float, n2_eps: fl
             w["n2_b"].data_ptr(), nf_w.data_ptr(), nf_b.data_ptr(), float(n1_eps), float(n2_eps),
             float(nf_eps), float(scale), _stream(x))
     return out
+
+
+def transformer_forward(model: "_lib.Model", x, out, valid, flags: int) -> None:
+    """Every launch of a forward by one call into the library (tk_forward).
+
+    ``model``: the packed weights' addresses (OptimizedTransformer._native);
+    x, out: [B, S, D] fp32 contiguous; ``valid``: [B, S] bool or None.  Under
+    ``kernel_timer`` the same launches go out one by one, each timed.
+    """
+    _require_cuda(x, out, valid)
+    b, s, _ = x.shape
+    lib = _lib.load()
+    ref = ctypes.byref(model)
+    dense = int(valid is None)
+    size = lib.tk_forward_workspace(ref, b, s, dense, flags)
+    if size < 0:
+        raise _lib.TkError("tk_forward_workspace", size, lib.tk_last_error_string().decode())
+    ws = torch.empty(size, dtype=torch.uint8, device=x.device)
+    vp = valid.data_ptr() if valid is not None else None
+    args = (ref, x.data_ptr(), out.data_ptr(), b, s, vp, ws.data_ptr(), size, flags)
+    if _timer is None:
+        _lib.call("tk_forward", *args, 0, -1, _stream(x))
+        return
+    for i in range(lib.tk_forward_steps(ref, b, s, dense, flags)):
+        name = lib.tk_forward_step_name(ref, b, s, dense, flags, i).decode()
+        _launch(name, "tk_forward", *args, i, 1, _stream(x))
 
 
 def masked_softmax(scores, causal: bool, key_len=None, heads_per_batch: int = 1):

@@ -22,7 +22,8 @@ SHAPES = {
     "tall_three_stages": (520, 2056, 192),   # 128 x 64, two K-tiles in flight
     "tall_two_stages": (777, 3080, 192),
     "mid_three_stages": (777, 3080, 2048),   # 128 x 128, 8 waves
-    "tall_short_k": (1500, 4104, 192),
+    "wide": (1500, 4104, 2048),              # 128 x 256
+    "tall_short_k": (1500, 3976, 192),
     "mid": (1500, 4104, 576),
     "two_stage_256": (4000, 2824, 576),      # 256 x 256, K an odd multiple of 64
     "pingpong_one_round": (4001, 2312, 512),  # last tile row 161 rows, last column 8 columns

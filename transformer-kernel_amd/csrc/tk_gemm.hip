@@ -720,15 +720,35 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
 // kPfStores output stores, all of which may stay in flight into the next tile.
 // Rows below m_lo and columns below n_lo are not stored (tile_m0); their stores
 // are issued all the same (the count of instructions in flight must not
-// depend on the tile), to an offset past the buffer's range, which drops them.
+// depend on the tile) and dropped by the buffer's range check: see ShiftStore.
 constexpr int kPfStores = 16;
-constexpr uint32_t kDropOffset = 0x80000000u;  // past every range that tile_store_rsrc gives
 
-// Buffer over output tile rows: offsets below 2^31 (the dispatch checks that a
-// tile's rows fit) are stored, kDropOffset is out of range.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_store_rsrc(void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
-}
+// Stores of an output tile whose rows start at m_lo and columns at n_lo,
+// through a buffer over kRange bytes from element (m_lo, n0).  With every row
+// offset inside (-kRange, kRange) (the dispatch bounds ldc), a row below m_lo
+// has a negative offset, past the range as an unsigned number, and kDropColumn
+// added for a column below n_lo keeps any row outside it: no select per store.
+template <typename T>
+struct ShiftStore {
+  static constexpr uint32_t kRange = 1u << 29, kDropColumn = 1u << 30;
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t row_bytes;
+  int m_lo;
+  __device__ __forceinline__ ShiftStore(const GemmArgs& p, int m_lo_, int n0)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<T*>(p.c) + (int64_t)m_lo_ * p.ldc + n0, 0, kRange,
+                                               0x00020000)),
+        row_bytes((uint32_t)p.ldc * (uint32_t)sizeof(T)),
+        m_lo(m_lo_) {}
+  // Offset of columns n.. of a row's 16 bytes, and the store of them in row m.
+  static __device__ __forceinline__ uint32_t column(int n, int n0, int n_lo) {
+    return (uint32_t)(n - n0) * (uint32_t)sizeof(T) + (n >= n_lo ? 0u : kDropColumn);
+  }
+  template <typename V>
+  __device__ __forceinline__ void operator()(int m, uint32_t col, V v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, (uint32_t)(m - m_lo) * row_bytes + col,
+                                           0, 0);
+  }
+};
 
 template <class ML, int WAVES_M, int EPI>
 __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x16 (&acc)[ML::FN][ML::FM], int m0,
@@ -759,7 +779,7 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
 #pragma unroll
     for (int q = 0; q < 4; ++q) asm volatile("" ::"v"(bias[i][q]));  // the loads have returned here
   if (has_next) ML::pp_prefetch(p, next_m0, next_n0, smem);
-  const __amdgpu_buffer_rsrc_t rsrc = tile_store_rsrc(reinterpret_cast<f16*>(p.c) + (int64_t)m0 * p.ldc + n0);
+  const ShiftStore<f16> put(p, m_lo, n0);
 #pragma unroll
   for (int jb = 0; jb < FM; ++jb) {
 #pragma unroll
@@ -788,9 +808,7 @@ __device__ __forceinline__ void store_tile_lds_pf(const GemmArgs& p, const f32x1
       const int m = mw + jb * 32 + row;
       const int n = nw + ch * EPC;
       const f16x8 d = *reinterpret_cast<const f16x8*>(region + epi_off<CPR>(row, ch));
-      const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 2) + (uint32_t)(n - n0) * 2;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, d), rsrc,
-                                             m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
+      put(m, put.column(n, n0, n_lo), d);
     }
     asm volatile("" ::: "memory");
   }
@@ -956,7 +974,7 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
   for (int h = 0; h < 2; ++h) asm volatile("" ::"v"(bias[h]));  // the loads have returned here
   if (has_next) ML::pp_prefetch(p, next_m0, next_n0, smem);
   const uint32_t ldr = (uint32_t)p.ldr;
-  const __amdgpu_buffer_rsrc_t rsrc = tile_store_rsrc(reinterpret_cast<float*>(p.c) + (int64_t)m0 * p.ldc + n0);
+  const ShiftStore<float> put(p, m_lo, n0);
   f32x4 r[2][NIT];
   auto fetch = [&](int k, f32x4 (&rk)[NIT]) {
     const float* rbase = p.resid + (int64_t)(mw + (k >> 1) * 32) * p.ldr + nw + (k & 1) * 64;
@@ -985,10 +1003,7 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = rk[it][e] + (d[e] + b[e]);
-      const int m = mw + (k >> 1) * 32 + row, n = nw + (k & 1) * 64 + ch * 4;
-      const uint32_t off = (uint32_t)(m - m0) * ((uint32_t)p.ldc * 4) + (uint32_t)(n - n0) * 4;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rsrc,
-                                             m >= m_lo && n >= n_lo ? off : kDropOffset, 0, 0);
+      put(mw + (k >> 1) * 32 + row, put.column(nw + (k & 1) * 64 + ch * 4, n0, n_lo), o);
     }
   };
   fetch(0, r[0]);
@@ -1010,9 +1025,7 @@ __device__ __forceinline__ void store_tile_resid_pf(const GemmArgs& p, const f32
 // load stays in range without a test; the rows and columns that the tile
 // before it owns are computed again and not stored (with an in-place residual
 // their residual may be read before or after the owner's update; the value is
-// dropped).  Where M and N are whole tiles the masks cost nothing on the fp16
-// epilogues and up to 1 % on the fp32 residual one (M32768 N2048 K2048 289.5
-// -> 291.2 us), so there is no second variant without them.
+// dropped).
 template <class T>
 __device__ __forceinline__ int tile_m0(const GemmArgs& p, int tm) {
   return T::PP ? min(tm * T::BM, p.M - T::BM) : tm * T::BM;
@@ -1222,6 +1235,7 @@ using TileBig = Tile<256, 256, 4, 2, 64, 2>;   // 8 waves of 64 x 128
 using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop
 using TileMid = Tile<128, 128, 2, 2, 64, 2>;   // 4 waves of 64 x 64, 2 blocks per CU
 using TileMid3 = Tile<128, 128, 4, 2, 64, 3>;  // 8 waves of 32 x 64, 1 block per CU (96 KB LDS)
+using TileWide3 = Tile<128, 256, 2, 4, 64, 3>;  // 8 waves of 64 x 64, 1 block per CU (144 KB LDS)
 using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
 using TileTall3 = Tile<128, 64, 4, 2, 64, 3>;  // the same, two K-tiles in flight
 using TileSmall = Tile<64, 64, 2, 2, 64, 3>;   // 4 waves of 32 x 32, 3 blocks per CU
@@ -1269,7 +1283,7 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   // 126; M6000 N4096 K1024, 0.72: 65.5 vs 68.6; M6000 N3072 K1024, 0.55: 53.6
   // vs 53.1).  Below K = 512 the smaller tiles are as fast.
   const bool pp_fits = direct && p.K > 0 && p.K % 128 == 0 && p.vec && (p.bias == nullptr || p.bias16) &&
-                       p.M >= 256 && p.N >= 256 && p.N % 8 == 0 && p.ldc < (1 << 20) && p.ldr < (1 << 20) &&
+                       p.M >= 256 && p.N >= 256 && p.N % 8 == 0 && p.ldc < (1 << 19) && p.ldr < (1 << 19) &&
                        p.lda < (1 << 24) && p.ldw < (1 << 24);
   if (pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.52 : 0.66)) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
   if (!direct) {  // register-staged operands
@@ -1294,9 +1308,13 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   // else two or three 128 x 64 tiles per CU, whose waves cover one another's
   // waits (M2048 N2048 K512 12.1 -> 11.1, M3000 N768 K768 13.4 -> 11.8).
   if (t128 <= 256) return p.K >= 2048 ? launch_gemm<TileMid3, EPI, true>(p, st) : launch_gemm<TileTall2, EPI, true>(p, st);
-  // Up to 512 the same 128 x 64 tiles with a short K (M3000 N2048 K512 15.7 ->
-  // 14.8, M6000 N768 K256 10.0 -> 8.8); beyond, or with a longer K, 128 x 128.
-  if (t128 <= 512 && p.K <= 512) return launch_gemm<TileTall2, EPI, true>(p, st);
+  // Up to 512 of them: 128 x 256 tiles, one per CU, where a long K pays for
+  // the larger tile's epilogue (M16384 N512 K2048 54.0 -> 49.3, M6000 N1024
+  // K4096 75.8 -> 68.9); 128 x 64 ones where K is short and all are resident
+  // (M3000 N2048 K512 15.7 -> 14.8, M6000 N768 K256 10.0 -> 8.8; with more
+  // M16384 N512 K512 24.9 -> 27.6).  Everything else: 128 x 128.
+  if (t128 <= 512 && p.K >= 2048) return launch_gemm<TileWide3, EPI, true>(p, st);
+  if (tall <= 768 && p.K <= 512) return launch_gemm<TileTall2, EPI, true>(p, st);
   return launch_gemm<TileMid, EPI, true>(p, st);
 }
 

@@ -255,6 +255,27 @@ int tk_small_forward_noalloc(const float *x, float *out, int64_t batch,
                              const float *nf_b, float n1_eps, float n2_eps,
                              float nf_eps, float scale, void *stream);
 
+/* tk_small_forward on weights packed once into the kernel's fragment order
+ * (tk_small_pack, from the stacked weights above): the same work and results
+ * bit for bit, with one contiguous kilobyte per weight load instead of 32
+ * rows.  packed: tk_small_pack_halves(layers) f16 elements, 16-byte aligned.
+ * d_model = ffn = 128. */
+int64_t tk_small_pack_halves(int64_t layers);
+int tk_small_pack(const tk_half *w_qkv, const tk_half *w_o, const tk_half *w_1,
+                  const tk_half *w_2, tk_half *packed, int64_t layers,
+                  void *stream);
+int tk_small_forward_packed(const float *x, float *out, int64_t batch,
+                            int64_t seq, int64_t heads,
+                            int64_t head_dim_padded, int64_t layers,
+                            int causal, const tk_half *packed,
+                            const float *b_qkv, const float *b_o,
+                            const float *b_1, const float *b_2,
+                            const float *n1_w, const float *n1_b,
+                            const float *n2_w, const float *n2_b,
+                            const float *nf_w, const float *nf_b, float n1_eps,
+                            float n2_eps, float nf_eps, float scale,
+                            void *stream);
+
 /* Fused QKV projection + attention for one-key-tile sequences:
  *   ctx[t, h*64 + :64] = attention_h( h . W_qkv^T + b_qkv )
  * i.e. tk_gemm(h, w_qkv, b_qkv) into a [T, 3*d_model] q|k|v buffer followed

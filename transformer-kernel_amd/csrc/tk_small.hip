@@ -13,8 +13,8 @@
 //     (lane l holds 4 consecutive columns of row 32*mb + (l & 31) per 4
 //     registers), so the out-projection and FFN-down products accumulate
 //     straight into it;
-//   * LayerNorm row statistics are combined across the 4 column waves of a
-//     row through a small LDS table (exact two-pass mean / variance);
+//   * LayerNorm row statistics (two-pass within a wave's 32 columns) are
+//     merged across the 4 column waves of a row through a small LDS table;
 //   * the GEMMs compute C^T = W . A^T on v_mfma_f32_32x32x16_f16: the A
 //     operand is a weight fragment (16 bytes per lane, read from L2 one phase
 //     ahead of its use, the QKV blocks one block ahead), the B operand an
@@ -65,7 +65,37 @@ struct SmallArgs {
   int B;
   char* ws;
   unsigned* flags;
+  const f16* packed;  // PACKED: the four weights in fragment order (pack_weights)
 };
+
+// Weights in fragment order: per layer 24 blocks of 32 output rows (12 of
+// W_qkv, 4 each of W_o, W_1, W_2), each as the 8 MFMA fragments of its 128
+// columns, lane by lane (1 KB per fragment: lane l holds row l & 31, columns
+// 16 kk + 8 (l >> 5) .. + 8).  Read from the row-major weights a fragment
+// touches 32 rows, 32 bytes of each, and the vector-memory path takes ~110
+// cycles for it (8 loads: ~900 cycles of a wave's time); in this order it is
+// one contiguous kilobyte.
+constexpr int kBlocksPerLayer = 24, kFragsPerBlock = 8, kFragHalves = 64 * 8;
+constexpr int kPackO = 12, kPack1 = 16, kPack2 = 20;  // first block of W_o, W_1, W_2
+__device__ __forceinline__ int64_t packed_block(int l, int blk) {
+  return ((int64_t)l * kBlocksPerLayer + blk) * (kFragsPerBlock * kFragHalves);
+}
+
+// One 16-byte chunk per thread.
+__global__ void small_pack_kernel(const f16* w_qkv, const f16* w_o, const f16* w_1, const f16* w_2, f16* packed,
+                                  int layers) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)layers * kBlocksPerLayer * kFragsPerBlock * 64) return;
+  const int lane = (int)(i & 63), kk = (int)(i >> 6) % kFragsPerBlock;
+  const int blk = (int)((i / (64 * kFragsPerBlock)) % kBlocksPerLayer);
+  const int64_t l = i / (64 * kFragsPerBlock * kBlocksPerLayer);
+  const f16* w = blk < kPackO   ? w_qkv + (l * 384 + blk * 32) * 128
+                 : blk < kPack1 ? w_o + (l * 128 + (blk - kPackO) * 32) * 128
+                 : blk < kPack2 ? w_1 + (l * 128 + (blk - kPack1) * 32) * 128
+                                : w_2 + (l * 128 + (blk - kPack2) * 32) * 128;
+  *reinterpret_cast<f16x8*>(packed + i * 8) =
+      *reinterpret_cast<const f16x8*>(w + (lane & 31) * 128 + kk * 16 + (lane >> 5) * 8);
+}
 
 // Byte offset of 16-byte chunk c of row r in an activation tile: the chunk
 // index is XOR-ed with r mod 16, so the 32 rows of a fragment read (one
@@ -98,8 +128,8 @@ constexpr int kSlotBytes = 2 * 32 * kPitch;  // K then V rows of one 32-row bloc
 // only).  Every other phase is row-local.  The ids are j-major, so the blocks a workgroup waits
 // for were dispatched before it, and with a batch that is a multiple of 8 a sequence's blocks
 // share an XCD (ids are dealt round-robin over the 8 XCDs) and its L2.
-template <int D, int DP, int F, int HDP, bool CAUSAL, bool SPLIT>
-__global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
+template <int D, int DP, int F, int HDP, bool CAUSAL, bool SPLIT, bool PACKED>
+__device__ __forceinline__ void small_forward_body(const SmallArgs& p) {
   static_assert(!SPLIT || CAUSAL, "split sequences: causal attention only");
   static_assert(D == 128 && DP == 128 && F == 128, "one width: 4 column waves x 32 columns");
   static_assert(HDP == 16 || HDP == 32 || HDP == 64 || HDP == 128, "head dims with an MFMA k-step");
@@ -119,9 +149,10 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
   char* Qt = smem + kTile;        // Q / u
   char* Kt = smem + 2 * kTile;    // K
   char* Vt = smem + 3 * kTile;    // V
-  float* stats = reinterpret_cast<float*>(smem + 4 * kTile);  // [2][4 column waves][128 rows]
-  float* vecs = stats + 2 * 4 * kMaxRows;                     // [2][VEC], then nf_w, nf_b
+  f32x2* stats = reinterpret_cast<f32x2*>(smem + 4 * kTile);         // [4 column waves][128 rows] (mean, M2)
+  float* vecs = reinterpret_cast<float*>(stats + 4 * kMaxRows);      // [2][VEC], then nf_w, nf_b
   int* lost = reinterpret_cast<int*>(vecs + 2 * VEC + 2 * D);  // split: an earlier block was not seen
+  int* early = lost + 1;                                       // split: the next hand-off can be taken early
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -163,6 +194,9 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
   auto wfrag = [&](const f16* W, int K, int n0, int kk) {
     return *reinterpret_cast<const f16x8*>(W + (uint32_t)((n0 + rl) * K + 8 * g) + kk * 16);
   };
+  auto pfrag = [&](int l, int blk, int kk) {
+    return *reinterpret_cast<const f16x8*>(p.packed + packed_block(l, blk) + kk * kFragHalves + (uint32_t)(lane * 8));
+  };
   // activation fragment (B operand): tile row r, k-step kk (+ chunk offset c0)
   auto afrag = [&](const char* T, int r, int c0, int kk) {
     return *reinterpret_cast<const f16x8*>(T + act_off(r, c0 + 2 * kk + g));
@@ -172,7 +206,12 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
     *reinterpret_cast<f16x4*>(T + act_off(r, n >> 3) + (n & 7) * 2) = t;
   };
 
-  // ---- LayerNorm of the residual stream (exact two passes over the 4 column waves) ----
+  // ---- LayerNorm of the residual stream ----
+  // Each column wave takes the mean of its 32 columns of a row and their squared
+  // deviations from it (two passes over registers); one hand-over merges the
+  // four: mean of means, deviations plus 32 (mean_w - mean)^2 (Chan, Golub and
+  // LeVeque's pairwise update), which has no cancellation either and saves a barrier
+  // and a round trip through LDS over two exchanged sums.
   // FINAL: fp32 to the output; else fp16 into the h tile.
   auto layer_norm = [&](const float* gw, const float* gb, float eps, auto final_c) {
     constexpr bool FINAL = decltype(final_c)::value;
@@ -184,32 +223,26 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
       float s = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s += xr[i][r];
-      s = pair_sum(s);
-      if (g == 0) stats[wc * kMaxRows + mb_of(i) * 32 + rl] = s;
-    }
-    lds_sync();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (SPLIT && i > 0) break;
-      const int m = mb_of(i) * 32 + rl;
-      mean[i] = (stats[m] + stats[kMaxRows + m] + stats[2 * kMaxRows + m] + stats[3 * kMaxRows + m]) / (float)D;
-      float s = 0.f;
+      const float mw = pair_sum(s) * (1.f / 32);
+      s = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float d = xr[i][r] - mean[i];
+        const float d = xr[i][r] - mw;
         s += d * d;
       }
       s = pair_sum(s);
-      if (g == 0) stats[4 * kMaxRows + wc * kMaxRows + m] = s;
+      if (g == 0) stats[wc * kMaxRows + mb_of(i) * 32 + rl] = f32x2{mw, s};
     }
     lds_sync();
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       if (SPLIT && i > 0) break;
       const int m = mb_of(i) * 32 + rl;
-      const float* s2 = stats + 4 * kMaxRows;
-      const float var = (s2[m] + s2[kMaxRows + m] + s2[2 * kMaxRows + m] + s2[3 * kMaxRows + m]) / (float)D;
-      rstd[i] = 1.0f / sqrtf(var + eps);
+      const f32x2 s0 = stats[m], s1 = stats[kMaxRows + m], s2 = stats[2 * kMaxRows + m], s3 = stats[3 * kMaxRows + m];
+      mean[i] = (s0[0] + s1[0] + s2[0] + s3[0]) * 0.25f;
+      const float d0 = s0[0] - mean[i], d1 = s1[0] - mean[i], d2 = s2[0] - mean[i], d3 = s3[0] - mean[i];
+      const float m2 = (s0[1] + s1[1] + s2[1] + s3[1]) + 32.f * (d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3);
+      rstd[i] = 1.0f / sqrtf(m2 * (1.f / D) + eps);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -235,23 +268,31 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
 
   // QKV weight blocks go through a two-deep buffer (block j in wq[j & 1]),
   // the others one phase ahead: at most two phases' fragments are live.
-  f16x8 wq[2][KD], wo[KP], w1[KD], w2[KF];
+  // Split: all three QKV blocks are loaded ahead, one under each of the phases
+  // after the attention (192 KB of weights per layer and workgroup at the
+  // ~60 B/clk a CU gets from L2: issued together they hold a wave up 2200 cycles).
+  constexpr int NWQ = SPLIT ? NQ : 2;
+  f16x8 wq[NWQ][KD], wo[KP], w1[KD], w2[KF];
   auto load_wq = [&](int l, int j) {
     const f16* W = p.w_qkv + (int64_t)l * 3 * DP * D;
 #pragma unroll
-    for (int kk = 0; kk < KD; ++kk) wq[j & 1][kk] = wfrag(W, D, 32 * (wc + 4 * j), kk);
+    for (int kk = 0; kk < KD; ++kk)
+      wq[j % NWQ][kk] = PACKED ? pfrag(l, wc + 4 * j, kk) : wfrag(W, D, 32 * (wc + 4 * j), kk);
   };
   auto load_wo = [&](int l) {
 #pragma unroll
-    for (int kk = 0; kk < KP; ++kk) wo[kk] = wfrag(p.w_o + (int64_t)l * D * DP, DP, 32 * wc, kk);
+    for (int kk = 0; kk < KP; ++kk)
+      wo[kk] = PACKED ? pfrag(l, kPackO + wc, kk) : wfrag(p.w_o + (int64_t)l * D * DP, DP, 32 * wc, kk);
   };
   auto load_w1 = [&](int l) {
 #pragma unroll
-    for (int kk = 0; kk < KD; ++kk) w1[kk] = wfrag(p.w_1 + (int64_t)l * F * D, D, 32 * wc, kk);
+    for (int kk = 0; kk < KD; ++kk)
+      w1[kk] = PACKED ? pfrag(l, kPack1 + wc, kk) : wfrag(p.w_1 + (int64_t)l * F * D, D, 32 * wc, kk);
   };
   auto load_w2 = [&](int l) {
 #pragma unroll
-    for (int kk = 0; kk < KF; ++kk) w2[kk] = wfrag(p.w_2 + (int64_t)l * D * F, F, 32 * wc, kk);
+    for (int kk = 0; kk < KF; ++kk)
+      w2[kk] = PACKED ? pfrag(l, kPack2 + wc, kk) : wfrag(p.w_2 + (int64_t)l * D * F, F, 32 * wc, kk);
   };
 
   // V^T fragment offsets (see flash_dma_body): lane = 16*tq + ts covers
@@ -291,73 +332,88 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
       v[V_N2B + tid] = vreg[7];
     }
   };
-  // Split: K/V hand-off of layer l (after its QKV phase).  This block's K and V rows go to its
-  // slot as they sit in its LDS tiles (the tiles' swizzle depends on the row only); once every
-  // wave's stores have completed, its count of consumers (the later blocks) is published; an
-  // earlier block's rows are read once its count is seen non-zero, and the count is decremented
-  // when they are in LDS, so every count is back at 0 when the launch ends.
+  // Split: K/V hand-off of layer l.  A block's slot is the image of its 32 rows of
+  // the K and V tiles (the tiles' swizzle depends on the row only).  As K and V
+  // come out of the QKV products each lane stores its chunks of them (send_kv:
+  // lanes l and l + 32 hold the two halves of a 16-byte chunk and trade halves
+  // of two chunks); once every wave's stores have completed, the count of
+  // consumers (the later blocks) is published.  A consumer copies an earlier
+  // block's slot to LDS (take_kv) once it has seen its count, and decrements the
+  // count when the rows are there, so every count is back at 0 when the launch
+  // ends.  The earlier blocks are usually ahead (causal attention costs
+  // them less), so wave 0 looks at their counts while LayerNorm runs (peek) and the
+  // rows then come in under the QKV products; otherwise the block waits after
+  // it has published its own rows.
   // Ordering: the rows and the counts move only with agent-scope coherent accesses (sc1: what
   // the compiler emits for relaxed agent-scope atomics, each location coherent across the
   // device).  A producer's row stores have completed (vmcnt(0), every wave, then the barrier)
   // before its count is stored; a consumer issues its row loads after it has read the count.
   // So a consumer that sees the count reads the rows, without the release / acquire fences'
   // L2 write-back and invalidate (18 us of a 73 us C1 forward).
-  auto exchange_kv = [&](int l) {
-    const int64_t slot0 = ((int64_t)b * p.L + l) * 4;
-    constexpr int kChunks = kSlotBytes / 16, kHalf = kChunks / 2;
-    if (jb + 1 < MB) {
-      char* dst = p.ws + (slot0 + jb) * kSlotBytes;
-      for (int c = tid; c < kChunks; c += (int)blockDim.x) {
-        const int half = c >= kHalf, off = (c - half * kHalf) * 16;
-        const f32x4 v = *reinterpret_cast<const f32x4*>((half ? Vt : Kt) + jb * 32 * kPitch + off);
-        asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(dst + half * (kSlotBytes / 2) + off), "v"(v)
-                     : "memory");
-      }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      if (tid == 0)
-        __hip_atomic_store(p.flags + slot0 + jb, (unsigned)(MB - 1 - jb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (jb > 0) {
-      if (tid < jb) {
-        unsigned tries = 0;
-        while (__hip_atomic_load(p.flags + slot0 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u &&
-               ++tries < kSpinLimit)
-          __builtin_amdgcn_s_sleep(2);
-        if (tries >= kSpinLimit) *lost = 1;  // (its count is not decremented below)
-      }
-      __builtin_amdgcn_s_barrier();
-      static_assert(kChunks == 4 * 256, "four 16-byte chunks per thread of a 256-thread workgroup");
-      for (int blk = 0; blk < jb; ++blk) {
-        const char* src = p.ws + (slot0 + blk) * kSlotBytes;
-        const char* a[4];
+  auto slot_of = [&](int l, int blk) { return ((int64_t)b * p.L + l) * 4 + blk; };
+  auto send_kv = [&](int l, int part, const f16x4 (&h4)[4]) {  // part 0 K, 1 V
+    // (a builtin store: the compiler then keeps the data registers until it has read them)
+    const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
+        p.ws + slot_of(l, jb) * kSlotBytes + part * (kSlotBytes / 2), 0, kSlotBytes / 2, 0x00020000);
+    constexpr int kSc1 = 16;  // cache policy: device scope
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int c = tid + 256 * u, half = c >= kHalf;
-          a[u] = src + half * (kSlotBytes / 2) + (c - half * kHalf) * 16;
-        }
-        // loads and their wait in one statement: the outputs are complete when it ends
-        f32x4 v0, v1, v2, v3;
+    for (int q = 0; q < 4; q += 2) {
+      typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+      const u32x2v lo = __builtin_bit_cast(u32x2v, h4[q]), hi = __builtin_bit_cast(u32x2v, h4[q + 1]);
+      // lanes < 32: chunk q (own half, partner's half); lanes >= 32: chunk q + 1
+      const auto a0 = __builtin_amdgcn_permlane32_swap(lo[0], hi[0], false, false);
+      const auto a1 = __builtin_amdgcn_permlane32_swap(lo[1], hi[1], false, false);
+      typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+      const u32x4v v = {a0[0], a1[0], a0[1], a1[1]};
+      const int c = 4 * wc + q + g;  // 16-byte chunk of the row
+      const int off = part ? v_off(rl, c) : act_off(rl, c);
+      __builtin_amdgcn_raw_buffer_store_b128(v, dst, off, 0, kSc1);
+    }
+  };
+  // This wave's share (4 KB of each slot) of the earlier blocks' rows, global -> LDS.
+  auto take_kv = [&](int l) {
+    const uint32_t kv0 = (uint32_t)(size_t)(lds_char*)Kt;
+    for (int blk = 0; blk < jb; ++blk) {
+      const char* src = p.ws + slot_of(l, blk) * kSlotBytes + w * 2048 + (uint32_t)lane * 16u;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {  // K, K, V, V
+        const int off = (u & 1) * 1024;
+        const uint32_t dst = kv0 + (u >> 1) * kTile + blk * (kSlotBytes / 2) + w * 2048 + off;
+        uint32_t saved;
         asm volatile(
-            "global_load_dwordx4 %0, %4, off sc1\n\t"
-            "global_load_dwordx4 %1, %5, off sc1\n\t"
-            "global_load_dwordx4 %2, %6, off sc1\n\t"
-            "global_load_dwordx4 %3, %7, off sc1\n\t"
-            "s_waitcnt vmcnt(0)"
-            : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
-            : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3])
+            "s_mov_b32 %0, m0\n\t"
+            "s_mov_b32 m0, %2\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %1, off sc1\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "v"(src + (u >> 1) * (kSlotBytes / 2) + off), "s"(__builtin_amdgcn_readfirstlane(dst))
             : "memory");
-        const f32x4 vv[4] = {v0, v1, v2, v3};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int c = tid + 256 * u, half = c >= kHalf, off = (c - half * kHalf) * 16;
-          *reinterpret_cast<f32x4*>((half ? Vt : Kt) + blk * 32 * kPitch + off) = vv[u];
-        }
       }
-      lds_sync();
-      if (tid < jb && !*lost)
-        __hip_atomic_fetch_add(p.flags + slot0 + tid, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+  };
+  auto counts_seen = [&](int l) {  // every earlier block of layer l has published
+    return __all(lane >= jb || __hip_atomic_load(p.flags + slot_of(l, min(lane, jb - 1)), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) != 0u);
+  };
+  // In the place of the barrier after the QKV phase.  taken: take_kv has been issued.
+  auto exchange_kv = [&](int l, bool taken) {
+    if (jb + 1 < MB || taken) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_sync();  // this block's Q, K, V tiles complete, and its stores
+    if (jb + 1 < MB && tid == 0)
+      __hip_atomic_store(p.flags + slot_of(l, jb), (unsigned)(MB - 1 - jb), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    if (jb == 0) return;
+    if (!taken) {
+      unsigned tries = 0;
+      while (!counts_seen(l) && ++tries < kSpinLimit) __builtin_amdgcn_s_sleep(1);  // every wave for itself
+      if (tries >= kSpinLimit && lane == 0) *lost = 1;  // (the counts are not decremented below)
+      take_kv(l);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_sync();
+    }
+    if (tid < jb && !*lost)
+      __hip_atomic_fetch_add(p.flags + slot_of(l, tid), ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   vec_load(0);
   vec_store(0);
@@ -365,8 +421,12 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
     vecs[2 * VEC + threadIdx.x] = p.nf_w[threadIdx.x];
     vecs[2 * VEC + D + threadIdx.x] = p.nf_b[threadIdx.x];
   }
-  if (threadIdx.x == 0) *lost = 0;
+  if (threadIdx.x == 0) *lost = *early = 0;
   load_wq(0, 0);
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int j = 1; j < NQ; ++j) load_wq(0, j);
+  }
   lds_sync();  // vectors of layer 0 and the final norm staged
   layer_norm(vecs + V_N1W, vecs + V_N1B, p.n1_eps, std::false_type{});
   // Attention work items: (head, 32-row query block), heaviest first (causal
@@ -375,48 +435,77 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
   const int NWV = blockDim.x >> 6;
   for (int l = 0; l < p.L; ++l) {
     lds_sync();  // h complete
+    bool taken = false;
+    if constexpr (SPLIT) {
+      taken = __builtin_amdgcn_readfirstlane(*early) != 0;
+      if (taken) take_kv(l);
+    }
     // ---- QKV = h . W_qkv^T + b -> Q, K, V tiles ----
     {
       refresh();
       const float* bq = vecs + (l & 1) * VEC;
+      // acc + bias of block j (32 columns of [Q | K | V]), rows of block mb, as fp16
+      auto land = [&](const f32x16& acc, int j, int mb, f16x4 (&h4)[4]) {
+        const int nb = wc + 4 * j;
+        const int part = nb / (DP / 32), col0 = (nb % (DP / 32)) * 32;
 #pragma unroll
-      for (int j = 0; j < NQ; ++j) {
-        if (j + 1 < NQ) load_wq(l, j + 1);
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 bv = *reinterpret_cast<const f32x4*>(bq + 32 * nb + 8 * q + 4 * g);
+          h4[q] = f16x4{(f16)(acc[4 * q] + bv[0]), (f16)(acc[4 * q + 1] + bv[1]), (f16)(acc[4 * q + 2] + bv[2]),
+                        (f16)(acc[4 * q + 3] + bv[3])};
+          const int c = col0 + 8 * q + 4 * g, r = mb * 32 + rl;
+          char* dst = part == 2 ? Vt + v_off(r, c >> 3) : (part == 0 ? Qt : Kt) + act_off(r, c >> 3);
+          *reinterpret_cast<f16x4*>(dst + (c & 7) * 2) = h4[q];
+        }
+      };
+      f16x4 h4[4];
+      if constexpr (SPLIT) {
+        // The three blocks' chains interleave, on one read of the activations
+        // (a lone wave otherwise waits out each chain: 3400 -> 1500 cycles); K
+        // and V leave for the later blocks before Q is finished.
+        f32x16 acc[NQ];
+        f16x8 af[KD];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          if (SPLIT && i > 0) break;
-          const int mb = mb_of(i);
-          if (!SPLIT && mb >= MB) break;
-          f32x16 acc = {};
+        for (int kk = 0; kk < KD; ++kk) af[kk] = afrag(Ht, jb * 32 + rl, 0, kk);
 #pragma unroll
-          for (int kk = 0; kk < KD; ++kk)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[j & 1][kk], afrag(Ht, mb * 32 + rl, 0, kk), acc, 0, 0, 0);
-          const int nb = wc + 4 * j;  // 32-column block of [Q | K | V]
-          const int part = nb / (DP / 32), col0 = (nb % (DP / 32)) * 32;
+        for (int kk = 0; kk < KD; ++kk)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = 32 * nb + 8 * q + 4 * g;
-            const f32x4 bv = *reinterpret_cast<const f32x4*>(bq + n);
-            float v[4];
+          for (int j = NQ - 1; j >= 0; --j)
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[j][kk], af[kk], kk == 0 ? f32x16{} : acc[j], 0, 0, 0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[4 * q + e] + bv[e];
-            const int c = col0 + 8 * q + 4 * g, r = mb * 32 + rl;
-            if (part == 2) {
-              const f16x4 t = {(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
-              *reinterpret_cast<f16x4*>(Vt + v_off(r, c >> 3) + (c & 7) * 2) = t;
-            } else {
-              store_h4(part == 0 ? Qt : Kt, r, c, v);
-            }
+        for (int j = NQ - 1; j >= 0; --j) {
+          land(acc[j], j, jb, h4);
+          if (j > 0 && jb + 1 < MB) send_kv(l, j - 1, h4);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+          if (j + 1 < NQ) load_wq(l, j + 1);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int mb = mb_of(i);
+            if (mb >= MB) break;
+            f32x16 acc = {};
+#pragma unroll
+            for (int kk = 0; kk < KD; ++kk)
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wq[j % NWQ][kk], afrag(Ht, mb * 32 + rl, 0, kk), acc, 0, 0,
+                                                           0);
+            land(acc, j, mb, h4);
           }
         }
       }
     }
     // W_o's fragments load under the attention phase; at head_dim 128 its
     // 64-register O leaves no room for them, so they follow it.
-    if constexpr (HDP < 128) load_wo(l);
-    if (l + 1 < p.L) vec_load(l + 1);
-    lds_sync();  // Q, K, V complete
-    if constexpr (SPLIT) exchange_kv(l);
+    // (Split: after the hand-off, whose stores would otherwise wait for them.)
+    if constexpr (SPLIT) {
+      exchange_kv(l, taken);
+      load_wo(l);
+    } else {
+      if constexpr (HDP < 128) load_wo(l);
+      if (l + 1 < p.L) vec_load(l + 1);
+      lds_sync();  // Q, K, V complete
+    }
     // ---- attention over this wave's (head, query block) items; ctx -> h tile ----
     for (int k = 0; k < items; ++k) {
       refresh();
@@ -518,8 +607,9 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
           }
         }
     }
-    if constexpr (HDP == 128) load_wo(l);
+    if constexpr (HDP == 128 && !SPLIT) load_wo(l);
     load_w1(l);
+    if (SPLIT && l + 1 < p.L) vec_load(l + 1);
     lds_sync();  // ctx complete
     // ---- x += ctx . W_o^T + b_o ----
     {
@@ -544,6 +634,7 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
     }
     load_w2(l);
     layer_norm(vecs + (l & 1) * VEC + V_N2W, vecs + (l & 1) * VEC + V_N2B, p.n2_eps, std::false_type{});
+    if (SPLIT && l + 1 < p.L) load_wq(l + 1, 2 % NWQ);
     lds_sync();  // h complete
     // ---- u = gelu(h . W_1^T + b_1) -> u tile (reuses Q) ----
     {
@@ -570,7 +661,7 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
     }
     if (l + 1 < p.L) vec_store((l + 1) & 1);  // layer l+1's vectors (its LN1 runs below)
     lds_sync();  // u complete
-    if (l + 1 < p.L) load_wq(l + 1, 0);
+    if (l + 1 < p.L) load_wq(l + 1, SPLIT ? 1 : 0);
     // ---- x += u . W_2^T + b_2 ----
     {
       refresh();
@@ -592,6 +683,13 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
         }
       }
     }
+    if (SPLIT && l + 1 < p.L) {
+      load_wq(l + 1, 0);
+      if (jb > 0 && w == 0) {
+        const bool seen = counts_seen(l + 1);
+        if (lane == 0) *early = seen;
+      }
+    }
     if (l + 1 < p.L)
       layer_norm(vecs + ((l + 1) & 1) * VEC + V_N1W, vecs + ((l + 1) & 1) * VEC + V_N1B, p.n1_eps,
                  std::false_type{});
@@ -600,20 +698,38 @@ __global__ __launch_bounds__(512, 1) void small_forward_kernel(SmallArgs p) {
   }
 }
 
+// Split workgroups have 256 threads, but are compiled for 512 at head dims 16 and
+// 32: within 256 registers the accumulators stay out of the AGPRs, whose moves
+// made the attention phase a quarter longer; the wider heads' O needs more.
+template <int D, int DP, int F, int HDP, bool CAUSAL, bool SPLIT>
+__global__ __launch_bounds__(SPLIT && HDP >= 64 ? 256 : 512, 1) void small_forward_kernel(SmallArgs p) {
+  small_forward_body<D, DP, F, HDP, CAUSAL, SPLIT, false>(p);
+}
+template <int HDP, bool CAUSAL, bool SPLIT>
+__global__ __launch_bounds__(SPLIT && HDP >= 64 ? 256 : 512, 1) void small_packed_kernel(SmallArgs p) {
+  small_forward_body<128, 128, 128, HDP, CAUSAL, SPLIT, true>(p);
+}
+
 template <int HDP, bool CAUSAL>
 int launch_small(const SmallArgs& p, int64_t batch, hipStream_t st) {
   if constexpr (CAUSAL) {
     if (p.ws != nullptr) {  // split: one 32-row block per workgroup, 4 waves
       const unsigned blocks = (unsigned)batch * (unsigned)((p.S + 31) / 32);
-      hipLaunchKernelGGL((small_forward_kernel<128, 128, 128, HDP, true, true>), dim3(blocks), dim3(256), 0, st, p);
+      if (p.packed)
+        hipLaunchKernelGGL((small_packed_kernel<HDP, true, true>), dim3(blocks), dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((small_forward_kernel<128, 128, 128, HDP, true, true>), dim3(blocks), dim3(256), 0, st, p);
       return check_launch("tk_small_forward");
     }
   }
   // 8 waves: column block w & 3, row blocks (w >> 2) + {0, 2}.  A single row
   // block (S <= 32) leaves waves 4-7 without rows: 4 waves then.
   const unsigned threads = p.S <= 32 ? 256 : 512;
-  hipLaunchKernelGGL((small_forward_kernel<128, 128, 128, HDP, CAUSAL, false>), dim3((unsigned)batch), dim3(threads),
-                     0, st, p);
+  if (p.packed)
+    hipLaunchKernelGGL((small_packed_kernel<HDP, CAUSAL, false>), dim3((unsigned)batch), dim3(threads), 0, st, p);
+  else
+    hipLaunchKernelGGL((small_forward_kernel<128, 128, 128, HDP, CAUSAL, false>), dim3((unsigned)batch),
+                       dim3(threads), 0, st, p);
   return check_launch("tk_small_forward");
 }
 
@@ -712,15 +828,15 @@ __global__ void clear_counts(unsigned* counts, int n) {
   if (i < n) counts[i] = 0u;
 }
 
-int small_forward_call(const char* fn, bool noalloc, const float* x, float* out, int64_t batch, int64_t seq,
+int small_forward_call(const char* fn, bool noalloc, const tk_half* packed, const float* x, float* out, int64_t batch, int64_t seq,
                        int64_t d_model, int64_t heads, int64_t head_dim_padded, int64_t ffn_dim, int64_t layers,
                        int causal, const tk_half* w_qkv, const float* b_qkv, const tk_half* w_o, const float* b_o,
                        const tk_half* w_1, const float* b_1, const tk_half* w_2, const float* b_2, const float* n1_w,
                        const float* n1_b, const float* n2_w, const float* n2_b, const float* nf_w,
                        const float* nf_b, float n1_eps, float n2_eps, float nf_eps, float scale, void* stream) {
   clear_error();
-  TK_REQUIRE(x && out && w_qkv && b_qkv && w_o && b_o && w_1 && b_1 && w_2 && b_2 && n1_w && n1_b && n2_w &&
-                 n2_b && nf_w && nf_b,
+  TK_REQUIRE(x && out && (packed || (w_qkv && w_o && w_1 && w_2)) && b_qkv && b_o && b_1 && b_2 && n1_w && n1_b &&
+                 n2_w && n2_b && nf_w && nf_b,
              TK_ERR_ARG, "%s: null pointer", fn);
   TK_REQUIRE(tk_small_forward_supported(seq, d_model, heads, head_dim_padded, ffn_dim), TK_ERR_UNSUPPORTED,
              "%s: shape S=%lld D=%lld H=%lld hd=%lld F=%lld outside the kernel's "
@@ -731,7 +847,7 @@ int small_forward_call(const char* fn, bool noalloc, const float* x, float* out,
              "%s: batch=%lld layers=%lld", fn, (long long)batch, (long long)layers);
   TK_REQUIRE(scale > 0.f, TK_ERR_ARG, "%s: scale must be > 0", fn);
   auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
-  TK_REQUIRE(al16(x) && al16(out) && al16(w_qkv) && al16(w_o) && al16(w_1) && al16(w_2) && al16(b_qkv) &&
+  TK_REQUIRE(al16(packed) && al16(x) && al16(out) && al16(w_qkv) && al16(w_o) && al16(w_1) && al16(w_2) && al16(b_qkv) &&
                  al16(b_o) && al16(b_1) && al16(b_2) && al16(n1_w) && al16(n1_b) && al16(n2_w) && al16(n2_b) &&
                  al16(nf_w) && al16(nf_b),
              TK_ERR_ARG, "%s: every buffer must be 16-byte aligned", fn);
@@ -739,6 +855,7 @@ int small_forward_call(const char* fn, bool noalloc, const float* x, float* out,
   SmallArgs p;
   p.x = x;
   p.out = out;
+  p.packed = reinterpret_cast<const f16*>(packed);
   p.w_qkv = reinterpret_cast<const f16*>(w_qkv);
   p.b_qkv = b_qkv;
   p.w_o = reinterpret_cast<const f16*>(w_o);
@@ -807,7 +924,7 @@ extern "C" int tk_small_forward(const float* x, float* out, int64_t batch, int64
                                 const float* n1_w, const float* n1_b, const float* n2_w, const float* n2_b,
                                 const float* nf_w, const float* nf_b, float n1_eps, float n2_eps, float nf_eps,
                                 float scale, void* stream) {
-  return small_forward_call("tk_small_forward", false, x, out, batch, seq, d_model, heads, head_dim_padded, ffn_dim,
+  return small_forward_call("tk_small_forward", false, nullptr, x, out, batch, seq, d_model, heads, head_dim_padded, ffn_dim,
                             layers, causal, w_qkv, b_qkv, w_o, b_o, w_1, b_1, w_2, b_2, n1_w, n1_b, n2_w, n2_b, nf_w,
                             nf_b, n1_eps, n2_eps, nf_eps, scale, stream);
 }
@@ -819,7 +936,37 @@ extern "C" int tk_small_forward_noalloc(const float* x, float* out, int64_t batc
                                         const float* b_2, const float* n1_w, const float* n1_b, const float* n2_w,
                                         const float* n2_b, const float* nf_w, const float* nf_b, float n1_eps,
                                         float n2_eps, float nf_eps, float scale, void* stream) {
-  return small_forward_call("tk_small_forward_noalloc", true, x, out, batch, seq, d_model, heads, head_dim_padded,
+  return small_forward_call("tk_small_forward_noalloc", true, nullptr, x, out, batch, seq, d_model, heads, head_dim_padded,
                             ffn_dim, layers, causal, w_qkv, b_qkv, w_o, b_o, w_1, b_1, w_2, b_2, n1_w, n1_b, n2_w,
                             n2_b, nf_w, nf_b, n1_eps, n2_eps, nf_eps, scale, stream);
+}
+
+extern "C" int64_t tk_small_pack_halves(int64_t layers) {
+  return layers < 0 ? TK_ERR_ARG : layers * (int64_t)kBlocksPerLayer * kFragsPerBlock * kFragHalves;
+}
+
+extern "C" int tk_small_pack(const tk_half* w_qkv, const tk_half* w_o, const tk_half* w_1, const tk_half* w_2,
+                             tk_half* packed, int64_t layers, void* stream) {
+  TK_REQUIRE(w_qkv && w_o && w_1 && w_2 && packed, TK_ERR_ARG, "tk_small_pack: null pointer");
+  TK_REQUIRE(layers >= 1 && layers < (1 << 16), TK_ERR_ARG, "tk_small_pack: layers=%lld", (long long)layers);
+  for (const void* q : {(const void*)w_qkv, (const void*)w_o, (const void*)w_1, (const void*)w_2, (const void*)packed})
+    TK_REQUIRE(((uintptr_t)q & 15) == 0, TK_ERR_ARG, "tk_small_pack: every buffer must be 16-byte aligned");
+  const int64_t chunks = tk_small_pack_halves(layers) / 8;
+  hipLaunchKernelGGL(small_pack_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, as_stream(stream),
+                     reinterpret_cast<const f16*>(w_qkv), reinterpret_cast<const f16*>(w_o),
+                     reinterpret_cast<const f16*>(w_1), reinterpret_cast<const f16*>(w_2),
+                     reinterpret_cast<f16*>(packed), (int)layers);
+  return check_launch("tk_small_pack");
+}
+
+extern "C" int tk_small_forward_packed(const float* x, float* out, int64_t batch, int64_t seq, int64_t heads,
+                                       int64_t head_dim_padded, int64_t layers, int causal, const tk_half* packed,
+                                       const float* b_qkv, const float* b_o, const float* b_1, const float* b_2,
+                                       const float* n1_w, const float* n1_b, const float* n2_w, const float* n2_b,
+                                       const float* nf_w, const float* nf_b, float n1_eps, float n2_eps,
+                                       float nf_eps, float scale, void* stream) {
+  TK_REQUIRE(packed, TK_ERR_ARG, "tk_small_forward_packed: null pointer");
+  return small_forward_call("tk_small_forward_packed", false, packed, x, out, batch, seq, 128, heads,
+                            head_dim_padded, 128, layers, causal, nullptr, b_qkv, nullptr, b_o, nullptr, b_1, nullptr,
+                            b_2, n1_w, n1_b, n2_w, n2_b, nf_w, nf_b, n1_eps, n2_eps, nf_eps, scale, stream);
 }

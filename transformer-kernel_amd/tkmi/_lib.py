@@ -88,6 +88,13 @@ SIGNATURES = {
         [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int]
         + [c_void_p] * 14 + [c_float, c_float, c_float, c_float, c_void_p],
     ),
+    "tk_small_pack_halves": (c_int64, [c_int64]),
+    "tk_small_pack": (c_int, [c_void_p] * 5 + [c_int64, c_void_p]),
+    "tk_small_forward_packed": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int]
+        + [c_void_p] * 11 + [c_float, c_float, c_float, c_float, c_void_p],
+    ),
     "tk_small_forward_supported": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64]),
     "tk_forward_workspace": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),
     "tk_forward_steps": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),

@@ -243,6 +243,7 @@ class OptimizedTransformer(BaselineTransformer):
         if self._stacked is None:
             names = ("w_qkv", "b_qkv", "w_o", "b_o", "w_1", "b_1", "w_2", "b_2", "n1_w", "n1_b", "n2_w", "n2_b")
             self._stacked = {n: torch.stack([getattr(lw, n) for lw in built]).contiguous() for n in names}
+            self._stacked["packed"] = ops.small_pack(self._stacked)
         return self._stacked
 
     def _small_forward_ok(self, seq: int, built: List[_LayerWeights]) -> bool:

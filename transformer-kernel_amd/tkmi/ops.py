@@ -321,13 +321,28 @@ def small_forward_supported(seq: int, d_model: int, heads: int, head_dim_padded:
     return bool(_lib.load().tk_small_forward_supported(seq, d_model, heads, head_dim_padded, ffn_dim))
 
 
+def small_pack(stacked: dict):
+    """The stacked projections in the whole-forward kernel's fragment order (tk_small_pack)."""
+    w = [stacked[k] for k in ("w_qkv", "w_o", "w_1", "w_2")]
+    _require_cuda(*w)
+    layers = w[0].shape[0]
+    shapes = [(layers, 384, 128)] + [(layers, 128, 128)] * 3
+    if any(tuple(t.shape) != s or t.dtype != torch.float16 or not t.is_contiguous() for t, s in zip(w, shapes)):
+        raise ValueError("small_pack: contiguous fp16 w_qkv [L, 384, 128] and w_o, w_1, w_2 [L, 128, 128] expected")
+    packed = torch.empty(_lib.load().tk_small_pack_halves(layers), dtype=torch.float16, device=w[0].device)
+    _launch("small_pack", "tk_small_pack", *(t.data_ptr() for t in w), packed.data_ptr(), layers, _stream(w[0]))
+    return packed
+
+
 def small_forward(x, out, stacked: dict, final: tuple, n1_eps: float, n2_eps: float, heads: int,
                   head_dim_padded: int, ffn_dim: int, causal: bool, scale: float, name: str = "small_forward"):
     """The whole dense forward of a narrow model in one launch (tk_small_forward).
 
     x, out: [B, S, D] fp32 contiguous; ``stacked``: the layers' packed weights
-    stacked over layers (OptimizedTransformer._stacked_weights); ``final`` =
-    (weight, bias, eps) of the final LayerNorm.
+    stacked over layers (OptimizedTransformer._stacked_weights), with the four
+    projections also in the kernel's fragment order under ``"packed"``
+    (small_pack; optional, the same results); ``final`` = (weight, bias, eps)
+    of the final LayerNorm.
     """
     _require_cuda(x, out)
     if x.dtype != torch.float32 or out.dtype != torch.float32 or not x.is_contiguous() or not out.is_contiguous():
@@ -336,12 +351,17 @@ def small_forward(x, out, stacked: dict, final: tuple, n1_eps: float, n2_eps: fl
     w = stacked
     layers = w["w_qkv"].shape[0]
     nf_w, nf_b, nf_eps = final
-    _launch(name, "tk_small_forward", x.data_ptr(), out.data_ptr(), b, s, d, heads, head_dim_padded, ffn_dim,
-            layers, int(causal), w["w_qkv"].data_ptr(), w["b_qkv"].data_ptr(), w["w_o"].data_ptr(),
-            w["b_o"].data_ptr(), w["w_1"].data_ptr(), w["b_1"].data_ptr(), w["w_2"].data_ptr(),
-            w["b_2"].data_ptr(), w["n1_w"].data_ptr(), w["n1_b"].data_ptr(), w["n2_w"].data_ptr(),
-            w["n2_b"].data_ptr(), nf_w.data_ptr(), nf_b.data_ptr(), float(n1_eps), float(n2_eps),
-            float(nf_eps), float(scale), _stream(x))
+    vectors = [w[k].data_ptr() for k in ("n1_w", "n1_b", "n2_w", "n2_b")] + [nf_w.data_ptr(), nf_b.data_ptr()]
+    tail = (*vectors, float(n1_eps), float(n2_eps), float(nf_eps), float(scale), _stream(x))
+    if "packed" in w:
+        _launch(name, "tk_small_forward_packed", x.data_ptr(), out.data_ptr(), b, s, heads, head_dim_padded, layers,
+                int(causal), w["packed"].data_ptr(), w["b_qkv"].data_ptr(), w["b_o"].data_ptr(), w["b_1"].data_ptr(),
+                w["b_2"].data_ptr(), *tail)
+    else:
+        _launch(name, "tk_small_forward", x.data_ptr(), out.data_ptr(), b, s, d, heads, head_dim_padded, ffn_dim,
+                layers, int(causal), w["w_qkv"].data_ptr(), w["b_qkv"].data_ptr(), w["w_o"].data_ptr(),
+                w["b_o"].data_ptr(), w["w_1"].data_ptr(), w["b_1"].data_ptr(), w["w_2"].data_ptr(),
+                w["b_2"].data_ptr(), *tail)
     return out
 
 

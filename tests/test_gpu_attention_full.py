@@ -1,0 +1,76 @@
+"""Non-causal attention through the generated steady-state loops, and key masks whose tail is skipped."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import or_rule_violations, seeded
+from tkmi import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _reference(q, k, v, causal, valid):
+    """fp64 softmax of the fp16 operands; rows without a valid key are NaN."""
+    s = q.shape[2]
+    scores = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * q.shape[3] ** -0.5
+    ok = torch.ones(s, s, dtype=torch.bool).tril() if causal else torch.ones(s, s, dtype=torch.bool)
+    if valid is not None:
+        ok = ok & valid[:, None, None, :]
+    p = torch.softmax(scores.masked_fill(~ok, float("-inf")), -1)
+    return torch.matmul(p, v.double()).transpose(1, 2).flatten(2)
+
+
+def _check(q, k, v, causal, valid=None):
+    b, h, s, hd = q.shape
+    got = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal,
+                              key_valid=None if valid is None else valid.to(DEV)).cpu()
+    want = _reference(q, k, v, causal, valid)
+    seen = torch.isfinite(want).all(-1)
+    bad, err = or_rule_violations(got[seen], want[seen].float())
+    assert bad == 0, err
+    assert not bool(torch.isfinite(got[~seen]).any())
+
+
+# key tiles: 2 (no loop step) .. 21, whole and one key off; head_dim 128 loops in groups of 4, 64 of 2
+@pytest.mark.parametrize("s", [129, 191, 256, 383, 384, 449, 512, 833, 1344])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_full_attention_over_tile_counts(s, hd):
+    q, k, v = (seeded(2, 2, s, hd, dtype=torch.float16, seed=60 + i) for i in range(3))
+    _check(q, k, v, False)
+    # scores rising along the keys: every tile moves the running max
+    ramp = torch.arange(s, dtype=torch.float32)[:, None] * 0.05
+    _check(q, (k.float() + ramp * q.float().mean((0, 1, 2)).sign()).half(), v, False)
+
+
+@pytest.mark.parametrize("pattern", ["tail", "head", "holes", "one_batch_empty"])
+@pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
+@pytest.mark.parametrize("hd", [32, 64, 128, 256, 80])
+def test_key_masks(hd, causal, pattern):
+    b, h, s = 3, 2, 777
+    q, k, v = (seeded(b, h, s, hd, dtype=torch.float16, seed=70 + i) for i in range(3))
+    valid = torch.ones(b, s, dtype=torch.bool)
+    if pattern == "tail":  # one key, a whole number of tiles, one key past it
+        valid[0, 1:] = False
+        valid[1, 512:] = False
+        valid[2, 513:] = False
+    elif pattern == "head":
+        valid[:, :200] = False
+    elif pattern == "holes":
+        valid = torch.rand(b, s, generator=torch.Generator().manual_seed(5)) > 0.3
+    else:
+        valid[1] = False
+    _check(q, k, v, causal, valid)
+
+
+def test_eight_byte_value_rows_keep_their_path():
+    """head_dim 128, V rows 8-byte but not 16-byte aligned: no DMA copy possible."""
+    b, h, s, hd = 2, 2, 400, 128
+    q, k, v = (seeded(b, h, s, hd, dtype=torch.float16, seed=80 + i) for i in range(3))
+    wide = torch.zeros(b, h, s, hd + 4, dtype=torch.float16, device=DEV)
+    wide[..., 4:] = v.to(DEV)
+    got = ops.flash_attention(q.to(DEV), k.to(DEV), wide[..., 4:], hd ** -0.5, False).cpu()
+    bad, err = or_rule_violations(got, _reference(q, k, v, False, None).float())
+    assert bad == 0, err

@@ -77,6 +77,27 @@ __device__ __forceinline__ int vpos(int k) { return (k & ~12) | ((k & 4) << 1) |
 // stub, fail.  KMASK: the key-validity mask p.kv is applied (a separate
 // instantiation, so the unmasked kernels carry none of its registers or
 // loads).
+// Number of key tiles up to the last one with a valid key (at least 1): the tiles
+// after it change no row's max, sum or O, so a padded batch skips the tail of
+// its shorter sequences (b6 h12 s777 head_dim 64, lengths from 70 %: 28.5 ->
+// 25.3 us).  256 keys per trip, from the end; every wave for itself.
+// Not for causal launches: their query blocks end at the diagonal, only those past
+// the padding would gain, and the scan cost more (head_dim 256 s369 +4 %).
+template <bool TRIM>
+__device__ __forceinline__ int valid_tiles(const uint8_t* kvb, int n_kt, int S) {
+  if constexpr (!TRIM) return n_kt;
+  const int lane = threadIdx.x & 63;
+  for (int base = ((n_kt - 1) / 4) * 4; base >= 0; base -= 4) {
+    uint8_t by[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) by[i] = kvb[min((base + i) * kBN + lane, S - 1)];
+#pragma unroll
+    for (int i = 3; i >= 0; --i)
+      if (base + i < n_kt && __ballot(by[i] != 0) != 0ull) return __builtin_amdgcn_readfirstlane(base + i + 1);
+  }
+  return 1;
+}
+
 template <int HD, int NW, bool CAUSAL, bool KMASK>
 __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   constexpr int BM = 32 * NW;
@@ -147,7 +168,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
 
   // ---- copies: lane sources within a tile are fixed; a tile adds 64 rows ----
   // Lane l of wave copy ci writes physical chunk l % CPR of tile row
@@ -328,8 +349,8 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
         p_cur[e >> 3][e & 7] = hp[1];
         // Row sum.  Causal: the fp32 exponentials in entry order, as the asm loop (two
         // adds per pair cost less beside the MFMAs than one fp16 dot of the packed pair);
-        // non-causal (no asm loop): the fp16 dot, which keeps these instantiations within
-        // 256 VGPRs without scratch.
+        // non-causal: the fp16 dot, which keeps these instantiations within 256 VGPRs
+        // without scratch.
         if constexpr (CAUSAL) {
           ls += pe[e - 1];
           ls += pe[e];
@@ -412,19 +433,22 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   for (int e = 0; e < 32; ++e) mx_a = fmaxf(mx_a, s_a[e >> 4][e & 15]);
   __syncthreads();  // K(0) read by every wave before step 0 refills its slot
 
-  // ---- hand-ordered steady state (head_dim 64, 4 or 8 waves, causal; dense or key-masked) ----
+  // ---- hand-ordered steady state (head_dim 64, 4 or 8 waves; dense or key-masked) ----
   // Steps [1, 1 + 2*groups) run from an asm loop (tk_attn_steps64{,_w8}.inc, made by
   // gen_attn_steps64.py) that keeps each step's 32 exponentials between its 16
   // MFMAs; every lane does the compiled step's arithmetic in the same order, so
-  // the results are bit-identical.  Those steps' key tiles lie below the query
-  // block (no causal mask; a key mask is applied by the _kmask loops, which
-  // set invalid keys' scores to -inf) and their copies are whole tiles (K tile
+  // the results are bit-identical (without the causal mask the row sums are the
+  // loop's fp32 ones here and fp16 dots in the compiled steps).  Those steps' key
+  // tiles lie below the query block if causal (no causal mask; a key mask is
+  // applied by the _kmask loops, which set invalid keys' scores to -inf) and
+  // their copies are whole tiles (K tile
   // kt+2 < S/kBN); the
   // copies use 32-bit offsets from the K and V bases (span check) and the K read
   // addresses are formed by XOR on bits 5-6 of a 256-byte-aligned row offset.
   int groups = 0;
-  if constexpr (HD == 64 && (NW == 4 || NW == 8) && CAUSAL) {
-    const int last = min(q0 / kBN - 1, min(n_kt, p.S / kBN) - 3);
+  if constexpr (HD == 64 && (NW == 4 || NW == 8)) {
+    int last = min(n_kt, p.S / kBN) - 3;
+    if constexpr (CAUSAL) last = min(last, q0 / kBN - 1);
     const int64_t span =
         ((int64_t)n_kt + 2) * max(k_tile, v_tile) * 2 + (int64_t)kBN * max(p.ks[2], p.vs[2]) * 2;
     // 32-bit unsigned offsets: only for non-negative row strides
@@ -442,7 +466,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
     // Two steps per iteration with no branch between them: the loop-carried
     // accumulators then keep one register assignment.
     int kt = 1;
-    if constexpr (HD == 64 && (NW == 4 || NW == 8) && CAUSAL) {
+    if constexpr (HD == 64 && (NW == 4 || NW == 8)) {
       if (groups > 0) {
         // Pinned: O^T v[64:95], Q v[96:111], the scores of tile kt v[112:143] (s_b), P of
         // tile kt-1 v[144:159] (pf_a), m_run v161, l_run v162; v160 (mx_b, no longer read
@@ -618,7 +642,7 @@ __device__ __forceinline__ void flash_vreg_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
 
   // ---- K tile: direct copies; per-lane source offsets fixed, tile stride added ----
   int k_src_row[K_CPW], k_src_col[K_CPW];
@@ -944,7 +968,7 @@ __device__ __forceinline__ void flash_ring_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
 
   // ---- copies (the layouts of flash_dma_body) ----
   int c_row[CPW], k_col[CPW], v_col[CPW];
@@ -1227,7 +1251,7 @@ __device__ __forceinline__ void flash_pair_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
 
   // ---- copies (the layouts of flash_dma_body) ----
   int c_row[CPW];
@@ -1410,9 +1434,9 @@ __device__ __forceinline__ void flash_pair_body(const AttnArgs& p) {
 
   f32x16 s[2];
   f16x8 pf_a[4], pf_b[4];
-  const bool older = wave < NW / 2;
+  const bool older = !CAUSAL || wave < NW / 2;
 
-  // ---- hand-ordered steady state (head_dim 128, 8 waves, causal; with or without key mask) ----
+  // ---- hand-ordered steady state (head_dim 128, 8 waves; with or without key mask) ----
   // Epochs [1, 1 + 4*groups) run from one asm loop (tk_attn_epochs.inc, made by
   // gen_attn_epochs.py), in one instruction order for every wave.  Each lane does
   // the arithmetic of the compiled epoch in the same order, so O, m and l come out
@@ -1421,15 +1445,16 @@ __device__ __forceinline__ void flash_pair_body(const AttnArgs& p) {
   // tk_attn_epochs_kmask.inc: each epoch also reads its tile's validity bytes,
   // sets invalid keys' scores to -inf and, like the compiled epoch, exponentiates
   // against 0 for rows with no valid key yet.  The epochs it covers need no
-  // causal or length mask (every key tile lies below q0, so below every row of
-  // the workgroup) and copy only
+  // causal or length mask (if causal every key tile lies below q0, so below every
+  // row of the workgroup) and copy only
   // whole tiles (K tile e+2 <= e_lim+1 < S/kBN), so none of the compiled epoch's
   // clamps and guards apply.  The copies use 32-bit offsets from the K and V
   // bases (span check), and the read addresses are formed by XOR on bits 5-7 of
   // a 256-byte-aligned row offset.
   int groups = 0;
-  if constexpr (HD == 128 && NW == 8 && CAUSAL) {
-    const int e_lim = min(q0 / kBN, min(n_kt, p.S / kBN) - 2);
+  if constexpr (HD == 128 && NW == 8) {
+    int e_lim = min(n_kt, p.S / kBN) - 2;
+    if constexpr (CAUSAL) e_lim = min(e_lim, q0 / kBN);
     const int64_t span =
         ((int64_t)n_kt + 2) * max(k_tile, v_tile) * 2 + (int64_t)kBN * max(p.ks[2], p.vs[2]) * 2;
     // 32-bit unsigned offsets: only for non-negative row strides
@@ -1741,7 +1766,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
   const bool d_ok = HDP % 32 == 0 || (lane & 31) < HDP;
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
   for (int kt = 0; kt < n_kt; ++kt) {
     const int k0 = kt * kBN;
     __syncthreads();  // the previous tile's operands are no longer read
@@ -1882,6 +1907,23 @@ __global__ __launch_bounds__(NW * 64, (NW <= 4 && HD <= 64) ? 2 : 1) void flash_
     flash_dma_body<HD, NW, CAUSAL, KMASK>(p);
   }
 }
+// head_dim 128 without the causal mask, more than 128 keys, V rows 16-byte
+// vectors: the pair body too, whose asm loop then covers all but the first and the
+// last few key tiles.  Against the register body (kept for V rows of 8-byte
+// vectors, which cannot be copied by DMA): b4 h16 s2048 172 -> 142 us (798 -> 965
+// TFLOP/s), key-masked 191 -> 156; b2 h8 s8192 589 -> 490; b120 h12 s288, too
+// short for the loop, 231 -> 216.  One epoch order for all waves: with two the
+// key-masked build spills 36 B.
+template <bool KMASK>
+__global__ __launch_bounds__(512, 1) void flash_full_kernel(AttnArgs p) {
+  flash_pair_body<128, 8, false, KMASK>(p);
+}
+int launch_full128(const AttnArgs& p, hipStream_t st) {
+  const dim3 g((unsigned)((int64_t)((p.S + 255) / 256) * p.B * p.H)), blk(512);
+  if (p.kv) hipLaunchKernelGGL((flash_full_kernel<true>), g, blk, 0, st, p);
+  else hipLaunchKernelGGL((flash_full_kernel<false>), g, blk, 0, st, p);
+  return check_launch("tk_flash_attn_fwd");
+}
 template <int HD, int NW, bool CAUSAL, bool KMASK>
 __global__ __launch_bounds__(NW * 64, 4) void flash_single_kernel(AttnArgs p) {
   flash_single_body<HD, NW, CAUSAL, KMASK>(p);
@@ -2002,6 +2044,8 @@ extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_ha
     vec = vec && q_strides[i] % 8 == 0 && k_strides[i] % 8 == 0 && v_strides[i] % (v8 ? 4 : 8) == 0 &&
           o_strides[i] % 4 == 0;
   if (vec) {
+    if (v8 && seq > 128 && al(v, 16) && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0 && v_strides[2] % 8 == 0)
+      return launch_full128(p, st);
     switch (head_dim) {
       case 16: return dispatch_flash<16>(p, c, st);
       case 32: return dispatch_flash<32>(p, c, st);

@@ -306,6 +306,35 @@ int tk_small_forward_supported(int64_t seq, int64_t d_model, int64_t heads,
                                int64_t head_dim_padded, int64_t ffn_dim);
 
 /*
+ * The row-local parts of a block of width 128 (tk_narrow_supported: d_model and
+ * attention width 128, ffn_dim a multiple of 128 up to 1024), fused:
+ *   tk_narrow_qkv:  qkv[rows][384] f16 = LN(x) . W_qkv^T + b
+ *   tk_narrow_tail: s = resid + ctx . W_o^T + b_o;
+ *                   s += gelu(LN(s; n2) . W_1^T + b_1) . W_2^T + b_2;
+ *                   out = LN(s; next) (out_dtype), sum_out (nullable) = s
+ * ctx [rows][128] f16, resid and sum_out [rows][128] f32 (sum_out may alias
+ * resid).  A weight W[N][K] f16 is given in fragment order: [K/128][N/32] blocks
+ * of 8 fragments of 64 lanes of 8 values, lane l of fragment kk holding row
+ * l & 31, columns 16 kk + 8 (l >> 5) .. + 8 of its block.  row_valid (nullable,
+ * rows bytes): an invalid row keeps its residual after attention and is 0 after
+ * the FFN (row_mode TK_ROWS_ZERO), its normalised output too with
+ * TK_ROWS_ZERO_ALL (f32 output).  All buffers 16-byte aligned.
+ * Replaces add_ln_fwd and F.linear / F.gelu between two attention calls
+ * (src/optimized.py:523-553,572,627-636) at that width.
+ */
+int tk_narrow_supported(int64_t d_model, int64_t attn_width, int64_t ffn_dim);
+int tk_narrow_qkv(const float *x, const float *ln_w, const float *ln_b,
+                  float eps, const tk_half *w_packed, const float *b_qkv,
+                  tk_half *qkv, int64_t rows, void *stream);
+int tk_narrow_tail(const tk_half *ctx, const float *resid, const tk_half *w_o,
+                   const float *b_o, const float *n2_w, const float *n2_b,
+                   float n2_eps, const tk_half *w_1, const float *b_1,
+                   const tk_half *w_2, const float *b_2, int64_t ffn_dim,
+                   const float *next_w, const float *next_b, float next_eps,
+                   float *sum_out, void *out, int out_dtype, int64_t rows,
+                   const uint8_t *row_valid, int row_mode, void *stream);
+
+/*
  * The layer loop of the forward: every launch of a dense or padded forward of
  * any width, enqueued by one call with the arguments the entry points above
  * take (no other work, so the results are those of the separate calls).
@@ -327,6 +356,8 @@ typedef struct tk_layer {
   const float *b_1;
   const tk_half *w_2;
   const float *b_2;
+  /* The four projections in fragment order (tk_narrow_qkv, tk_narrow_tail); NULL: not used. */
+  const tk_half *w_qkv_packed, *w_o_packed, *w_1_packed, *w_2_packed;
   float n1_eps, n2_eps;
 } tk_layer;
 
@@ -340,7 +371,9 @@ typedef struct tk_model {
 } tk_model;
 
 enum tk_forward_flags {
-  TK_FWD_FUSED_NORM = 1,   /* residual + LayerNorm in the GEMM epilogues where tk_gemm_ln_supported */
+  TK_FWD_FUSED_NORM = 1,   /* tk_narrow_qkv / tk_narrow_tail where they take the shape and every layer's
+                              packed weights are given, else residual + LayerNorm in the GEMM epilogues
+                              where tk_gemm_ln_supported */
   TK_FWD_QKV_ATTENTION = 2 /* tk_qkv_attention where it takes the shape (dense inputs) */
 };
 

@@ -15,18 +15,24 @@ namespace tk {
 namespace {
 
 enum StepKind {
-  kLnIn, kQkv, kAttn, kQkvAttn, kOutLn, kOutResid, kLn2, kUp, kDownLn, kDownResid, kLnNext, kLnFinal
+  kLnIn, kQkv, kAttn, kQkvAttn, kOutLn, kOutResid, kLn2, kUp, kDownLn, kDownResid, kLnNext, kLnFinal, kLnQkv, kTail
 };
 const char* const kStepNames[] = {"ln_in", "qkv", "flash_attn", "qkv_attn", "out_proj_ln", "out_proj_resid",
-                                  "ln2", "ffn_up_gelu", "ffn_down_ln", "ffn_down_resid", "ln_next", "ln_final"};
+                                  "ln2", "ffn_up_gelu", "ffn_down_ln", "ffn_down_resid", "ln_next", "ln_final",
+                                  "ln_qkv", "block_tail"};
 
 struct Schedule {
   bool fused_qa;  // QKV projection and attention in one kernel
   bool fuse;      // residual + LayerNorm in the GEMM epilogues
+  bool narrow;    // every row-local part of a block in one kernel
   int per_layer;
   int64_t layers;
-  int64_t steps() const { return 1 + layers * per_layer; }
+  int64_t steps() const { return (narrow ? 0 : 1) + layers * per_layer; }
+  int64_t layer_of(int64_t step) const {
+    return narrow ? step / per_layer : step == 0 ? 0 : (step - 1) / per_layer;
+  }
   StepKind kind(int64_t step) const {
+    if (narrow) return step == 0 ? kLnQkv : step % per_layer == 0 ? kQkv : step % per_layer == 1 ? kAttn : kTail;
     if (step == 0) return kLnIn;
     const int64_t layer = (step - 1) / per_layer;
     int k = (int)((step - 1) % per_layer);
@@ -49,7 +55,13 @@ Schedule schedule(const tk_model& m, int64_t batch, int64_t seq, bool dense, int
   s.fused_qa = dense && (flags & TK_FWD_QKV_ATTENTION) && m.heads * m.head_dim == m.d_model &&
                tk_qkv_attention_supported(batch, seq, m.heads, m.head_dim);
   s.fuse = (flags & TK_FWD_FUSED_NORM) && tk_gemm_ln_supported(m.d_model);
-  s.per_layer = (s.fused_qa ? 1 : 2) + (s.fuse ? 3 : 5);
+  bool packed = true;
+  for (int64_t i = 0; i < m.num_layers; ++i)
+    packed = packed && m.layers[i].w_qkv_packed && m.layers[i].w_o_packed && m.layers[i].w_1_packed &&
+             m.layers[i].w_2_packed;
+  s.narrow = packed && !s.fused_qa && (flags & TK_FWD_FUSED_NORM) &&
+             tk_narrow_supported(m.d_model, m.heads * m.head_dim, m.ffn_dim);
+  s.per_layer = s.narrow ? 3 : (s.fused_qa ? 1 : 2) + (s.fuse ? 3 : 5);
   s.layers = m.num_layers;
   return s;
 }
@@ -130,7 +142,7 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
   tk_half* u = qkv;
   const int64_t in_st[3] = {seq * 3 * dp, hd, 3 * dp}, out_st[3] = {seq * dp, hd, dp};
   for (int64_t i = first_step; i < first_step + num_steps; ++i) {
-    const int64_t li = i == 0 ? 0 : (i - 1) / s.per_layer;
+    const int64_t li = s.layer_of(i);
     const tk_layer& w = m->layers[li];
     const bool last = li + 1 == m->num_layers;
     // Residual input of the first layer's attention update: the caller's x, which is never written.
@@ -178,6 +190,14 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
       case kDownResid:
         rc = tk_gemm(u, f, w.w_2, f, w.b_2, resid, d, resid, d, t, d, f, TK_EPI_BIAS_RESID, valid,
                      valid ? TK_ROWS_ZERO : 0, stream);
+        break;
+      case kLnQkv:
+        rc = tk_narrow_qkv(x, w.n1_w, w.n1_b, w.n1_eps, w.w_qkv_packed, w.b_qkv, qkv, t, stream);
+        break;
+      case kTail:
+        rc = tk_narrow_tail(ctx, src, w.w_o_packed, w.b_o, w.n2_w, w.n2_b, w.n2_eps, w.w_1_packed, w.b_1,
+                            w.w_2_packed, w.b_2, f, nw, nb, ne, last ? nullptr : resid, ndst, ndt, t, valid,
+                            valid ? (last ? TK_ROWS_ZERO_ALL : TK_ROWS_ZERO) : 0, stream);
         break;
       case kLnNext:
       case kLnFinal:

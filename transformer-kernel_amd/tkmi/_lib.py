@@ -29,7 +29,8 @@ class Layer(ctypes.Structure):
     """tk_layer of include/tkmi.h."""
 
     _fields_ = [(n, c_void_p) for n in ("n1_w", "n1_b", "w_qkv", "b_qkv", "w_o", "b_o", "n2_w", "n2_b", "w_1", "b_1",
-                                        "w_2", "b_2")] + [("n1_eps", c_float), ("n2_eps", c_float)]
+                                        "w_2", "b_2", "w_qkv_packed", "w_o_packed",
+                                        "w_1_packed", "w_2_packed")] + [("n1_eps", c_float), ("n2_eps", c_float)]
 
 
 class Model(ctypes.Structure):
@@ -96,6 +97,15 @@ SIGNATURES = {
         + [c_void_p] * 11 + [c_float, c_float, c_float, c_float, c_void_p],
     ),
     "tk_small_forward_supported": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "tk_narrow_supported": (c_int, [c_int64, c_int64, c_int64]),
+    "tk_narrow_qkv": (
+        c_int, [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]
+    ),
+    "tk_narrow_tail": (
+        c_int,
+        [c_void_p] * 6 + [c_float] + [c_void_p] * 4 + [c_int64, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_int,
+                                                       c_int64, c_void_p, c_int, c_void_p],
+    ),
     "tk_forward_workspace": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),
     "tk_forward_steps": (c_int64, [c_void_p, c_int64, c_int64, c_int, c_int]),
     "tk_forward_step_name": (ctypes.c_char_p, [c_void_p, c_int64, c_int64, c_int, c_int, c_int64]),

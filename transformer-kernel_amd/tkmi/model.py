@@ -114,6 +114,18 @@ class _LayerWeights:
     b_1: torch.Tensor
     w_2: torch.Tensor  # [D, F]
     b_2: torch.Tensor
+    # The same in the narrow kernels' fragment order (width 128 only, else None; made
+    # when the layer path first runs).
+    w_qkv_packed: Optional[torch.Tensor] = None
+    w_o_packed: Optional[torch.Tensor] = None
+    w_1_packed: Optional[torch.Tensor] = None
+    w_2_packed: Optional[torch.Tensor] = None
+
+
+def _fragments(w: torch.Tensor) -> torch.Tensor:
+    """A packed weight [N, K] as [K/128][N/32] blocks of MFMA fragments (include/tkmi.h, tk_narrow_tail)."""
+    n, k = w.shape
+    return w.view(n // 32, 32, k // 128, 8, 2, 8).permute(2, 0, 3, 4, 1, 5).contiguous()
 
 
 # Head dims the attention kernel has tiles for (tk_attention_supported).
@@ -219,11 +231,15 @@ class OptimizedTransformer(BaselineTransformer):
         """Addresses of the packed weights as the library's host call takes them."""
         built = self._weights()
         if self._native is None:
+            if ops.narrow_supported(self.d_model, self.num_heads * self.head_dim_padded, self.config.ffn_dim):
+                for lw in built:
+                    lw.w_qkv_packed, lw.w_o_packed = _fragments(lw.w_qkv), _fragments(lw.w_o)
+                    lw.w_1_packed, lw.w_2_packed = _fragments(lw.w_1), _fragments(lw.w_2)
             layers = (_lib.Layer * len(built))()
             for dst, lw in zip(layers, built):
                 for name, _ in _lib.Layer._fields_:
                     val = getattr(lw, name)
-                    setattr(dst, name, val if name.endswith("_eps") else val.data_ptr())
+                    setattr(dst, name, val.data_ptr() if isinstance(val, torch.Tensor) else val)
             nf_w, nf_b, nf_eps = self._final
             self._native = _lib.Model(
                 d_model=self.d_model, heads=self.num_heads, head_dim=self.head_dim_padded,

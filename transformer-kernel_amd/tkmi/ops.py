@@ -365,6 +365,10 @@ def small_forward(x, out, stacked: dict, final: tuple, n1_eps: float, n2_eps: fl
     return out
 
 
+def narrow_supported(d_model: int, attn_width: int, ffn_dim: int) -> bool:
+    return bool(_lib.load().tk_narrow_supported(d_model, attn_width, ffn_dim))
+
+
 def transformer_forward(model: "_lib.Model", x, out, valid, flags: int) -> None:
     """Every launch of a forward by one call into the library (tk_forward).
 

@@ -371,10 +371,12 @@ typedef struct tk_model {
 } tk_model;
 
 enum tk_forward_flags {
-  TK_FWD_FUSED_NORM = 1,   /* tk_narrow_qkv / tk_narrow_tail where they take the shape and every layer's
+  TK_FWD_FUSED_NORM = 1,    /* tk_narrow_qkv / tk_narrow_tail where they take the shape and every layer's
                               packed weights are given, else residual + LayerNorm in the GEMM epilogues
                               where tk_gemm_ln_supported */
-  TK_FWD_QKV_ATTENTION = 2 /* tk_qkv_attention where it takes the shape (dense inputs) */
+  TK_FWD_QKV_ATTENTION = 2, /* tk_qkv_attention where it takes the shape (dense inputs) */
+  TK_FWD_BATCH_INVARIANT = 4 /* no kernel whose choice and order of sums depend on the batch size: a
+                                sequence's output bits are the same in every batch */
 };
 
 /* Bytes of the workspace that tk_forward needs; negative: a tk_status. */

@@ -34,7 +34,7 @@
 // into one FMA before exp2: exp2(s*c - m*c) = exp(scale*(s - m))), -inf
 // masking of future and invalid keys, fp32 running max and sums, fp16 P for
 // the PV product, fp32 accumulation, one final divide.
-#include "tk_attn_tile.hpp"
+#include "tk_attn_keysplit.hpp"
 
 namespace tk {
 namespace {
@@ -1943,6 +1943,35 @@ int launch_single(const AttnArgs& p, bool causal, hipStream_t st) {
   return check_launch("tk_flash_attn_fwd");
 }
 
+template <int HD, int NW, bool CAUSAL, bool KMASK>
+__global__ __launch_bounds__(NW * 64, HD <= 64 ? 2 : 1) void flash_keysplit_kernel(AttnArgs p) {
+  keysplit_body<HD, NW, CAUSAL, KMASK>(p);
+}
+// Where the key-split kernel is taken: head dims 32, 64 and 128, more than one key
+// tile, and at most two workgroups of it per CU (32 query rows each).  Measured on 87
+// launches, us (others -> key split): b1 h16 s512 causal, head_dim 64 10.1 -> 5.7,
+// 128 23.8 -> 8.9, 32 8.6 -> 4.7; b1 h4 s2048 23.1 -> 11.0 (eight waves); at 512
+// workgroups b1 h16 s1024 without the causal mask 14.1 -> 11.8, 128 31.6 -> 25.3,
+// 32 12.8 -> 8.4.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs 12.6,
+// b1 h16 s2048 full 26.1 vs 35.5) except for head_dim 32 causal (b1 h16 s2048 24.5 ->
+// 18.3, b64 h4 s128 6.6 -> 6.4).  Eight waves: from 1024 keys, one workgroup per CU
+// (b1 h1 s4096 22.7 -> 17.7; b1 h16 s512 5.7 vs 5.9).
+int64_t keysplit_blocks(int64_t bh, int64_t s) { return bh * ((s + 31) / 32); }
+bool keysplit_pays(int64_t bh, int64_t s, int64_t hd, bool causal) {
+  return (hd == 32 || hd == 64 || hd == 128) && s > 64 &&
+         keysplit_blocks(bh, s) <= (hd == 32 && causal ? 1024 : 512);
+}
+template <int HD, int NW>
+int launch_keysplit(const AttnArgs& p, bool causal, hipStream_t st) {
+  const dim3 g((unsigned)((int64_t)((p.S + 31) / 32) * p.B * p.H)), blk(NW * 64);
+  const bool km = p.kv != nullptr;
+  if (causal && km) hipLaunchKernelGGL((flash_keysplit_kernel<HD, NW, true, true>), g, blk, 0, st, p);
+  else if (causal) hipLaunchKernelGGL((flash_keysplit_kernel<HD, NW, true, false>), g, blk, 0, st, p);
+  else if (km) hipLaunchKernelGGL((flash_keysplit_kernel<HD, NW, false, true>), g, blk, 0, st, p);
+  else hipLaunchKernelGGL((flash_keysplit_kernel<HD, NW, false, false>), g, blk, 0, st, p);
+  return check_launch("tk_flash_attn_fwd");
+}
+
 template <int HD, int NW>
 int launch_flash(const AttnArgs& p, bool causal, hipStream_t st) {
   constexpr int BM = 32 * NW;
@@ -2000,12 +2029,10 @@ int64_t head_dim_block(int64_t hd) {
 }
 }  // namespace
 
-extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* out,
-                                 int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
-                                 const int64_t* q_strides, const int64_t* k_strides,
-                                 const int64_t* v_strides, const int64_t* o_strides, float scale,
-                                 int causal, const uint8_t* key_valid, int64_t key_valid_stride,
-                                 void* stream) {
+int tk::flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* out, int64_t batch, int64_t heads,
+                   int64_t seq, int64_t head_dim, const int64_t* q_strides, const int64_t* k_strides,
+                   const int64_t* v_strides, const int64_t* o_strides, float scale, int causal,
+                   const uint8_t* key_valid, int64_t key_valid_stride, bool batch_invariant, void* stream) {
   TK_REQUIRE(q && k && v && out && q_strides && k_strides && v_strides && o_strides, TK_ERR_ARG,
              "tk_flash_attn_fwd: null pointer");
   TK_REQUIRE(head_dim >= 0, TK_ERR_ARG, "tk_flash_attn_fwd: head_dim=%lld < 0", (long long)head_dim);
@@ -2044,8 +2071,14 @@ extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_ha
     vec = vec && q_strides[i] % 8 == 0 && k_strides[i] % 8 == 0 && v_strides[i] % (v8 ? 4 : 8) == 0 &&
           o_strides[i] % 4 == 0;
   if (vec) {
-    if (v8 && seq > 128 && al(v, 16) && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0 && v_strides[2] % 8 == 0)
-      return launch_full128(p, st);
+    const bool v16 = al(v, 16) && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0 && v_strides[2] % 8 == 0;
+    if (v16 && !batch_invariant && keysplit_pays(batch * heads, seq, head_dim, c)) {
+      const bool w8 = keysplit_blocks(batch * heads, seq) <= 256 && seq > 1024;
+      if (head_dim == 32) return w8 ? launch_keysplit<32, 8>(p, c, st) : launch_keysplit<32, 4>(p, c, st);
+      if (head_dim == 64) return w8 ? launch_keysplit<64, 8>(p, c, st) : launch_keysplit<64, 4>(p, c, st);
+      return launch_keysplit<128, 4>(p, c, st);
+    }
+    if (v8 && seq > 128 && v16) return launch_full128(p, st);
     switch (head_dim) {
       case 16: return dispatch_flash<16>(p, c, st);
       case 32: return dispatch_flash<32>(p, c, st);
@@ -2065,4 +2098,14 @@ extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_ha
     case 128: return launch_generic<128>(p, hd, c, st);
     default: return launch_generic<256>(p, hd, c, st);
   }
+}
+
+extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* out,
+                                 int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
+                                 const int64_t* q_strides, const int64_t* k_strides,
+                                 const int64_t* v_strides, const int64_t* o_strides, float scale,
+                                 int causal, const uint8_t* key_valid, int64_t key_valid_stride,
+                                 void* stream) {
+  return flash_attn(q, k, v, out, batch, heads, seq, head_dim, q_strides, k_strides, v_strides, o_strides, scale,
+                    causal, key_valid, key_valid_stride, false, stream);
 }

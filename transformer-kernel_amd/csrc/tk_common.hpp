@@ -98,6 +98,13 @@ int check_launch(const char* what);
     }                                    \
   } while (0)
 
+// tk_flash_attn_fwd; batch_invariant: no kernel choice that depends on the batch
+// size, so that a sequence's output bits don't.
+int flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* out, int64_t batch, int64_t heads,
+               int64_t seq, int64_t head_dim, const int64_t* q_strides, const int64_t* k_strides,
+               const int64_t* v_strides, const int64_t* o_strides, float scale, int causal, const uint8_t* key_valid,
+               int64_t key_valid_stride, bool batch_invariant, void* stream);
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ------------------------------------------------------- wave reductions --

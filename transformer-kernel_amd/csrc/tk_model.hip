@@ -140,6 +140,7 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
   tk_half* ctx = reinterpret_cast<tk_half*>(ws + l.ctx);
   tk_half* qkv = reinterpret_cast<tk_half*>(ws + l.shared);
   tk_half* u = qkv;
+  const bool invariant = flags & TK_FWD_BATCH_INVARIANT;
   const int64_t in_st[3] = {seq * 3 * dp, hd, 3 * dp}, out_st[3] = {seq * dp, hd, dp};
   for (int64_t i = first_step; i < first_step + num_steps; ++i) {
     const int64_t li = s.layer_of(i);
@@ -163,8 +164,8 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
                      stream);
         break;
       case kAttn:
-        rc = tk_flash_attn_fwd(qkv, qkv + dp, qkv + 2 * dp, ctx, batch, nh, seq, hd, in_st, in_st, in_st, out_st,
-                               m->scale, m->causal, valid, seq, stream);
+        rc = flash_attn(qkv, qkv + dp, qkv + 2 * dp, ctx, batch, nh, seq, hd, in_st, in_st, in_st, out_st, m->scale,
+                        m->causal, valid, seq, invariant, stream);
         break;
       case kQkvAttn:
         rc = tk_qkv_attention(h, d, w.w_qkv, d, w.b_qkv, ctx, dp, batch, seq, nh, hd, m->scale, m->causal, stream);

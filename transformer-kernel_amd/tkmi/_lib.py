@@ -20,7 +20,7 @@ TK_F32, TK_F16 = 0, 1
 TK_EPI_BIAS, TK_EPI_BIAS_GELU, TK_EPI_BIAS_RESID = 0, 1, 2
 TK_ROWS_KEEP_RESID, TK_ROWS_ZERO, TK_ROWS_ZERO_ALL = 1, 2, 3
 
-TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION = 1, 2
+TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION, TK_FWD_BATCH_INVARIANT = 1, 2, 4
 
 _I64_3 = c_int64 * 3
 

@@ -32,11 +32,12 @@ import argparse
 import json
 import statistics
 import sys
+from dataclasses import replace
 from typing import Dict, Optional
 
 import torch
 
-from .model import OptimizedTransformer
+from .model import OptimizedTransformer, active_settings
 from .modules import TransformerConfig
 
 # src/run_case14.py:67-75 (the case's shape)
@@ -45,9 +46,11 @@ CASE = dict(batch_size=32, seq_len=100000, d_model=1024, num_heads=16, ffn_dim=1
 
 def make_model(config: TransformerConfig, seed: int, device: str = "cuda") -> OptimizedTransformer:
     """Seeded weights in the baseline's construction order (torch.manual_seed(seed)
-    then the module tree), as the reference's build_pair (src/run_case14.py:115-128)."""
+    then the module tree), as the reference's build_pair (src/run_case14.py:115-128).
+    Batch-invariant: a chunk's outputs are the whole batch's, bit for bit."""
     torch.manual_seed(seed)
-    return OptimizedTransformer(config).to(device).eval()
+    settings = replace(active_settings(), batch_invariant=True)
+    return OptimizedTransformer(config, settings).to(device).eval()
 
 
 def sample_inputs(config: TransformerConfig, seed: int, start: int, stop: int, device: str = "cuda") -> torch.Tensor:
@@ -129,10 +132,15 @@ def time_streamed(model, host_x: torch.Tensor, chunk: int, warmup: int, repeats:
 
 
 def check_chunks(model, x: torch.Tensor, chunk: int) -> Dict[str, float]:
-    """Chunked forward against the resident forward of the same samples."""
-    with torch.inference_mode():
-        whole = model(x)
-        parts = torch.cat([model(x[s:s + chunk]) for s in range(0, x.shape[0], chunk)])
+    """Chunked forward against the resident forward of the same samples, both batch-invariant."""
+    settings = model.settings
+    model.settings = replace(settings, batch_invariant=True)
+    try:
+        with torch.inference_mode():
+            whole = model(x)
+            parts = torch.cat([model(x[s:s + chunk]) for s in range(0, x.shape[0], chunk)])
+    finally:
+        model.settings = settings
     diff = (whole.float() - parts.float()).abs()
     return {"max_abs": float(diff.max().item()), "bit_exact": bool(torch.equal(whole, parts))}
 

@@ -41,7 +41,7 @@ from typing import List, Optional
 import torch
 
 from . import _lib, ops
-from ._lib import TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION
+from ._lib import TK_FWD_BATCH_INVARIANT, TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION
 from .modules import BaselineTransformer
 
 __all__ = ["OptimizerSettings", "OptimizedTransformer", "configure", "active_settings"]
@@ -69,6 +69,10 @@ class OptimizerSettings:
     qkv_attention     -- for dense one-key-tile sequences (S = 64, head_dim
                          64) run the QKV projection and attention as one
                          kernel (tk_qkv_attention), q/k/v kept on chip.
+    batch_invariant   -- only kernels whose order of sums does not depend on the
+                         batch size, so that a sequence's output bits are the
+                         same whatever batch it is in; off (default), launches
+                         that would leave the chip idle split their sums.
     """
 
     fused_norm: bool = True
@@ -76,6 +80,7 @@ class OptimizerSettings:
     assume_dense_mask: bool = False
     small_forward: bool = True
     qkv_attention: bool = True
+    batch_invariant: bool = False
 
 
 _ACTIVE = OptimizerSettings()
@@ -336,5 +341,7 @@ class OptimizedTransformer(BaselineTransformer):
             flags |= TK_FWD_FUSED_NORM
         if self.settings.qkv_attention:
             flags |= TK_FWD_QKV_ATTENTION
+        if self.settings.batch_invariant:
+            flags |= TK_FWD_BATCH_INVARIANT
         ops.transformer_forward(self._native_model(), xin.view(bsz, seq, d), out, mask, flags)
         return out

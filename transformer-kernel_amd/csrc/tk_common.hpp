@@ -105,6 +105,11 @@ int flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* ou
                const int64_t* v_strides, const int64_t* o_strides, float scale, int causal, const uint8_t* key_valid,
                int64_t key_valid_stride, bool batch_invariant, void* stream);
 
+// tk_gemm, likewise.
+int gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const float* bias, const float* resid,
+         int64_t ldr, void* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int epilogue, const uint8_t* row_valid,
+         int row_mode, bool batch_invariant, void* stream);
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ------------------------------------------------------- wave reductions --

@@ -48,6 +48,7 @@ struct GemmArgs {
   float eps;
   bool vec;     // output rows admit 4-wide vector stores
   bool bias16;  // bias is 16-byte aligned
+  bool one_order;  // one order of sums for every M and N (TK_FWD_BATCH_INVARIANT)
   bool kvec;    // K, lda, ldw multiples of 8 and A, W 16-byte aligned: 16-byte operand loads
   int64_t w_gstride;  // grouped W rows (Mainloop WG > 0): group stride in rows
 };
@@ -160,9 +161,12 @@ __device__ __forceinline__ void phase_barrier() {
 // one head in the fused QKV weight); every row must exist.
 // PP (direct path, 256 x 256 tiles of 4 x 2 waves, BK 64, two stages, whole
 // tiles only): the ping-pong K loop, run_pingpong below.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool DIRECT, int WG = 0, bool PP = false>
+// KG > 1 (direct path): KG groups of WAVES_M x WAVES_N waves, each with stages of
+// its own, accumulate a KG-th of the K-tiles each; merge_groups adds their sums.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool DIRECT, int WG = 0, bool PP = false,
+          int KG = 1>
 struct Mainloop {
-  static constexpr int NW = WAVES_M * WAVES_N;
+  static constexpr int NW = WAVES_M * WAVES_N;  // waves of a group
   static constexpr int NT = 64 * NW;
   static constexpr bool PINGPONG = PP;
   static constexpr int WM = BM / WAVES_M;
@@ -177,7 +181,9 @@ struct Mainloop {
   static constexpr int W_INSTS = BN / RPC / NW;
   static constexpr int INSTS = A_INSTS + W_INSTS;
   static constexpr int KSTEPS = BK / 16;
-  static constexpr int LDS_HALVES = STAGES * (BM + BN) * BK;
+  static constexpr int GROUP_HALVES = STAGES * (BM + BN) * BK;
+  static constexpr int LDS_HALVES = KG * GROUP_HALVES;
+  static_assert(KG == 1 || (DIRECT && !PP && WG == 0), "K groups: direct path");
   static_assert(BK == 32 || BK == 64, "BK is 32 or 64");
   static_assert(KSTEPS % 2 == 0, "even number of k-steps per K-tile");
   static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be a multiple of 32");
@@ -382,16 +388,22 @@ struct Mainloop {
     }
   }
 
-  __device__ __forceinline__ static void run_direct(const GemmArgs& p, int m0, int n0, f16* smem, f32x16 (&acc)[FN][FM]) {
+  // KG wave groups: group kg accumulates the K-tiles [kg, kg + 1) * nk / KG.
+  __device__ __forceinline__ static void run_direct(const GemmArgs& p, int m0, int n0, f16* smem_all,
+                                                    f32x16 (&acc)[FN][FM]) {
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = KG == 1 ? wave_all : wave_all % NW;
+    const int kg = KG == 1 ? 0 : wave_all / NW;
+    f16* smem = smem_all + kg * GROUP_HALVES;
     const int wm = wave % WAVES_M;
     const int wn = wave / WAVES_M;
     f16* As = smem;                      // [STAGES][BM][BK]
     f16* Ws = smem + STAGES * BM * BK;   // [STAGES][BN][BK]
     const uint32_t lds_a = (uint32_t)(size_t)(lds_char*)As;
     const uint32_t lds_w = (uint32_t)(size_t)(lds_char*)Ws;
-    const int nk = p.K / BK;
+    const int nk = p.K / (BK * KG);
+    const int k0 = kg * nk * BK;
 
     const f16* ga[A_INSTS];
     const f16* gw[W_INSTS];
@@ -399,16 +411,16 @@ struct Mainloop {
     for (int i = 0; i < A_INSTS; ++i) {
       const int r = (wave * A_INSTS + i) * RPC + lane / CPR;
       const int c = swz<BK>(r, lane % CPR) - r * BK;  // physical -> logical is the same XOR
-      ga[i] = p.a + (int64_t)min(m0 + r, p.M - 1) * p.lda + c;
+      ga[i] = p.a + (int64_t)min(m0 + r, p.M - 1) * p.lda + (c + k0);
     }
 #pragma unroll
     for (int i = 0; i < W_INSTS; ++i) {
       const int r = (wave * W_INSTS + i) * RPC + lane / CPR;
       const int c = swz<BK>(r, lane % CPR) - r * BK;
       if constexpr (WG > 0)
-        gw[i] = p.w + (n0 + (int64_t)(r / WG) * p.w_gstride + r % WG) * p.ldw + c;
+        gw[i] = p.w + (n0 + (int64_t)(r / WG) * p.w_gstride + r % WG) * p.ldw + (c + k0);
       else
-        gw[i] = p.w + (int64_t)min(n0 + r, p.N - 1) * p.ldw + c;
+        gw[i] = p.w + (int64_t)min(n0 + r, p.N - 1) * p.ldw + (c + k0);
     }
     // Wave copy c of tile kt into `stage`: copies 0..A_INSTS-1 are A rows,
     // the rest W rows, 1 KB each.
@@ -496,6 +508,45 @@ struct Mainloop {
       ksteps();
       mma(1);
     }
+  }
+
+  // After every group's loop and a barrier: the sums of groups 1.. pass through
+  // their own LDS to group 0, which adds them in that order and returns true.
+  __device__ __forceinline__ static bool merge_groups(f16* smem, f32x16 (&acc)[FN][FM]) {
+    static_assert(GROUP_HALVES * 2 >= NW * FN * FM * 4096, "a group's sums fit its stages");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave / NW;
+    auto slot = [&](int g, int i, int j, int q) {
+      char* base = reinterpret_cast<char*>(smem + g * GROUP_HALVES) + (wave % NW) * (FN * FM * 4096);
+      return reinterpret_cast<f32x4*>(base + ((i * FM + j) * 4 + q) * 1024 + lane * 16);
+    };
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x16& a = acc[i][j];
+            *slot(kg, i, j, q) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+          }
+    }
+    __syncthreads();
+    if (kg > 0) return false;
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 v = *slot(g, i, j, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += v[e];
+          }
+    return true;
   }
 
   __device__ __forceinline__ static void run_staged(const GemmArgs& p, int m0, int n0, f16* smem, f32x16 (&acc)[FN][FM]) {
@@ -603,9 +654,18 @@ struct Tile {
   static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int BK = BK_, STAGES = STAGES_;
   static constexpr bool PP = PP_;
+  static constexpr int KG = 1;
   static constexpr int NT = 64 * WAVES_M_ * WAVES_N_;
   template <bool DIRECT>
   using ML = Mainloop<BM, BN, WAVES_M, WAVES_N, DIRECT ? BK : 64, DIRECT ? STAGES : 2, DIRECT, 0, PP && DIRECT>;
+};
+// The same tile by KG_ groups of its waves, each with a KG_-th of the K loop (direct path).
+template <class T, int KG_>
+struct KSplit : T {
+  static constexpr int KG = KG_;
+  static constexpr int NT = T::NT * KG_;
+  template <bool DIRECT>
+  using ML = Mainloop<T::BM, T::BN, T::WAVES_M, T::WAVES_N, T::BK, T::STAGES, DIRECT, 0, false, KG_>;
 };
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a row-major LDS
@@ -641,7 +701,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& p, const f32x16 (
   constexpr int WM = ML::WM, WN = ML::WN, FM = ML::FM, FN = ML::FN, NW = ML::NW;
   constexpr int ROWB = WN * 2;
   constexpr int CPR = ROWB / 16;
-  constexpr int LDS_BYTES = ML::LDS_HALVES * 2;
+  constexpr int LDS_BYTES = ML::GROUP_HALVES * 2;
   constexpr int JC = (NW * FM * 32 * ROWB <= LDS_BYTES) ? FM : (NW * 32 * ROWB <= LDS_BYTES ? 1 : 0);
   static_assert(JC > 0 && FM % JC == 0, "staging region does not fit");
   constexpr int EPC = 8;  // elements per chunk
@@ -924,7 +984,7 @@ __device__ __forceinline__ void store_tile_resid(const GemmArgs& p, const f32x16
                                                  int n0, f16* smem, int m_lo, int n_lo) {
   constexpr int FM = ML::FM, NW = ML::NW;
   constexpr int ROWB = ML::WN * 4;
-  constexpr int LDS_BYTES = ML::LDS_HALVES * 2;
+  constexpr int LDS_BYTES = ML::GROUP_HALVES * 2;
   constexpr int JC = (NW * FM * 32 * ROWB <= LDS_BYTES) ? FM : (NW * 32 * ROWB <= LDS_BYTES ? 1 : 0);
   static_assert(JC > 0 && FM % JC == 0 && FM / JC <= 2, "staging region does not fit");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1053,6 +1113,8 @@ __global__ __launch_bounds__(T::NT) void gemm_kernel(GemmArgs p) {
   // completed before group 0's last barrier, so group 0 starts its epilogue
   // while group 1 issues the last K-tile's MFMAs.
   if constexpr (!ML::PINGPONG) __syncthreads();
+  if constexpr (T::KG > 1)
+    if (!ML::merge_groups(smem, acc)) return;
   if constexpr (EPI == TK_EPI_BIAS_RESID || EPI == kEpiResidRows)
     store_tile_resid<ML, T::WAVES_M, EPI == kEpiResidRows, ML::PINGPONG>(p, acc, m0, n0, smem, tm * BM, tn * BN);
   else
@@ -1239,6 +1301,8 @@ using TileWide3 = Tile<128, 256, 2, 4, 64, 3>;  // 8 waves of 64 x 64, 1 block p
 using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
 using TileTall3 = Tile<128, 64, 4, 2, 64, 3>;  // the same, two K-tiles in flight
 using TileSmall = Tile<64, 64, 2, 2, 64, 3>;   // 4 waves of 32 x 32, 3 blocks per CU
+using TileWide32 = Tile<32, 64, 1, 2, 64, 3>;  // K groups of 2 waves (36 KB LDS each)
+using Tile32 = Tile<32, 32, 1, 1, 64, 3>;      // K groups of 1 wave (24 KB LDS each)
 
 #ifndef TK_GEMM_PF
 #define TK_GEMM_PF 1
@@ -1260,7 +1324,8 @@ int launch_pingpong(const GemmArgs& p, int64_t tiles, hipStream_t st) {
 // Every figure: MI355X, us per launch, operands rotated through four buffers,
 // all tiles timed on 200 shapes (M 16 .. 30000, N 384 .. 6144, K 256 .. 4096,
 // the three epilogues).  Per accumulator the k order is the same for every
-// tile, so the choice never changes a result.
+// tile but the K-split ones, which one_order rules out: the choice then never
+// changes a result.
 template <int EPI>
 int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   const int64_t t256 = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
@@ -1298,8 +1363,25 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   if (p.K >= 512 && fill >= (rounds == 1 ? 0.62 : 0.8)) return launch_gemm<TileBig, EPI, true>(p, st);
   // Up to one workgroup per CU the K loop is a chain of copy latencies: the
   // smallest tile that keeps every workgroup resident, more waves on each and
-  // two K-tiles in flight.  Four-wave 64 x 64 tiles: M512 N1024 K4096 35.3
-  // (one wave, one K-tile in flight) -> 20.6, M128 N3072 K1024 12.5 -> 7.7.
+  // two K-tiles in flight.  From K = 768 the K loop is split over two or four
+  // groups of the workgroup's waves (KSplit), whose chains run side by side:
+  // four groups on 32 x 32 tiles (M64 N2048 K8192 37.9 on four-wave 64 x 64 tiles ->
+  // 15.1, M256 N1024 K1024 7.2 -> 4.8) or, past 256 of them, 32 x 64 (M512 N1024
+  // K4096 20.6 -> 12.4, M128 N4096 K1024 7.8 -> 6.2), then two on 64 x 64 (M1024
+  // N1024 K4096 23.1 -> 17.3, M1500 N512 K2048 11.9 -> 10.0).  Past those 128 x 64
+  // tiles with two groups are within 3 % of one (M2048 N1024 K4096 27.3 vs 28.1,
+  // M1024 N2048 K2048 15.6 vs 15.2).  Below K = 768 every launch keeps one order of
+  // sums, that of the fused QKV + attention kernel; the split saves 0.2 to 1 us there.
+  if (!p.one_order && p.K >= 768) {
+    const int64_t t32 = (int64_t)((p.M + 31) / 32) * ((p.N + 31) / 32);
+    const int64_t wide32 = (int64_t)((p.M + 31) / 32) * ((p.N + 63) / 64);
+    if (t32 <= 256 && p.K % 256 == 0) return launch_gemm<KSplit<Tile32, 4>, EPI, true>(p, st);
+    if (wide32 <= 256 && p.K % 256 == 0) return launch_gemm<KSplit<TileWide32, 4>, EPI, true>(p, st);
+    if (wide32 <= 256 && p.K % 128 == 0) return launch_gemm<KSplit<TileWide32, 2>, EPI, true>(p, st);
+    if (t64 <= 256 && p.K % 128 == 0) return launch_gemm<KSplit<TileSmall, 2>, EPI, true>(p, st);
+  }
+  // Four-wave 64 x 64 tiles: M512 N1024 K4096 35.3 (one wave, one K-tile in
+  // flight) -> 20.6, M128 N3072 K1024 12.5 -> 7.7.
   if (t64 <= 256) return launch_gemm<TileSmall, EPI, true>(p, st);
   // 128 x 64: M512 N4096 K1024 15.8 -> 10.1, M2048 N1024 K4096 41.2 -> 28.4.
   if (tall <= 256) return launch_gemm<TileTall3, EPI, true>(p, st);
@@ -1416,10 +1498,9 @@ bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
 
 using namespace tk;
 
-extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw,
-                       const float* bias, const float* resid, int64_t ldr, void* c, int64_t ldc,
-                       int64_t m, int64_t n, int64_t k, int epilogue, const uint8_t* row_valid,
-                       int row_mode, void* stream) {
+int tk::gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const float* bias, const float* resid,
+             int64_t ldr, void* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int epilogue,
+             const uint8_t* row_valid, int row_mode, bool batch_invariant, void* stream) {
   TK_REQUIRE(a && w && c, TK_ERR_ARG, "tk_gemm: null pointer");
   TK_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31),
              TK_ERR_ARG, "tk_gemm: bad sizes m=%lld n=%lld k=%lld", (long long)m, (long long)n,
@@ -1440,6 +1521,7 @@ extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t 
   GemmArgs p{};
   p.row_valid = row_valid;
   p.row_mode = row_mode;
+  p.one_order = batch_invariant;
   // 16-byte vector stores (and residual loads) when every output row start
   // is aligned for them; element-wise otherwise.
   if (epilogue == TK_EPI_BIAS_RESID)
@@ -1462,6 +1544,13 @@ extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t 
     default:
       return p.row_valid ? gemm_dispatch<kEpiResidRows>(p, st) : gemm_dispatch<TK_EPI_BIAS_RESID>(p, st);
   }
+}
+
+extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw,
+                       const float* bias, const float* resid, int64_t ldr, void* c, int64_t ldc,
+                       int64_t m, int64_t n, int64_t k, int epilogue, const uint8_t* row_valid,
+                       int row_mode, void* stream) {
+  return gemm(a, lda, w, ldw, bias, resid, ldr, c, ldc, m, n, k, epilogue, row_valid, row_mode, false, stream);
 }
 
 extern "C" int tk_gemm_ln_supported(int64_t n) { return n == 128 || n == 256 || n == 512; }

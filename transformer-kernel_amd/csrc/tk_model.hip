@@ -160,8 +160,8 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
         rc = tk_ln_cast(x, w.n1_w, w.n1_b, h, TK_F16, t, d, w.n1_eps, nullptr, stream);
         break;
       case kQkv:
-        rc = tk_gemm(h, d, w.w_qkv, d, w.b_qkv, nullptr, 0, qkv, 3 * dp, t, 3 * dp, d, TK_EPI_BIAS, nullptr, 0,
-                     stream);
+        rc = gemm(h, d, w.w_qkv, d, w.b_qkv, nullptr, 0, qkv, 3 * dp, t, 3 * dp, d, TK_EPI_BIAS, nullptr, 0, invariant,
+                  stream);
         break;
       case kAttn:
         rc = flash_attn(qkv, qkv + dp, qkv + 2 * dp, ctx, batch, nh, seq, hd, in_st, in_st, in_st, out_st, m->scale,
@@ -175,22 +175,22 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
                                  w.n2_eps, valid, valid ? TK_ROWS_KEEP_RESID : 0, stream);
         break;
       case kOutResid:
-        rc = tk_gemm(ctx, dp, w.w_o, dp, w.b_o, src, d, resid, d, t, d, dp, TK_EPI_BIAS_RESID, valid,
-                     valid ? TK_ROWS_KEEP_RESID : 0, stream);
+        rc = gemm(ctx, dp, w.w_o, dp, w.b_o, src, d, resid, d, t, d, dp, TK_EPI_BIAS_RESID, valid,
+                  valid ? TK_ROWS_KEEP_RESID : 0, invariant, stream);
         break;
       case kLn2:
         rc = tk_ln_cast(resid, w.n2_w, w.n2_b, h, TK_F16, t, d, w.n2_eps, nullptr, stream);
         break;
       case kUp:
-        rc = tk_gemm(h, d, w.w_1, d, w.b_1, nullptr, 0, u, f, t, f, d, TK_EPI_BIAS_GELU, nullptr, 0, stream);
+        rc = gemm(h, d, w.w_1, d, w.b_1, nullptr, 0, u, f, t, f, d, TK_EPI_BIAS_GELU, nullptr, 0, invariant, stream);
         break;
       case kDownLn:  // the summed residual is dead after the last layer
         rc = tk_gemm_bias_add_ln(u, f, w.w_2, f, w.b_2, resid, nw, nb, last ? nullptr : resid, ndst, ndt, t, d, f,
                                  ne, valid, valid ? (last ? TK_ROWS_ZERO_ALL : TK_ROWS_ZERO) : 0, stream);
         break;
       case kDownResid:
-        rc = tk_gemm(u, f, w.w_2, f, w.b_2, resid, d, resid, d, t, d, f, TK_EPI_BIAS_RESID, valid,
-                     valid ? TK_ROWS_ZERO : 0, stream);
+        rc = gemm(u, f, w.w_2, f, w.b_2, resid, d, resid, d, t, d, f, TK_EPI_BIAS_RESID, valid,
+                  valid ? TK_ROWS_ZERO : 0, invariant, stream);
         break;
       case kLnQkv:
         rc = tk_narrow_qkv(x, w.n1_w, w.n1_b, w.n1_eps, w.w_qkv_packed, w.b_qkv, qkv, t, stream);

@@ -20,11 +20,12 @@ def _qkv(b, h, s, hd, seed):
 
 
 # One key past a tile, fewer tiles than waves, tiles of four and eight waves that end
-# unevenly, the last launch inside the rule (512 blocks of 32 rows) and the first past it.
+# unevenly, the last launch inside the rule (512 blocks of 32 rows) and the first past it
+# (for head_dim 256 that is the pipelined generic kernel).
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
-@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
 @pytest.mark.parametrize("b,h,s", [(1, 1, 65), (2, 3, 127), (1, 5, 200), (1, 2, 513), (1, 2, 1057), (2, 1, 1990),
-                                   (16, 8, 128), (16, 8, 129), (13, 3, 385)])
+                                   (16, 8, 128), (16, 8, 129), (13, 3, 385), (20, 4, 300)])
 def test_edges(b, h, s, hd, causal):
     q, k, v = _qkv(b, h, s, hd, seed=s + hd)
     out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal)
@@ -33,11 +34,12 @@ def test_edges(b, h, s, hd, causal):
 
 
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
-@pytest.mark.parametrize("hd,s", [(32, 300), (64, 1090), (128, 300)])
-def test_key_mask(hd, s, causal):
+@pytest.mark.parametrize("hd,s,h", [(32, 300, 2), (64, 1090, 2), (128, 300, 2), (256, 300, 2), (256, 300, 18)],
+                         ids=["d32", "d64", "d128", "d256", "d256_past_rule"])
+def test_key_mask(hd, s, h, causal):
     """Padded tails, whole tiles without a valid key, holes; rows without any valid key
     come out non-finite, as from the other kernels."""
-    b, h = 3, 2
+    b = 3
     q, k, v = _qkv(b, h, s, hd, seed=s)
     valid = torch.ones(b, s, dtype=torch.bool)
     valid[0, s - 90:] = False
@@ -57,7 +59,7 @@ def test_key_mask(hd, s, causal):
     assert bad == 0, err
 
 
-@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
 def test_growing_scores(hd):
     """Row maxima that rise from tile to tile by up to 40 in the exponent, and scores past
     fp16's range: every wave's sums are rescaled and merged at different references."""

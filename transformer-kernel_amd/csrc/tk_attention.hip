@@ -1696,9 +1696,13 @@ __device__ __forceinline__ void flash_single_body(const AttnArgs& p) {
 // one 64-key tile at a time through registers into the flash_dma_body LDS
 // layouts (K chunk-swizzled, V for the transposed reads), exact online
 // softmax (the running max moves with every tile), O stored element-wise.
-// VEC (hd == HDP, 16-byte q/k/v rows, 8-byte out rows): the same loop with
-// 16-byte Q/K/V loads and 8-byte O stores -- the head_dim-256 path, where
-// this plain loop fits its registers (one wave per SIMD, no spill).
+// VEC (hd == HDP, 16-byte q/k/v rows, 8-byte out rows): the head_dim-256 path.  The
+// same arithmetic with 16-byte Q loads, direct K / V copies and 8-byte O stores;
+// bound by its chain of copy, products and softmax at one wave per SIMD (256
+// VGPRs, no spill).  With the copies of the next tile crossing this one's work
+// instead of a load through registers between two barriers: b2 h8 s4096 causal
+// 481 -> 295 us, full 866 -> 504 (546 TFLOP/s), b4 h8 s1024 100 -> 69, b64 h4
+// s128 24.5 -> 21.6 (3.1 TB/s).
 template <int HDP, bool CAUSAL, bool KMASK, bool VEC>
 __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) {
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
@@ -1767,23 +1771,37 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
   const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  // VEC: one K and one V slot, filled by direct copies, 1 KB per wave and copy; the
+  // next K tile is on its way from the moment that every wave has this one's
+  // fragments, the next V tile from the end of P.V, so each crosses the other
+  // product and the softmax.  Rows past S re-read row S - 1 (masked).
+  constexpr int CPW = VEC ? TILE / 1024 / NW : 1;  // copies per wave and tile
+  const uint32_t k_lds = (uint32_t)(size_t)(lds_char*)ks_, v_lds = k_lds + TILE;
+  auto copy = [&](const f16* base, int64_t rs, int j, uint32_t dst, bool is_v) {
+    constexpr int RPC = 1024 / RB;
+#pragma unroll
+    for (int i = 0; i < CPW; ++i) {
+      const int c = wave * CPW + i, row = c * RPC + lane / CPR, phys = lane % CPR;
+      const int chunk = is_v ? phys ^ vswz<RB>(row) : (swz_off<RB>(row, phys) - row * RB) >> 4;
+      dma16(base + (int64_t)min(j * kBN + row, p.S - 1) * rs + chunk * 8, dst + c * 1024);
+    }
+  };
+  if constexpr (VEC) {
+    copy(kb, p.ks[2], 0, k_lds, false);
+    copy(vb, p.vs[2], 0, v_lds, true);
+  }
   for (int kt = 0; kt < n_kt; ++kt) {
     const int k0 = kt * kBN;
-    __syncthreads();  // the previous tile's operands are no longer read
+    const bool more = kt + 1 < n_kt;
+    if constexpr (!VEC) {
+      __syncthreads();  // the previous tile's operands are no longer read
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int idx = tid + i * NT;
-      if (LOADS * NT == kBN * CPR || idx < kBN * CPR) {
-        const int row = idx / CPR, ch = idx % CPR;
-        const int key = k0 + row;
-        f16x8 kv8, vv8;
-        if constexpr (VEC) {
-          kv8 = vv8 = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-          if (key < p.S) {
-            kv8 = *reinterpret_cast<const f16x8*>(kb + (int64_t)key * p.ks[2] + ch * 8);
-            vv8 = *reinterpret_cast<const f16x8*>(vb + (int64_t)key * p.vs[2] + ch * 8);
-          }
-        } else {
+      for (int i = 0; i < LOADS; ++i) {
+        const int idx = tid + i * NT;
+        if (LOADS * NT == kBN * CPR || idx < kBN * CPR) {
+          const int row = idx / CPR, ch = idx % CPR;
+          const int key = k0 + row;
+          f16x8 kv8, vv8;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const int col = ch * 8 + e;
@@ -1791,13 +1809,18 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
             kv8[e] = in ? kb[(int64_t)key * p.ks[2] + col] : (f16)0;
             vv8[e] = in ? vb[(int64_t)key * p.vs[2] + col] : (f16)0;
           }
+          *reinterpret_cast<f16x8*>(ks_ + swz_off<RB>(row, ch)) = kv8;
+          *reinterpret_cast<f16x8*>(vs_ + row * RB + ((ch ^ vswz<RB>(row)) << 4)) = vv8;
         }
-        *reinterpret_cast<f16x8*>(ks_ + swz_off<RB>(row, ch)) = kv8;
-        *reinterpret_cast<f16x8*>(vs_ + row * RB + ((ch ^ vswz<RB>(row)) << 4)) = vv8;
       }
     }
     const uint64_t kbits = KMASK ? (uint64_t)__ballot(kvb[min(k0 + lane, p.S - 1)] != 0) >> (4 * g) : 0ull;
-    __syncthreads();
+    if constexpr (VEC) {
+      wait_vmcnt<CPW>();  // all but V's copies
+      lds_barrier();
+    } else {
+      __syncthreads();
+    }
 
     f32x16 s[2];
 #pragma unroll
@@ -1805,6 +1828,11 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
       const int kb2 = c / KSTEPS, kk = c % KSTEPS;
       const f16x8 kf = *reinterpret_cast<const f16x8*>(ks_ + swz_off<RB>(kb2 * 32 + (lane & 31), 2 * kk + g));
       s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kk], kk == 0 ? f32x16{} : s[kb2], 0, 0, 0);
+    }
+    if constexpr (VEC) {
+      wait_lds_reads();  // this wave's K fragments are in registers
+      lds_barrier();
+      if (more) copy(kb, p.ks[2], kt + 1, k_lds, false);
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -1835,6 +1863,11 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
       pf[e >> 3][e & 7] = ph;
       l_run += (float)ph;
     }
+    if constexpr (VEC) {
+      if (more) wait_vmcnt<CPW>();  // all but the next K's copies
+      else wait_vmcnt<0>();
+      lds_barrier();
+    }
 #pragma unroll
     for (int c = 0; c < NP; ++c) {
       const int t = c / DB, d = c % DB;
@@ -1845,6 +1878,13 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
                                          4, 5, 6, 7);
       if (!d_ok) vf = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
       acc_o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[t], acc_o[d], 0, 0, 0);
+    }
+    if constexpr (VEC) {
+      if (more) {
+        wait_lds_reads();
+        lds_barrier();
+        copy(vb, p.vs[2], kt + 1, v_lds, true);
+      }
     }
   }
 
@@ -1947,18 +1987,18 @@ template <int HD, int NW, bool CAUSAL, bool KMASK>
 __global__ __launch_bounds__(NW * 64, HD <= 64 ? 2 : 1) void flash_keysplit_kernel(AttnArgs p) {
   keysplit_body<HD, NW, CAUSAL, KMASK>(p);
 }
-// Where the key-split kernel is taken: head dims 32, 64 and 128, more than one key
+// Where the key-split kernel is taken: head dims 32, 64, 128 and 256, more than one key
 // tile, and at most two workgroups of it per CU (32 query rows each).  Measured on 87
 // launches, us (others -> key split): b1 h16 s512 causal, head_dim 64 10.1 -> 5.7,
-// 128 23.8 -> 8.9, 32 8.6 -> 4.7; b1 h4 s2048 23.1 -> 11.0 (eight waves); at 512
-// workgroups b1 h16 s1024 without the causal mask 14.1 -> 11.8, 128 31.6 -> 25.3,
-// 32 12.8 -> 8.4.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs 12.6,
+// 128 23.8 -> 8.9, 32 8.6 -> 4.7, 256 38.0 -> 16.9; b1 h4 s2048 23.1 -> 11.0 (eight waves); at 512
+// workgroups, b1 h16 s1024 without the causal mask 14.1 -> 11.8, 128 31.6 -> 25.3,
+// 32 12.8 -> 8.4, 256 66.3 -> 51.5.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs 12.6,
 // b1 h16 s2048 full 26.1 vs 35.5) except for head_dim 32 causal (b1 h16 s2048 24.5 ->
 // 18.3, b64 h4 s128 6.6 -> 6.4).  Eight waves: from 1024 keys, one workgroup per CU
 // (b1 h1 s4096 22.7 -> 17.7; b1 h16 s512 5.7 vs 5.9).
 int64_t keysplit_blocks(int64_t bh, int64_t s) { return bh * ((s + 31) / 32); }
 bool keysplit_pays(int64_t bh, int64_t s, int64_t hd, bool causal) {
-  return (hd == 32 || hd == 64 || hd == 128) && s > 64 &&
+  return (hd == 32 || hd == 64 || hd == 128 || hd == 256) && s > 64 &&
          keysplit_blocks(bh, s) <= (hd == 32 && causal ? 1024 : 512);
 }
 template <int HD, int NW>
@@ -2076,6 +2116,7 @@ int tk::flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half
       const bool w8 = keysplit_blocks(batch * heads, seq) <= 256 && seq > 1024;
       if (head_dim == 32) return w8 ? launch_keysplit<32, 8>(p, c, st) : launch_keysplit<32, 4>(p, c, st);
       if (head_dim == 64) return w8 ? launch_keysplit<64, 8>(p, c, st) : launch_keysplit<64, 4>(p, c, st);
+      if (head_dim == 256) return launch_keysplit<256, 4>(p, c, st);
       return launch_keysplit<128, 4>(p, c, st);
     }
     if (v8 && seq > 128 && v16) return launch_full128(p, st);
@@ -2084,9 +2125,9 @@ int tk::flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half
       case 32: return dispatch_flash<32>(p, c, st);
       case 64: return dispatch_flash<64>(p, c, st);
       case 128: return dispatch_flash<128>(p, c, st);
-      // head_dim 256: the generic kernel's plain tile loop on 16-byte rows
-      // (appendix case 8, b64 s128: 41 -> 29 us against a DMA-ring body
-      // that spilled 0.5-2.6 KB per lane at this width)
+      // head_dim 256: the generic kernel's tile loop on 16-byte rows (appendix case
+      // 8, b64 s128: 41 -> 29 us against a DMA-ring body that spilled 0.5-2.6 KB
+      // per lane at this width; 21.6 since its K and V are direct copies)
       default: return launch_generic<256, true>(p, 256, c, st);
     }
   }

@@ -25,7 +25,8 @@ __device__ __forceinline__ void wait_lds_reads() {
 
 template <int HD, int NW, bool CAUSAL, bool KMASK, typename Args>
 __device__ __forceinline__ void keysplit_body(const Args& p) {
-  constexpr int BN = 64;                  // keys per tile
+  constexpr int BN = HD <= 128 ? 64 : 32;  // keys per tile
+  constexpr int NB = BN / 32;              // 32-key blocks of S^T
   constexpr int RB = HD * 2;              // tile row bytes
   constexpr int CPR = RB / 16;            // 16-byte chunks per row
   constexpr int TILE = BN * RB;           // bytes per K or V tile
@@ -36,8 +37,9 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
   constexpr int SLOT = 2 * TILE;          // a wave's K and V
   constexpr int CHUNKS = 4 * DB;          // 4-register pieces of O
   static_assert(HD >= 32 && COPIES < 64 && (CHUNKS % NW == 0 || CHUNKS <= NW), "whole chunks per wave");
-  static_assert(CHUNKS * 1024 + 256 <= SLOT, "a wave's results fit its slots");
+  static_assert(CHUNKS * 1024 <= SLOT, "a wave's O fits its slots");
   __shared__ __attribute__((aligned(16))) char smem[NW * SLOT];
+  __shared__ float row_m[NW][32], row_l[NW][32];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -107,9 +109,9 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
     if (KMASK) kbyte = kvb[min(kt * BN + lane, p.S - 1)];
     wait_vmcnt<COPIES>();  // all but V's copies: K has landed
     asm volatile("" ::: "memory");
-    f32x16 s[2];
+    f32x16 s[NB];
 #pragma unroll
-    for (int c = 0; c < 2 * KSTEPS; ++c) {
+    for (int c = 0; c < NB * KSTEPS; ++c) {
       const int kb2 = c / KSTEPS, kk = c % KSTEPS;
       const f16x8 kf = *reinterpret_cast<const f16x8*>(ks_ + swz_off<RB>(kb2 * 32 + (lane & 31), 2 * kk + g));
       s[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kk], kk == 0 ? f32x16{} : s[kb2], 0, 0, 0);
@@ -125,22 +127,22 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
     float mx = -INFINITY;
     if (KMASK || k0 + BN > p.S || (CAUSAL && k0 + BN - 1 > q0)) {
 #pragma unroll
-      for (int e = 0; e < 32; ++e) {
+      for (int e = 0; e < 16 * NB; ++e) {
         const int j = (e >> 4) * 32 + 8 * ((e & 15) >> 2) + (e & 3), key = k0 + j + 4 * g;
         if (key >= p.S || (CAUSAL && key > my_row) || (KMASK && ((kbits >> j) & 1) == 0))
           s[e >> 4][e & 15] = -INFINITY;
       }
     }
 #pragma unroll
-    for (int e = 0; e < 32; ++e) mx = fmaxf(mx, s[e >> 4][e & 15]);
+    for (int e = 0; e < 16 * NB; ++e) mx = fmaxf(mx, s[e >> 4][e & 15]);
     const float m_new = fmaxf(m_run, pair_max(mx) * cs);  // cs > 0
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
     m_run = m_new;
-    f16x8 pf[4];
+    f16x8 pf[2 * NB];
     float ls = 0.f;
 #pragma unroll
-    for (int e = 0; e < 32; ++e) {
+    for (int e = 0; e < 16 * NB; ++e) {
       const float pe = __builtin_amdgcn_exp2f(fmaf(s[e >> 4][e & 15], cs, -m_use));
       pf[e >> 3][e & 7] = (f16)pe;
       ls += pe;
@@ -155,7 +157,7 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
     else wait_vmcnt<0>();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int c = 0; c < 4 * DB; ++c) {
+    for (int c = 0; c < 2 * NB * DB; ++c) {
       const int t = c / DB, d = c % DB;
       const lds_char* base = (const lds_char*)(vs_ + t * 16 * RB);
       const tr_f16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr_f16x4*)(base + v_rd[0][d]));
@@ -170,7 +172,7 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
   }
 
   // ---- merge: O rescaled to the rows' common max, sums in wave order ----
-  // A wave writes its O (CHUNKS of 64 lanes x 16 bytes) and (m, l) into its own slots.
+  // A wave writes its O (CHUNKS of 64 lanes x 16 bytes) into its own slots.
   asm volatile("" ::: "memory");
   l_run = pair_sum(l_run);
 #pragma unroll
@@ -179,23 +181,22 @@ __device__ __forceinline__ void keysplit_body(const Args& p) {
     const int q = c % 4;
     *reinterpret_cast<f32x4*>(ks_ + c * 1024 + lane * 16) = f32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
   }
-  float* ml = reinterpret_cast<float*>(ks_ + CHUNKS * 1024);
   if (g == 0) {
-    ml[lane] = m_run;
-    ml[32 + lane] = l_run;
+    row_m[wave][lane] = m_run;
+    row_l[wave][lane] = l_run;
   }
   __syncthreads();
   float f[NW], m_all = -INFINITY, l_all = 0.f;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    f[w] = reinterpret_cast<const float*>(smem + w * SLOT + CHUNKS * 1024)[lane & 31];
+    f[w] = row_m[w][lane & 31];
     m_all = fmaxf(m_all, f[w]);
   }
   const float m_ref = m_all == -INFINITY ? 0.f : m_all;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
     f[w] = __builtin_amdgcn_exp2f(f[w] - m_ref);
-    l_all += f[w] * reinterpret_cast<const float*>(smem + w * SLOT + CHUNKS * 1024)[32 + (lane & 31)];
+    l_all += f[w] * row_l[w][lane & 31];
   }
   const float inv = 1.0f / l_all;
   f16* orow = p.o + b * p.os[0] + h * p.os[1] + (int64_t)my_row * p.os[2];

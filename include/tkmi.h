@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define TKMI_ABI_VERSION 3
+#define TKMI_ABI_VERSION 4
 
 typedef uint16_t tk_half;
 
@@ -193,7 +193,8 @@ int tk_masked_softmax(const float *scores, tk_half *probs, int64_t groups,
  *   x += u.W_2^T + b_2
  * then out = LN_final(x), with the numerics of the layer-by-layer path
  * (fp16 operands, fp32 accumulation, residual and statistics).
- * x, out: [batch, seq, d_model] f32 (out may not alias x).
+ * x, out: [batch, seq, d_model] f32, or 16-bit as the flags say (out may not
+ * alias x).
  * Weights stacked over the layers, each layer's block as the layer-by-layer
  * calls take it: w_qkv [L][3*heads*hd][d] f16 (head rows zero-padded to hd =
  * head_dim_padded), b_qkv [L][3*heads*hd] f32, w_o [L][d][heads*hd] f16,
@@ -375,8 +376,10 @@ enum tk_forward_flags {
                               packed weights are given, else residual + LayerNorm in the GEMM epilogues
                               where tk_gemm_ln_supported */
   TK_FWD_QKV_ATTENTION = 2, /* tk_qkv_attention where it takes the shape (dense inputs) */
-  TK_FWD_BATCH_INVARIANT = 4 /* no kernel whose choice and order of sums depend on the batch size: a
-                                sequence's output bits are the same in every batch */
+  TK_FWD_BATCH_INVARIANT = 4, /* no kernel whose choice and order of sums depend on the batch size: a
+                                 sequence's output bits are the same in every batch */
+  TK_FWD_IO_F16 = 8,          /* x and out are fp16 ... */
+  TK_FWD_IO_BF16 = 16         /* ... or bf16 instead of fp32; without TK_FWD_FUSED_NORM only */
 };
 
 /* Bytes of the workspace that tk_forward needs; negative: a tk_status. */
@@ -388,7 +391,8 @@ const char *tk_forward_step_name(const tk_model *model, int64_t batch, int64_t s
                                  int64_t step);
 
 /*
- * x, out: [batch, seq, d_model] f32 (out may not alias x).  valid (nullable):
+ * x, out: [batch, seq, d_model] f32, or 16-bit as the flags say (out may not
+ * alias x).  valid (nullable):
  * [batch, seq] validity bytes, NULL = dense.  workspace: 256-byte aligned
  * device memory of at least tk_forward_workspace bytes, this call's own until
  * its launches have run.  Runs launches [first_step, first_step + num_steps);
@@ -396,7 +400,7 @@ const char *tk_forward_step_name(const tk_model *model, int64_t batch, int64_t s
  * Replaces the layer loop of OptimizedTransformer._run_layers_fused
  * (src/optimized.py:488-554).
  */
-int tk_forward(const tk_model *model, const float *x, float *out, int64_t batch, int64_t seq,
+int tk_forward(const tk_model *model, const void *x, void *out, int64_t batch, int64_t seq,
                const uint8_t *valid, void *workspace, int64_t workspace_bytes, int flags,
                int64_t first_step, int64_t num_steps, void *stream);
 

@@ -17,10 +17,14 @@
 // GEMM, and non-temporal stores made C2's forward 4 % slower.
 #include "tk_common.hpp"
 
+#include <type_traits>
+
 namespace tk {
 namespace {
 
 constexpr int kBlock = 256;
+typedef __bf16 bf16;
+typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 template <bool NT, typename V>
 __device__ __forceinline__ V ld(const V* p) {
@@ -62,14 +66,29 @@ struct Vec<f16, NT> {
   static __device__ __forceinline__ void store1(f16* p, float v) { *p = (f16)v; }
 };
 
+template <bool NT>
+struct Vec<bf16, NT> {
+  static __device__ __forceinline__ void load4(const bf16* p, float* v) {
+    bf16x4 t = ld<NT>(reinterpret_cast<const bf16x4*>(p));
+    v[0] = (float)t[0]; v[1] = (float)t[1]; v[2] = (float)t[2]; v[3] = (float)t[3];
+  }
+  static __device__ __forceinline__ void store4(bf16* p, const float* v) {
+    bf16x4 t = {(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+    st<NT>(reinterpret_cast<bf16x4*>(p), t);
+  }
+  static __device__ __forceinline__ float load1(const bf16* p) { return (float)*p; }
+  static __device__ __forceinline__ void store1(bf16* p, float v) { *p = (bf16)v; }
+};
+
 // HAS_Y: s = x + y (residual add, in fp32) else s = x.  The sum is stored in
 // x's type XT (src/fused_kernels.py:216,143-147: s = x + y in x's dtype); the
 // statistics use the fp32 sum before that rounding.  row_valid (nullable): an
 // invalid row's normalised output is written as zeros.
-template <int LPR, int NV, int VW, bool HAS_Y, typename XT, typename YT, typename OT, bool NT>
+// SumT other than XT (no y): sum_out takes x itself in that type.
+template <int LPR, int NV, int VW, bool HAS_Y, typename XT, typename YT, typename OT, bool NT, typename SumT>
 __global__ __launch_bounds__(kBlock) void ln_rows_kernel(
     const XT* x, const YT* __restrict__ y, const float* __restrict__ w,
-    const float* __restrict__ b, XT* sum_out, OT* __restrict__ out, int64_t rows,
+    const float* __restrict__ b, SumT* sum_out, OT* __restrict__ out, int64_t rows,
     int cols, float eps, const uint8_t* __restrict__ row_valid) {
   constexpr int kRowsPerBlock = kBlock / LPR;
   const int lane = threadIdx.x % LPR;
@@ -105,14 +124,14 @@ __global__ __launch_bounds__(kBlock) void ln_rows_kernel(
     }
   }
 
-  if (HAS_Y && sum_out != nullptr) {
-    XT* sr = sum_out + row * cols;
+  if ((HAS_Y || !std::is_same<XT, SumT>::value) && sum_out != nullptr) {
+    SumT* sr = sum_out + row * cols;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int c0 = (v * LPR + lane) * VW;
       if (c0 < cols) {
-        if constexpr (VW == 4) Vec<XT, NT>::store4(sr + c0, &s[v * 4]);
-        else Vec<XT>::store1(sr + c0, s[v]);
+        if constexpr (VW == 4) Vec<SumT, NT>::store4(sr + c0, &s[v * 4]);
+        else Vec<SumT>::store1(sr + c0, s[v]);
       }
     }
   }
@@ -160,31 +179,31 @@ __global__ __launch_bounds__(kBlock) void ln_rows_kernel(
 
 constexpr int64_t kStreamBytes = 128ll << 20;  // fp32 input size from which the accesses are non-temporal
 
-template <int LPR, int NV, int VW, bool HAS_Y, typename XT, typename YT, typename OT>
-int launch_rows(const XT* x, const YT* y, const float* w, const float* b, XT* sum_out,
+template <int LPR, int NV, int VW, bool HAS_Y, typename XT, typename YT, typename OT, typename SumT>
+int launch_rows(const XT* x, const YT* y, const float* w, const float* b, SumT* sum_out,
                 OT* out, int64_t rows, int cols, float eps, const uint8_t* row_valid, hipStream_t st) {
   constexpr int kRowsPerBlock = kBlock / LPR;
   const int64_t grid = (rows + kRowsPerBlock - 1) / kRowsPerBlock;
   if (VW == 4 && rows * cols * 4 >= kStreamBytes)
-    hipLaunchKernelGGL((ln_rows_kernel<LPR, NV, VW, HAS_Y, XT, YT, OT, true>), dim3((unsigned)grid),
+    hipLaunchKernelGGL((ln_rows_kernel<LPR, NV, VW, HAS_Y, XT, YT, OT, true, SumT>), dim3((unsigned)grid),
                        dim3(kBlock), 0, st, x, y, w, b, sum_out, out, rows, cols, eps, row_valid);
   else
-    hipLaunchKernelGGL((ln_rows_kernel<LPR, NV, VW, HAS_Y, XT, YT, OT, false>), dim3((unsigned)grid),
+    hipLaunchKernelGGL((ln_rows_kernel<LPR, NV, VW, HAS_Y, XT, YT, OT, false, SumT>), dim3((unsigned)grid),
                        dim3(kBlock), 0, st, x, y, w, b, sum_out, out, rows, cols, eps, row_valid);
   return check_launch("layernorm");
 }
 
 // Picks lanes-per-row and register-vector count for `cols`.
-template <bool HAS_Y, typename XT, typename YT, typename OT>
-int dispatch(const XT* x, const YT* y, const float* w, const float* b, XT* sum_out,
+template <bool HAS_Y, typename XT, typename YT, typename OT, typename SumT = XT>
+int dispatch(const XT* x, const YT* y, const float* w, const float* b, SumT* sum_out,
              OT* out, int64_t rows, int cols, float eps, const uint8_t* row_valid, hipStream_t st) {
 #define TK_LN(LPR, NV, VW) \
-  return launch_rows<LPR, NV, VW, HAS_Y, XT, YT, OT>(x, y, w, b, sum_out, out, rows, cols, eps, row_valid, st)
+  return launch_rows<LPR, NV, VW, HAS_Y, XT, YT, OT, SumT>(x, y, w, b, sum_out, out, rows, cols, eps, row_valid, st)
   // 4-wide vector path needs cols % 4 == 0 and rows aligned to 4 elements
   // (16 bytes for fp32 rows, 8 for fp16); anything else takes the scalar path.
   auto al = [](const void* p, uintptr_t a) { return p == nullptr || ((uintptr_t)p % a) == 0; };
   const bool vec_ok = cols % 4 == 0 && al(x, sizeof(XT) * 4) && al(w, 16) && al(b, 16) &&
-                      al(sum_out, sizeof(XT) * 4) && al(y, sizeof(YT) * 4) && al(out, sizeof(OT) * 4);
+                      al(sum_out, sizeof(SumT) * 4) && al(y, sizeof(YT) * 4) && al(out, sizeof(OT) * 4);
   if (vec_ok) {
     if (cols <= 64) TK_LN(16, 1, 4);
     if (cols <= 128) TK_LN(32, 1, 4);
@@ -230,8 +249,8 @@ extern "C" int tk_ln_cast(const float* x, const float* w, const float* b, void* 
   hipStream_t st = as_stream(stream);
   const int c = (int)cols;
   if (out_dtype == TK_F16)
-    return dispatch<false, float, float, f16>(x, nullptr, w, b, nullptr, (f16*)out, rows, c, eps, row_valid, st);
-  return dispatch<false, float, float, float>(x, nullptr, w, b, nullptr, (float*)out, rows, c, eps, row_valid,
+    return dispatch<false, float, float, f16>(x, nullptr, w, b, (float*)nullptr, (f16*)out, rows, c, eps, row_valid, st);
+  return dispatch<false, float, float, float>(x, nullptr, w, b, (float*)nullptr, (float*)out, rows, c, eps, row_valid,
                                               st);
 }
 
@@ -269,4 +288,28 @@ extern "C" int tk_add_ln_cast(const void* x, int x_dtype, const void* y, int y_d
   if (x_dtype == TK_F16)
     return add_ln_x<f16>((const f16*)x, y, y_dtype, w, b, (f16*)sum_out, h_out, h_dtype, rows, c, eps, st);
   return add_ln_x<float>((const float*)x, y, y_dtype, w, b, (float*)sum_out, h_out, h_dtype, rows, c, eps, st);
+}
+
+int tk::ln_first16(const void* x, bool is_bf16, const float* w, const float* b, float* x32, tk_half* h, int64_t rows,
+                   int64_t cols, float eps, void* stream) {
+  TK_REQUIRE(x && w && b && x32 && h, TK_ERR_ARG, "ln_first16: null pointer");
+  TK_REQUIRE(rows >= 0 && cols >= 1 && cols <= kMaxCols, TK_ERR_ARG, "tk_ln_cast: rows=%lld cols=%lld",
+             (long long)rows, (long long)cols);
+  if (rows == 0) return TK_OK;
+  hipStream_t st = as_stream(stream);
+  if (is_bf16)
+    return dispatch<false, bf16, float, f16>((const bf16*)x, nullptr, w, b, x32, (f16*)h, rows, (int)cols, eps,
+                                             nullptr, st);
+  return dispatch<false, f16, float, f16>((const f16*)x, nullptr, w, b, x32, (f16*)h, rows, (int)cols, eps, nullptr,
+                                          st);
+}
+
+int tk::ln_last_bf16(const float* x, const float* w, const float* b, void* out, int64_t rows, int64_t cols, float eps,
+                     const uint8_t* row_valid, void* stream) {
+  TK_REQUIRE(x && w && b && out, TK_ERR_ARG, "ln_last_bf16: null pointer");
+  TK_REQUIRE(rows >= 0 && cols >= 1 && cols <= kMaxCols, TK_ERR_ARG, "tk_ln_cast: rows=%lld cols=%lld",
+             (long long)rows, (long long)cols);
+  if (rows == 0) return TK_OK;
+  return dispatch<false, float, float, bf16>(x, nullptr, w, b, (float*)nullptr, (bf16*)out, rows, (int)cols, eps,
+                                             row_valid, as_stream(stream));
 }

@@ -118,7 +118,7 @@ extern "C" const char* tk_forward_step_name(const tk_model* m, int64_t batch, in
   return step >= 0 && step < s.steps() ? kStepNames[s.kind(step)] : nullptr;
 }
 
-extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t batch, int64_t seq,
+extern "C" int tk_forward(const tk_model* m, const void* x, void* out, int64_t batch, int64_t seq,
                           const uint8_t* valid, void* workspace, int64_t workspace_bytes, int flags,
                           int64_t first_step, int64_t num_steps, void* stream) {
   if (int rc = check_model(m, batch, seq, "tk_forward")) return rc;
@@ -129,6 +129,12 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
   TK_REQUIRE(workspace_bytes >= l.bytes && ((uintptr_t)workspace & 255) == 0, TK_ERR_ARG,
              "tk_forward: workspace of %lld bytes at %p; %lld bytes, 256-byte aligned, needed",
              (long long)workspace_bytes, workspace, (long long)l.bytes);
+  TK_REQUIRE((flags & ~31) == 0, TK_ERR_ARG, "tk_forward: unknown flags %d", flags);
+  const bool io16 = flags & (TK_FWD_IO_F16 | TK_FWD_IO_BF16), bf16 = flags & TK_FWD_IO_BF16;
+  TK_REQUIRE(!io16 || (!s.fuse && !s.narrow), TK_ERR_UNSUPPORTED,
+             "tk_forward: 16-bit x and out need the schedule without TK_FWD_FUSED_NORM");
+  TK_REQUIRE((flags & (TK_FWD_IO_F16 | TK_FWD_IO_BF16)) != (TK_FWD_IO_F16 | TK_FWD_IO_BF16), TK_ERR_ARG,
+             "tk_forward: x is either fp16 or bf16");
   const int64_t steps = s.steps();
   if (num_steps < 0) num_steps = steps - first_step;
   TK_REQUIRE(first_step >= 0 && num_steps >= 0 && first_step + num_steps <= steps, TK_ERR_ARG,
@@ -146,18 +152,21 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
     const int64_t li = s.layer_of(i);
     const tk_layer& w = m->layers[li];
     const bool last = li + 1 == m->num_layers;
-    // Residual input of the first layer's attention update: the caller's x, which is never written.
-    const float* src = li == 0 ? x : resid;
+    // Residual input of the first layer's attention update: the caller's x, which is never
+    // written (16-bit: its fp32 copy, left by the first LayerNorm).
+    const float* x32 = static_cast<const float*>(x);
+    const float* src = li == 0 && !io16 ? x32 : resid;
     // What the LayerNorm after the FFN is: the next block's first, or the final one (fp32, into out).
     const float* nw = last ? m->nf_w : m->layers[li + 1].n1_w;
     const float* nb = last ? m->nf_b : m->layers[li + 1].n1_b;
     const float ne = last ? m->nf_eps : m->layers[li + 1].n1_eps;
-    void* ndst = last ? static_cast<void*>(out) : static_cast<void*>(h);
-    const int ndt = last ? TK_F32 : TK_F16;
+    void* ndst = last ? out : static_cast<void*>(h);
+    const int ndt = last && !io16 ? TK_F32 : TK_F16;
     int rc = TK_OK;
     switch (s.kind(i)) {
       case kLnIn:
-        rc = tk_ln_cast(x, w.n1_w, w.n1_b, h, TK_F16, t, d, w.n1_eps, nullptr, stream);
+        if (io16) rc = ln_first16(x, bf16, w.n1_w, w.n1_b, resid, h, t, d, w.n1_eps, stream);
+        else rc = tk_ln_cast(x32, w.n1_w, w.n1_b, h, TK_F16, t, d, w.n1_eps, nullptr, stream);
         break;
       case kQkv:
         rc = gemm(h, d, w.w_qkv, d, w.b_qkv, nullptr, 0, qkv, 3 * dp, t, 3 * dp, d, TK_EPI_BIAS, nullptr, 0, invariant,
@@ -193,7 +202,7 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
                   valid ? TK_ROWS_ZERO : 0, invariant, stream);
         break;
       case kLnQkv:
-        rc = tk_narrow_qkv(x, w.n1_w, w.n1_b, w.n1_eps, w.w_qkv_packed, w.b_qkv, qkv, t, stream);
+        rc = tk_narrow_qkv(x32, w.n1_w, w.n1_b, w.n1_eps, w.w_qkv_packed, w.b_qkv, qkv, t, stream);
         break;
       case kTail:
         rc = tk_narrow_tail(ctx, src, w.w_o_packed, w.b_o, w.n2_w, w.n2_b, w.n2_eps, w.w_1_packed, w.b_1,
@@ -202,7 +211,8 @@ extern "C" int tk_forward(const tk_model* m, const float* x, float* out, int64_t
         break;
       case kLnNext:
       case kLnFinal:
-        rc = tk_ln_cast(resid, nw, nb, ndst, ndt, t, d, ne, last ? valid : nullptr, stream);
+        if (last && bf16) rc = ln_last_bf16(resid, nw, nb, ndst, t, d, ne, valid, stream);
+        else rc = tk_ln_cast(resid, nw, nb, ndst, ndt, t, d, ne, last ? valid : nullptr, stream);
         break;
     }
     if (rc != TK_OK) return rc;

@@ -13,7 +13,7 @@ import threading
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_void_p
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "libtkmi.so"
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 TK_OK, TK_ERR_ARG, TK_ERR_UNSUPPORTED, TK_ERR_HIP = 0, -1, -2, -3
 TK_F32, TK_F16 = 0, 1
@@ -21,6 +21,7 @@ TK_EPI_BIAS, TK_EPI_BIAS_GELU, TK_EPI_BIAS_RESID = 0, 1, 2
 TK_ROWS_KEEP_RESID, TK_ROWS_ZERO, TK_ROWS_ZERO_ALL = 1, 2, 3
 
 TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION, TK_FWD_BATCH_INVARIANT = 1, 2, 4
+TK_FWD_IO_F16, TK_FWD_IO_BF16 = 8, 16
 
 _I64_3 = c_int64 * 3
 

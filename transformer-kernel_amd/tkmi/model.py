@@ -41,7 +41,7 @@ from typing import List, Optional
 import torch
 
 from . import _lib, ops
-from ._lib import TK_FWD_BATCH_INVARIANT, TK_FWD_FUSED_NORM, TK_FWD_QKV_ATTENTION
+from ._lib import TK_FWD_BATCH_INVARIANT, TK_FWD_FUSED_NORM, TK_FWD_IO_BF16, TK_FWD_IO_F16, TK_FWD_QKV_ATTENTION
 from .modules import BaselineTransformer
 
 __all__ = ["OptimizerSettings", "OptimizedTransformer", "configure", "active_settings"]
@@ -132,6 +132,9 @@ def _fragments(w: torch.Tensor) -> torch.Tensor:
     n, k = w.shape
     return w.view(n // 32, 32, k // 128, 8, 2, 8).permute(2, 0, 3, 4, 1, 5).contiguous()
 
+
+# Input dtypes that tk_forward takes, and returns, as they are.
+_IO_FLAGS = {torch.float16: TK_FWD_IO_F16, torch.bfloat16: TK_FWD_IO_BF16}
 
 # Head dims the attention kernel has tiles for (tk_attention_supported).
 _KERNEL_HEAD_DIMS = (16, 32, 64, 128, 256)
@@ -325,20 +328,23 @@ class OptimizedTransformer(BaselineTransformer):
         fn_w, fn_b, fn_eps = self._final
         dev = x.device
         xin = x.reshape(t, d)
-        if xin.dtype != torch.float32:
+        small = mask is None and self._small_forward_ok(seq, weights)
+        flags = 0
+        if self.settings.fused_norm and d <= self.settings.fused_norm_max_d:
+            flags |= TK_FWD_FUSED_NORM
+        elif not small and x.dtype in _IO_FLAGS:  # converted in the first and last LayerNorm
+            flags |= _IO_FLAGS[x.dtype]
+        if xin.dtype != torch.float32 and not flags & (TK_FWD_IO_F16 | TK_FWD_IO_BF16):
             xin = xin.float()
         xin = xin.contiguous()
-        if mask is None and self._small_forward_ok(seq, weights):
+        if small:
             out = torch.empty((bsz, seq, d), dtype=torch.float32, device=dev)
             ops.small_forward(xin.view(bsz, seq, d), out, self._stacked_weights(), (fn_w, fn_b, fn_eps),
                               weights[0].n1_eps, weights[0].n2_eps, nh, hd, self.config.ffn_dim,
                               self.config.causal, self.attn_scale)
             return out
 
-        out = torch.empty((bsz, seq, d), dtype=torch.float32, device=dev)
-        flags = 0
-        if self.settings.fused_norm and d <= self.settings.fused_norm_max_d:
-            flags |= TK_FWD_FUSED_NORM
+        out = torch.empty((bsz, seq, d), dtype=xin.dtype, device=dev)
         if self.settings.qkv_attention:
             flags |= TK_FWD_QKV_ATTENTION
         if self.settings.batch_invariant:

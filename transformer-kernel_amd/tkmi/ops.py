@@ -373,7 +373,7 @@ def transformer_forward(model: "_lib.Model", x, out, valid, flags: int) -> None:
     """Every launch of a forward by one call into the library (tk_forward).
 
     ``model``: the packed weights' addresses (OptimizedTransformer._native);
-    x, out: [B, S, D] fp32 contiguous; ``valid``: [B, S] bool or None.  Under
+    x, out: [B, S, D] contiguous, fp32 or the 16-bit type that ``flags`` name; ``valid``: [B, S] bool or None.  Under
     ``kernel_timer`` the same launches go out one by one, each timed.
     """
     _require_cuda(x, out, valid)

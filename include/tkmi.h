@@ -116,10 +116,12 @@ int tk_gemm(const tk_half *a, int64_t lda, const tk_half *w, int64_t ldw,
             const uint8_t *row_valid, int row_mode, void *stream);
 
 /*
- * GEMM with the residual + LayerNorm + cast epilogue over full output rows:
+ * GEMM, residual add, LayerNorm and cast:
  *   s = resid + A.W^T + bias (fp32);  h = LN(s; ln_w, ln_b, eps) -> h_dtype
- * sum_out (may be NULL, may alias resid) receives s.  Rows of n elements
- * must fit one tile: n in {128, 256, 512} (tk_gemm_ln_supported).
+ * sum_out (may be NULL, may alias resid) receives s.  Given, it is the
+ * residual GEMM's output and a LayerNorm launch reads it; NULL, one kernel
+ * keeps whole rows on chip, so n must fit one tile: n in {128, 256, 512}
+ * (tk_gemm_ln_supported) in both cases.
  * row_valid (nullable, m bytes) / row_mode: an invalid row takes s per
  * row_mode (tk_row_mode); h = LN(s), or 0 under TK_ROWS_ZERO_ALL.
  * Replaces F.linear followed by fused_kernels.add_ln_fwd

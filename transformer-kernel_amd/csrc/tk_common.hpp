@@ -110,6 +110,12 @@ int gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const flo
          int64_t ldr, void* c, int64_t ldc, int64_t m, int64_t n, int64_t k, int epilogue, const uint8_t* row_valid,
          int row_mode, bool batch_invariant, void* stream);
 
+// tk_gemm_bias_add_ln, likewise.
+int gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const float* bias,
+                     const float* resid, const float* ln_w, const float* ln_b, float* sum_out, void* h_out,
+                     int h_dtype, int64_t m, int64_t n, int64_t k, float eps, const uint8_t* row_valid, int row_mode,
+                     bool batch_invariant, void* stream);
+
 // The first LayerNorm of a 16-bit input, which also leaves it in fp32, and the last one into bf16.
 int ln_first16(const void* x, bool is_bf16, const float* w, const float* b, float* x32, tk_half* h, int64_t rows,
                int64_t cols, float eps, void* stream);

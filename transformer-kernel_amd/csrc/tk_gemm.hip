@@ -1555,11 +1555,16 @@ extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t 
 
 extern "C" int tk_gemm_ln_supported(int64_t n) { return n == 128 || n == 256 || n == 512; }
 
-extern "C" int tk_gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw,
-                                   const float* bias, const float* resid, const float* ln_w,
-                                   const float* ln_b, float* sum_out, void* h_out, int h_dtype,
-                                   int64_t m, int64_t n, int64_t k, float eps, const uint8_t* row_valid,
-                                   int row_mode, void* stream) {
+// Where the sum is wanted too, it is the residual GEMM's output and the LayerNorm reads
+// it back: two launches, but coalesced rows on both sides and the GEMM's own choice of
+// tile.  The full-row kernel, whose workgroups of 64 whole rows wait for their residual
+// and store 32-byte pieces, loses at every size measured, us: n 256, m 26880 k 256 36.1 ->
+// 30.0, m 65536 k 1024 122 -> 82, m 256 k 1024 18.2 -> 7.2; n 128, m 65536 k 128 44.7 ->
+// 30.7; n 512, m 20000 k 2048 155 -> 79.  It runs where the sum is not stored.
+int tk::gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const float* bias,
+                         const float* resid, const float* ln_w, const float* ln_b, float* sum_out, void* h_out,
+                         int h_dtype, int64_t m, int64_t n, int64_t k, float eps, const uint8_t* row_valid,
+                         int row_mode, bool batch_invariant, void* stream) {
   TK_REQUIRE(a && w && resid && ln_w && ln_b && h_out, TK_ERR_ARG, "tk_gemm_bias_add_ln: null pointer");
   TK_REQUIRE(tk_gemm_ln_supported(n), TK_ERR_UNSUPPORTED,
              "tk_gemm_bias_add_ln: row width n=%lld not in {128, 256, 512}", (long long)n);
@@ -1575,6 +1580,13 @@ extern "C" int tk_gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half*
   TK_REQUIRE(row_valid == nullptr || (row_mode >= TK_ROWS_KEEP_RESID && row_mode <= TK_ROWS_ZERO_ALL),
              TK_ERR_ARG, "tk_gemm_bias_add_ln: bad row_mode %d", row_mode);
   if (m == 0) return TK_OK;
+  if (sum_out != nullptr) {
+    const int rc = gemm(a, lda, w, ldw, bias, resid, n, sum_out, n, m, n, k, TK_EPI_BIAS_RESID, row_valid, row_mode,
+                        batch_invariant, stream);
+    if (rc != TK_OK) return rc;
+    return tk_ln_cast(sum_out, ln_w, ln_b, h_out, h_dtype, m, n, eps,
+                      row_mode == TK_ROWS_ZERO_ALL ? row_valid : nullptr, stream);
+  }
   GemmArgs p{};
   p.row_valid = row_valid;
   p.row_mode = row_mode;
@@ -1595,6 +1607,15 @@ extern "C" int tk_gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half*
   if (n == 512) return launch_gemm_ln<Tile<64, 512, 1, 8, 64, 2>>(p, hh, st);
   if (n == 256) return launch_gemm_ln<Tile<64, 256, 1, 4, 64, 2>>(p, hh, st);
   return launch_gemm_ln<Tile<64, 128, 1, 2, 64, 2>>(p, hh, st);
+}
+
+extern "C" int tk_gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw,
+                                   const float* bias, const float* resid, const float* ln_w,
+                                   const float* ln_b, float* sum_out, void* h_out, int h_dtype,
+                                   int64_t m, int64_t n, int64_t k, float eps, const uint8_t* row_valid,
+                                   int row_mode, void* stream) {
+  return gemm_bias_add_ln(a, lda, w, ldw, bias, resid, ln_w, ln_b, sum_out, h_out, h_dtype, m, n, k, eps, row_valid,
+                          row_mode, false, stream);
 }
 
 extern "C" int tk_qkv_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim) {

@@ -180,8 +180,8 @@ extern "C" int tk_forward(const tk_model* m, const void* x, void* out, int64_t b
         rc = tk_qkv_attention(h, d, w.w_qkv, d, w.b_qkv, ctx, dp, batch, seq, nh, hd, m->scale, m->causal, stream);
         break;
       case kOutLn:
-        rc = tk_gemm_bias_add_ln(ctx, dp, w.w_o, dp, w.b_o, src, w.n2_w, w.n2_b, resid, h, TK_F16, t, d, dp,
-                                 w.n2_eps, valid, valid ? TK_ROWS_KEEP_RESID : 0, stream);
+        rc = gemm_bias_add_ln(ctx, dp, w.w_o, dp, w.b_o, src, w.n2_w, w.n2_b, resid, h, TK_F16, t, d, dp, w.n2_eps,
+                              valid, valid ? TK_ROWS_KEEP_RESID : 0, invariant, stream);
         break;
       case kOutResid:
         rc = gemm(ctx, dp, w.w_o, dp, w.b_o, src, d, resid, d, t, d, dp, TK_EPI_BIAS_RESID, valid,
@@ -193,9 +193,9 @@ extern "C" int tk_forward(const tk_model* m, const void* x, void* out, int64_t b
       case kUp:
         rc = gemm(h, d, w.w_1, d, w.b_1, nullptr, 0, u, f, t, f, d, TK_EPI_BIAS_GELU, nullptr, 0, invariant, stream);
         break;
-      case kDownLn:  // the summed residual is dead after the last layer
-        rc = tk_gemm_bias_add_ln(u, f, w.w_2, f, w.b_2, resid, nw, nb, last ? nullptr : resid, ndst, ndt, t, d, f,
-                                 ne, valid, valid ? (last ? TK_ROWS_ZERO_ALL : TK_ROWS_ZERO) : 0, stream);
+      case kDownLn:
+        rc = gemm_bias_add_ln(u, f, w.w_2, f, w.b_2, resid, nw, nb, resid, ndst, ndt, t, d, f, ne, valid,
+                              valid ? (last ? TK_ROWS_ZERO_ALL : TK_ROWS_ZERO) : 0, invariant, stream);
         break;
       case kDownResid:
         rc = gemm(u, f, w.w_2, f, w.b_2, resid, d, resid, d, t, d, f, TK_EPI_BIAS_RESID, valid,

@@ -24,10 +24,9 @@ reference schedule it replaces), all of them from one call into the library
 
 plus one LayerNorm before the first layer.  For one-key-tile sequences (S =
 64, head_dim 64; the reference's config 2) steps 1 and 2 run as one kernel
-that keeps q, k and v on chip.  Steps 3 and 5 run as one kernel
-when a whole row fits a GEMM tile and is narrow enough for that to pay
-(d_model <= OptimizerSettings.fused_norm_max_d); otherwise as a
-residual-epilogue GEMM followed by the standalone LayerNorm kernel.  The
+that keeps q, k and v on chip.  Steps 3 and 5 are a residual-epilogue GEMM
+followed by the LayerNorm kernel; at width 128 steps 3 to 5 run as one kernel,
+as do the first LayerNorm and step 1.  The
 residual stream and all statistics stay fp32; only GEMM/attention operands
 are fp16 (docs/pass1-decisions.md:41-65 of the reference).
 """
@@ -51,16 +50,13 @@ __all__ = ["OptimizerSettings", "OptimizedTransformer", "configure", "active_set
 class OptimizerSettings:
     """Knobs of the MI355X path (counterpart of src/optimized.py:85-139).
 
-    fused_norm        -- fuse residual + LayerNorm + cast into the out-proj /
-                         FFN-down GEMM epilogue where a row fits one tile; off
-                         uses the residual-epilogue GEMM + standalone
-                         LayerNorm kernel for every width (both are HIP).
-    fused_norm_max_d  -- widest d_model that takes the fused epilogue.  Its
-                         full-row tiles (64 rows x d_model) re-read the whole
-                         weight panel per 64 rows; measured on MI355X at
-                         d_model 512 (C2) the split path is ~15% faster per
-                         forward (0.75 vs 0.89 ms), so the fused one is kept
-                         for narrow rows.
+    fused_norm        -- at width 128, run everything after attention as one
+                         kernel (tk_narrow_tail); at other widths up to
+                         fused_norm_max_d, residual + LayerNorm + cast as one
+                         operator after the out-proj / FFN-down GEMM
+                         (tk_gemm_bias_add_ln: a residual GEMM and a LayerNorm
+                         launch).  Off: the same launches as separate steps.
+    fused_norm_max_d  -- widest d_model that takes those.
     assume_dense_mask -- skip the one device->host sync per new mask object
                          that checks the padding mask is all-True.
     small_forward     -- run dense forwards of narrow models (d_model =

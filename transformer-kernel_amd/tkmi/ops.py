@@ -214,9 +214,11 @@ def gemm_ln_supported(n: int) -> bool:
 def linear_add_ln(a, w, bias, resid, ln_weight, ln_bias, eps: float, out_dtype=torch.float16,
                   sum_out=None, h_out=None, name: str = "gemm_add_ln", row_valid=None,
                   row_mode: int = TK_ROWS_KEEP_RESID):
-    """``s = resid + a . w^T + bias``; ``h = LN(s)`` in one kernel (full-row tiles).
+    """``s = resid + a . w^T + bias``; ``h = LN(s)``.
 
-    ``sum_out`` receives s when given (it may be ``resid``); returns h.
+    ``sum_out`` receives s when given (it may be ``resid``), from a residual GEMM
+    whose rows a LayerNorm launch reads; without it one kernel (full-row tiles) keeps
+    s on chip.  Returns h.
     ``row_valid`` / ``row_mode``: an invalid row takes s = resid
     (``TK_ROWS_KEEP_RESID``) or s = 0 (``TK_ROWS_ZERO``; ``TK_ROWS_ZERO_ALL``
     also writes h = 0).

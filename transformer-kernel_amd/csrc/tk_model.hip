@@ -55,10 +55,12 @@ Schedule schedule(const tk_model& m, int64_t batch, int64_t seq, bool dense, int
   s.fused_qa = dense && (flags & TK_FWD_QKV_ATTENTION) && m.heads * m.head_dim == m.d_model &&
                tk_qkv_attention_supported(batch, seq, m.heads, m.head_dim);
   s.fuse = (flags & TK_FWD_FUSED_NORM) && tk_gemm_ln_supported(m.d_model);
+  // The narrow kernels read b_1 in 16-byte vectors; the separate launches take it at any address
+  // (a parameter that is a view into a flat buffer).
   bool packed = true;
   for (int64_t i = 0; i < m.num_layers; ++i)
     packed = packed && m.layers[i].w_qkv_packed && m.layers[i].w_o_packed && m.layers[i].w_1_packed &&
-             m.layers[i].w_2_packed;
+             m.layers[i].w_2_packed && ((uintptr_t)m.layers[i].b_1 & 15) == 0;
   s.narrow = packed && !s.fused_qa && (flags & TK_FWD_FUSED_NORM) &&
              tk_narrow_supported(m.d_model, m.heads * m.head_dim, m.ffn_dim);
   s.per_layer = s.narrow ? 3 : (s.fused_qa ? 1 : 2) + (s.fuse ? 3 : 5);

@@ -232,10 +232,14 @@ class OptimizedTransformer(BaselineTransformer):
         return built
 
     def _native_model(self) -> _lib.Model:
-        """Addresses of the packed weights as the library's host call takes them."""
+        """Addresses of the packed weights as the library's host call takes them, with the
+        causal flag and the scale as they are now (both may be assigned between calls)."""
         built = self._weights()
-        if self._native is None:
-            if ops.narrow_supported(self.d_model, self.num_heads * self.head_dim_padded, self.config.ffn_dim):
+        now = (bool(self.config.causal), float(self.attn_scale))
+        native = self._native
+        if native is None or native.made_for != now:
+            if built[0].w_qkv_packed is None and ops.narrow_supported(
+                    self.d_model, self.num_heads * self.head_dim_padded, self.config.ffn_dim):
                 for lw in built:
                     lw.w_qkv_packed, lw.w_o_packed = _fragments(lw.w_qkv), _fragments(lw.w_o)
                     lw.w_1_packed, lw.w_2_packed = _fragments(lw.w_1), _fragments(lw.w_2)
@@ -245,11 +249,13 @@ class OptimizedTransformer(BaselineTransformer):
                     val = getattr(lw, name)
                     setattr(dst, name, val.data_ptr() if isinstance(val, torch.Tensor) else val)
             nf_w, nf_b, nf_eps = self._final
-            self._native = _lib.Model(
+            native = _lib.Model(
                 d_model=self.d_model, heads=self.num_heads, head_dim=self.head_dim_padded,
                 ffn_dim=self.config.ffn_dim, num_layers=len(built), layers=layers, nf_w=nf_w.data_ptr(),
-                nf_b=nf_b.data_ptr(), nf_eps=nf_eps, scale=self.attn_scale, causal=int(self.config.causal))
-        return self._native
+                nf_b=nf_b.data_ptr(), nf_eps=nf_eps, scale=now[1], causal=int(now[0]))
+            native.made_for = now
+            self._native = native
+        return native
 
     def __getstate__(self):
         # The addresses belong to this object's packed weights: a copy makes its own.

@@ -155,6 +155,33 @@ def test_copied_model_uses_its_own_weights():
         assert twin._native.layers[0].w_qkv != model._native.layers[0].w_qkv
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("warm,captured", [(64, 200), (200, 64)], ids=["whole_then_layers", "layers_then_whole"])
+def test_capture_after_a_warm_up_of_the_other_path(warm, captured):
+    """Width 128: the capture holds launches of the forward only, so an eager call before the
+    first replay, and each replay, give what a model of the same weights gives eagerly."""
+    torch.manual_seed(73)
+    cfg = tkmi.TransformerConfig(2, 200, 128, 4, 128, 2, True)
+    model = tkmi.OptimizedTransformer(cfg).to(DEV).eval()
+    fresh = copy.deepcopy(model)
+    gen = torch.Generator().manual_seed(74)
+    x = torch.randn(2, captured, 128, generator=gen).to(DEV)
+    with torch.inference_mode():
+        want = fresh(x)
+        model(torch.randn(2, warm, 128, generator=gen).to(DEV))
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(x)
+        assert torch.equal(model(x), want)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            assert torch.equal(model(x), want)
+
+
 def test_bad_calls_are_refused():
     lib = _lib.load()
     assert lib.tk_forward_workspace(None, 1, 1, 1, 0) == _lib.TK_ERR_ARG

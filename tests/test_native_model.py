@@ -23,3 +23,20 @@ def test_changed_settings_reach_the_next_call():
     assert model._native_model().causal == 0
     model.attn_scale = 0.5
     assert model._native_model().scale == 0.5
+
+
+@pytest.mark.parametrize("ffn", [128, 256])
+def test_narrow_fragments_are_packed_with_the_weights(ffn):
+    """Every form of the weights exists once _weights() has run, whichever path a forward takes: a
+    capture of a path that an earlier forward did not take records no packing."""
+    model = _model(d_model=128, ffn=ffn)
+    built = model._weights()
+    n, k = built[0].w_qkv.shape
+    want = built[0].w_qkv.view(n // 32, 32, 8, 2, 8).permute(0, 2, 3, 1, 4)  # block, fragment, half, row, 8 columns
+    assert torch.equal(built[0].w_qkv_packed.flatten(), want.flatten())
+    held = [getattr(lw, name) for lw in built for name in ("w_qkv_packed", "w_o_packed", "w_1_packed", "w_2_packed")]
+    native = model._native_model()
+    assert all(getattr(lw, name) is t for (lw, name), t in zip(
+        [(lw, name) for lw in built for name in ("w_qkv_packed", "w_o_packed", "w_1_packed", "w_2_packed")], held))
+    assert native.layers[1].w_2_packed == held[7].data_ptr()
+    assert _model()._weights()[0].w_qkv_packed is None  # width 256: no kernel reads them

@@ -115,8 +115,7 @@ class _LayerWeights:
     b_1: torch.Tensor
     w_2: torch.Tensor  # [D, F]
     b_2: torch.Tensor
-    # The same in the narrow kernels' fragment order (width 128 only, else None; made
-    # when the layer path first runs).
+    # The same in the narrow kernels' fragment order (width 128 only, else None).
     w_qkv_packed: Optional[torch.Tensor] = None
     w_o_packed: Optional[torch.Tensor] = None
     w_1_packed: Optional[torch.Tensor] = None
@@ -224,12 +223,35 @@ class OptimizedTransformer(BaselineTransformer):
                         w_2=f16(layer.ffn_out.weight), b_2=f32(layer.ffn_out.bias),
                     )
                 )
-        self._final = (f32(self.final_norm.weight), f32(self.final_norm.bias), self.final_norm.eps)
+        final = (f32(self.final_norm.weight), f32(self.final_norm.bias), self.final_norm.eps)
+        stacked = self._pack_fragments(built)
+        self._final, self._stacked, self._native = final, stacked, None
         self._weight_cache = built
         self._weight_cache_key = key
-        self._stacked = None
-        self._native = None
         return built
+
+    def _pack_fragments(self, built: List[_LayerWeights]) -> Optional[dict]:
+        """The fragment orders that the kernels of width 128 read, made with the weights and not when
+        a path first runs: a capture after a warm-up through another path would record the packing,
+        and the weights would hold nothing until its first replay.  Returns _stacked_weights()."""
+        dp, f = self.num_heads * (self.head_dim_padded or 0), self.config.ffn_dim
+        if not ops.narrow_supported(self.d_model, dp, f):
+            return None
+        names = ("w_qkv", "w_o", "w_1", "w_2")
+        if not (built[0].w_qkv.is_cuda
+                and ops.small_forward_supported(1, self.d_model, self.num_heads, self.head_dim_padded, f)):
+            for lw in built:
+                for n in names:
+                    setattr(lw, n + "_packed", _fragments(getattr(lw, n)))
+            return None
+        stacked = {n: torch.stack([getattr(lw, n) for lw in built]).contiguous()
+                   for n in names + ("b_qkv", "b_o", "b_1", "b_2", "n1_w", "n1_b", "n2_w", "n2_b")}
+        stacked["packed"] = ops.small_pack(stacked)
+        # a layer's 12 + 4 + 4 + 4 blocks of 32 rows by 128 columns, in the order of `names`
+        for lw, blocks in zip(built, stacked["packed"].view(len(built), 24, -1)):
+            for n, part in zip(names, blocks.split((12, 4, 4, 4))):
+                setattr(lw, n + "_packed", part)
+        return stacked
 
     def _native_model(self) -> _lib.Model:
         """Addresses of the packed weights as the library's host call takes them, with the
@@ -238,11 +260,6 @@ class OptimizedTransformer(BaselineTransformer):
         now = (bool(self.config.causal), float(self.attn_scale))
         native = self._native
         if native is None or native.made_for != now:
-            if built[0].w_qkv_packed is None and ops.narrow_supported(
-                    self.d_model, self.num_heads * self.head_dim_padded, self.config.ffn_dim):
-                for lw in built:
-                    lw.w_qkv_packed, lw.w_o_packed = _fragments(lw.w_qkv), _fragments(lw.w_o)
-                    lw.w_1_packed, lw.w_2_packed = _fragments(lw.w_1), _fragments(lw.w_2)
             layers = (_lib.Layer * len(built))()
             for dst, lw in zip(layers, built):
                 for name, _ in _lib.Layer._fields_:
@@ -265,11 +282,7 @@ class OptimizedTransformer(BaselineTransformer):
 
     def _stacked_weights(self) -> dict:
         """The per-layer packed weights stacked over layers (tk_small_forward's layout)."""
-        built = self._weights()
-        if self._stacked is None:
-            names = ("w_qkv", "b_qkv", "w_o", "b_o", "w_1", "b_1", "w_2", "b_2", "n1_w", "n1_b", "n2_w", "n2_b")
-            self._stacked = {n: torch.stack([getattr(lw, n) for lw in built]).contiguous() for n in names}
-            self._stacked["packed"] = ops.small_pack(self._stacked)
+        self._weights()
         return self._stacked
 
     def _small_forward_ok(self, seq: int, built: List[_LayerWeights]) -> bool:

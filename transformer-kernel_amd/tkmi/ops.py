@@ -332,7 +332,7 @@ def small_pack(stacked: dict):
     if any(tuple(t.shape) != s or t.dtype != torch.float16 or not t.is_contiguous() for t, s in zip(w, shapes)):
         raise ValueError("small_pack: contiguous fp16 w_qkv [L, 384, 128] and w_o, w_1, w_2 [L, 128, 128] expected")
     packed = torch.empty(_lib.load().tk_small_pack_halves(layers), dtype=torch.float16, device=w[0].device)
-    _launch("small_pack", "tk_small_pack", *(t.data_ptr() for t in w), packed.data_ptr(), layers, _stream(w[0]))
+    _lib.call("tk_small_pack", *(t.data_ptr() for t in w), packed.data_ptr(), layers, _stream(w[0]))
     return packed
 
 

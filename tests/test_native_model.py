@@ -1,5 +1,6 @@
 """The weights' addresses and the settings that a model hands to tk_forward: host code only, no launch."""
 
+import weakref
 from dataclasses import replace
 
 import pytest
@@ -40,3 +41,20 @@ def test_narrow_fragments_are_packed_with_the_weights(ffn):
         [(lw, name) for lw in built for name in ("w_qkv_packed", "w_o_packed", "w_1_packed", "w_2_packed")], held))
     assert native.layers[1].w_2_packed == held[7].data_ptr()
     assert _model()._weights()[0].w_qkv_packed is None  # width 256: no kernel reads them
+
+
+def test_addresses_outlive_a_repacking_by_another_thread():
+    """The table holds the tensors whose addresses it gives away: another thread that packs changed
+    weights drops the model's own references, while this one has not launched yet."""
+    model = _model(d_model=128)
+    native = model._native_model()
+    refs = [weakref.ref(t) for lw in model._weights() for t in vars(lw).values() if isinstance(t, torch.Tensor)]
+    refs += [weakref.ref(t) for t in model._final[:2]]
+    with torch.no_grad():
+        for p in model.parameters():
+            p.add_(1.0)
+    model._weights()
+    assert native.layers[0].w_qkv != model._native_model().layers[0].w_qkv
+    assert all(r() is not None for r in refs)
+    del native
+    assert all(r() is None for r in refs)

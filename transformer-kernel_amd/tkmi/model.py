@@ -255,7 +255,9 @@ class OptimizedTransformer(BaselineTransformer):
 
     def _native_model(self) -> _lib.Model:
         """Addresses of the packed weights as the library's host call takes them, with the
-        causal flag and the scale as they are now (both may be assigned between calls)."""
+        causal flag and the scale as they are now (both may be assigned between calls).
+        The result holds the tensors: it may outlive the model's own references, when
+        another thread packs changed weights before this one has launched."""
         built = self._weights()
         now = (bool(self.config.causal), float(self.attn_scale))
         native = self._native
@@ -271,6 +273,7 @@ class OptimizedTransformer(BaselineTransformer):
                 ffn_dim=self.config.ffn_dim, num_layers=len(built), layers=layers, nf_w=nf_w.data_ptr(),
                 nf_b=nf_b.data_ptr(), nf_eps=nf_eps, scale=now[1], causal=int(now[0]))
             native.made_for = now
+            native.tensors = (built, self._final)
             self._native = native
         return native
 

@@ -182,6 +182,21 @@ def test_capture_after_a_warm_up_of_the_other_path(warm, captured):
             assert torch.equal(model(x), want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(6, 64, 128, 2, 256, 2, True), (6, 64, 768, 12, 768, 1, False)],
+                         ids=["narrow", "wide"])
+def test_batch_invariant_bits_at_one_key_tile(shape):
+    """S = 64, head_dim 64: batches that the fused QKV + attention kernel takes (even ones) and that it does not."""
+    torch.manual_seed(75)
+    model = tkmi.OptimizedTransformer(tkmi.TransformerConfig(*shape),
+                                      tkmi.OptimizerSettings(batch_invariant=True)).to(DEV).eval()
+    x = torch.randn(shape[:3], generator=torch.Generator().manual_seed(76)).to(DEV)
+    with torch.inference_mode():
+        whole = model(x)
+        for n in (1, 2, 3):
+            assert torch.equal(whole, torch.cat([model(x[i:i + n]) for i in range(0, 6, n)])), n
+
+
 def test_bad_calls_are_refused():
     lib = _lib.load()
     assert lib.tk_forward_workspace(None, 1, 1, 1, 0) == _lib.TK_ERR_ARG

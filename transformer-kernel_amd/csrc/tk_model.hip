@@ -61,8 +61,12 @@ Schedule schedule(const tk_model& m, int64_t batch, int64_t seq, bool dense, int
   for (int64_t i = 0; i < m.num_layers; ++i)
     packed = packed && m.layers[i].w_qkv_packed && m.layers[i].w_o_packed && m.layers[i].w_1_packed &&
              m.layers[i].w_2_packed && ((uintptr_t)m.layers[i].b_1 & 15) == 0;
-  s.narrow = packed && !s.fused_qa && (flags & TK_FWD_FUSED_NORM) &&
+  s.narrow = packed && (flags & TK_FWD_FUSED_NORM) &&
              tk_narrow_supported(m.d_model, m.heads * m.head_dim, m.ffn_dim);
+  // Which of the two runs where both take the model depends on the batch (the fused kernel takes
+  // even ones), and their LayerNorm statistics and residual sums round differently.
+  if (flags & TK_FWD_BATCH_INVARIANT) s.fused_qa = s.fused_qa && !s.narrow;
+  else s.narrow = s.narrow && !s.fused_qa;
   s.per_layer = s.narrow ? 3 : (s.fused_qa ? 1 : 2) + (s.fuse ? 3 : 5);
   s.layers = m.num_layers;
   return s;

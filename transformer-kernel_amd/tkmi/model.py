@@ -67,7 +67,9 @@ class OptimizerSettings:
                          kernel (tk_qkv_attention), q/k/v kept on chip.
     batch_invariant   -- only kernels whose order of sums does not depend on the
                          batch size, so that a sequence's output bits are the
-                         same whatever batch it is in; off (default), launches
+                         same in dense batches of every size, and in padded
+                         ones (small_forward, for dense batches only, rounds
+                         otherwise than the layers); off (default), launches
                          that would leave the chip idle split their sums.
     """
 

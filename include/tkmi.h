@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define TKMI_ABI_VERSION 4
+#define TKMI_ABI_VERSION 5
 
 typedef uint16_t tk_half;
 
@@ -138,6 +138,25 @@ int tk_gemm_bias_add_ln(const tk_half *a, int64_t lda, const tk_half *w,
 int tk_gemm_ln_supported(int64_t n);
 
 /*
+ * tk_gemm and tk_gemm_bias_add_ln with one order of sums for every m: an output
+ * row's bits do not depend on how many others the call has.  (Those two split
+ * the k sums of launches that would leave most of the chip idle.)
+ */
+int tk_gemm_invariant(const tk_half *a, int64_t lda, const tk_half *w,
+                      int64_t ldw, const float *bias, const float *resid,
+                      int64_t ldr, void *c, int64_t ldc, int64_t m, int64_t n,
+                      int64_t k, int epilogue, const uint8_t *row_valid,
+                      int row_mode, void *stream);
+int tk_gemm_bias_add_ln_invariant(const tk_half *a, int64_t lda,
+                                  const tk_half *w, int64_t ldw,
+                                  const float *bias, const float *resid,
+                                  const float *ln_w, const float *ln_b,
+                                  float *sum_out, void *h_out, int h_dtype,
+                                  int64_t m, int64_t n, int64_t k, float eps,
+                                  const uint8_t *row_valid, int row_mode,
+                                  void *stream);
+
+/*
  * FlashAttention-2-style forward (online softmax, scores never stored).
  * q, k, v: logical [batch, heads, seq, head_dim] f16 with element strides
  * {b, h, s} given in *_strides[3] (head_dim stride is 1).  out: logical
@@ -167,6 +186,19 @@ int tk_flash_attn_fwd(const tk_half *q, const tk_half *k, const tk_half *v,
                       const int64_t *o_strides, float scale, int causal,
                       const uint8_t *key_valid, int64_t key_valid_stride,
                       void *stream);
+
+/* tk_flash_attn_fwd with kernels whose choice does not depend on batch * heads:
+ * a sequence's bits do not depend on what else the call has.  (That call splits
+ * the keys of launches that would leave most of the chip idle.) */
+int tk_flash_attn_fwd_invariant(const tk_half *q, const tk_half *k,
+                                const tk_half *v, tk_half *out, int64_t batch,
+                                int64_t heads, int64_t seq, int64_t head_dim,
+                                const int64_t *q_strides,
+                                const int64_t *k_strides,
+                                const int64_t *v_strides,
+                                const int64_t *o_strides, float scale,
+                                int causal, const uint8_t *key_valid,
+                                int64_t key_valid_stride, void *stream);
 
 /* 1 when tk_flash_attn_fwd handles head_dim, else 0: the reference's rule
  * next_pow2(max(head_dim, 16)) <= 256, i.e. head_dim <= 256.

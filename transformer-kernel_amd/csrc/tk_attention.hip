@@ -2150,3 +2150,13 @@ extern "C" int tk_flash_attn_fwd(const tk_half* q, const tk_half* k, const tk_ha
   return flash_attn(q, k, v, out, batch, heads, seq, head_dim, q_strides, k_strides, v_strides, o_strides, scale,
                     causal, key_valid, key_valid_stride, false, stream);
 }
+
+extern "C" int tk_flash_attn_fwd_invariant(const tk_half* q, const tk_half* k, const tk_half* v, tk_half* out,
+                                           int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
+                                           const int64_t* q_strides, const int64_t* k_strides,
+                                           const int64_t* v_strides, const int64_t* o_strides, float scale,
+                                           int causal, const uint8_t* key_valid, int64_t key_valid_stride,
+                                           void* stream) {
+  return flash_attn(q, k, v, out, batch, heads, seq, head_dim, q_strides, k_strides, v_strides, o_strides, scale,
+                    causal, key_valid, key_valid_stride, true, stream);
+}

@@ -1553,6 +1553,12 @@ extern "C" int tk_gemm(const tk_half* a, int64_t lda, const tk_half* w, int64_t 
   return gemm(a, lda, w, ldw, bias, resid, ldr, c, ldc, m, n, k, epilogue, row_valid, row_mode, false, stream);
 }
 
+extern "C" int tk_gemm_invariant(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw, const float* bias,
+                                 const float* resid, int64_t ldr, void* c, int64_t ldc, int64_t m, int64_t n,
+                                 int64_t k, int epilogue, const uint8_t* row_valid, int row_mode, void* stream) {
+  return gemm(a, lda, w, ldw, bias, resid, ldr, c, ldc, m, n, k, epilogue, row_valid, row_mode, true, stream);
+}
+
 extern "C" int tk_gemm_ln_supported(int64_t n) { return n == 128 || n == 256 || n == 512; }
 
 // Where the sum is wanted too, it is the residual GEMM's output and the LayerNorm reads
@@ -1616,6 +1622,15 @@ extern "C" int tk_gemm_bias_add_ln(const tk_half* a, int64_t lda, const tk_half*
                                    int row_mode, void* stream) {
   return gemm_bias_add_ln(a, lda, w, ldw, bias, resid, ln_w, ln_b, sum_out, h_out, h_dtype, m, n, k, eps, row_valid,
                           row_mode, false, stream);
+}
+
+extern "C" int tk_gemm_bias_add_ln_invariant(const tk_half* a, int64_t lda, const tk_half* w, int64_t ldw,
+                                             const float* bias, const float* resid, const float* ln_w,
+                                             const float* ln_b, float* sum_out, void* h_out, int h_dtype, int64_t m,
+                                             int64_t n, int64_t k, float eps, const uint8_t* row_valid, int row_mode,
+                                             void* stream) {
+  return gemm_bias_add_ln(a, lda, w, ldw, bias, resid, ln_w, ln_b, sum_out, h_out, h_dtype, m, n, k, eps, row_valid,
+                          row_mode, true, stream);
 }
 
 extern "C" int tk_qkv_attention_supported(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim) {

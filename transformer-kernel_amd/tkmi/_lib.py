@@ -13,7 +13,7 @@ import threading
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_void_p
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "libtkmi.so"
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 TK_OK, TK_ERR_ARG, TK_ERR_UNSUPPORTED, TK_ERR_HIP = 0, -1, -2, -3
 TK_F32, TK_F16 = 0, 1
@@ -116,6 +116,8 @@ SIGNATURES = {
          c_void_p],
     ),
 }
+for _name in ("tk_gemm", "tk_gemm_bias_add_ln", "tk_flash_attn_fwd"):
+    SIGNATURES[_name + "_invariant"] = SIGNATURES[_name]
 
 _lock = threading.Lock()
 _lib = None

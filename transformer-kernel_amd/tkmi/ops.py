@@ -168,15 +168,24 @@ def _check_gemm_operands(a: torch.Tensor, w: torch.Tensor):
         raise ValueError("GEMM operands must be K-contiguous")
 
 
-def linear(a, w, bias=None, gelu: bool = False, out=None, name: Optional[str] = None):
-    """fp16 ``[M, N] = a[M, K] . w[N, K]^T + bias`` (optionally exact GELU), fp32 accumulate."""
+def _variant(fn: str, batch_invariant: bool) -> str:
+    """The entry point whose sums have one order for every batch size, if asked for."""
+    return fn + "_invariant" if batch_invariant else fn
+
+
+def linear(a, w, bias=None, gelu: bool = False, out=None, name: Optional[str] = None, batch_invariant: bool = False):
+    """fp16 ``[M, N] = a[M, K] . w[N, K]^T + bias`` (optionally exact GELU), fp32 accumulate.
+
+    ``batch_invariant`` (here and below): a row's bits do not depend on the number
+    of rows; without it launches that would leave the chip idle split their sums.
+    """
     _check_gemm_operands(a, w)
     m, k = a.shape
     n = w.shape[0]
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=a.device)
     _launch(
-        name or ("gemm_gelu" if gelu else "gemm"), "tk_gemm", a.data_ptr(), a.stride(0), w.data_ptr(),
+        name or ("gemm_gelu" if gelu else "gemm"), _variant("tk_gemm", batch_invariant), a.data_ptr(), a.stride(0), w.data_ptr(),
         w.stride(0), bias.data_ptr() if bias is not None else None, None, 0, out.data_ptr(),
         out.stride(0), m, n, k, TK_EPI_BIAS_GELU if gelu else TK_EPI_BIAS, None, 0, _stream(a),
     )
@@ -184,7 +193,7 @@ def linear(a, w, bias=None, gelu: bool = False, out=None, name: Optional[str] = 
 
 
 def linear_residual(a, w, bias, resid, out=None, name: str = "gemm_resid", row_valid=None,
-                    row_mode: int = TK_ROWS_KEEP_RESID):
+                    row_mode: int = TK_ROWS_KEEP_RESID, batch_invariant: bool = False):
     """fp32 ``out = resid + a . w^T + bias``; ``out`` may be ``resid`` (in place).
 
     ``row_valid`` (optional bool mask over the M rows): an invalid row becomes
@@ -199,7 +208,7 @@ def linear_residual(a, w, bias, resid, out=None, name: str = "gemm_resid", row_v
         out = torch.empty((m, n), dtype=torch.float32, device=a.device)
     rv = _row_mask(row_valid, m)
     _launch(
-        name, "tk_gemm", a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0),
+        name, _variant("tk_gemm", batch_invariant), a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0),
         bias.data_ptr() if bias is not None else None, resid.data_ptr(), resid.stride(0),
         out.data_ptr(), out.stride(0), m, n, k, TK_EPI_BIAS_RESID, rv.data_ptr() if rv is not None else None,
         int(row_mode) if rv is not None else 0, _stream(a),
@@ -213,7 +222,7 @@ def gemm_ln_supported(n: int) -> bool:
 
 def linear_add_ln(a, w, bias, resid, ln_weight, ln_bias, eps: float, out_dtype=torch.float16,
                   sum_out=None, h_out=None, name: str = "gemm_add_ln", row_valid=None,
-                  row_mode: int = TK_ROWS_KEEP_RESID):
+                  row_mode: int = TK_ROWS_KEEP_RESID, batch_invariant: bool = False):
     """``s = resid + a . w^T + bias``; ``h = LN(s)``.
 
     ``sum_out`` receives s when given (it may be ``resid``), from a residual GEMM
@@ -232,7 +241,7 @@ def linear_add_ln(a, w, bias, resid, ln_weight, ln_bias, eps: float, out_dtype=t
         h_out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     rv = _row_mask(row_valid, m)
     _launch(
-        name, "tk_gemm_bias_add_ln", a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0),
+        name, _variant("tk_gemm_bias_add_ln", batch_invariant), a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0),
         bias.data_ptr() if bias is not None else None, resid.data_ptr(), ln_weight.data_ptr(),
         ln_bias.data_ptr(), sum_out.data_ptr() if sum_out is not None else None, h_out.data_ptr(),
         _code(h_out.dtype), m, n, k, float(eps), rv.data_ptr() if rv is not None else None,
@@ -255,7 +264,7 @@ def attention_supported(head_dim: int, dtype: torch.dtype = torch.float16, devic
     return bool(_lib.load().tk_attention_supported(int(head_dim)))
 
 
-def flash_attention(q, k, v, scale: float, causal: bool, out=None, key_valid=None):
+def flash_attention(q, k, v, scale: float, causal: bool, out=None, key_valid=None, batch_invariant: bool = False):
     """Exact attention; returns the context as ``[B, S, H*hd]`` fp16.
 
     q/k/v are logically ``[B, H, S, hd]`` fp16 and may be strided views in
@@ -263,7 +272,8 @@ def flash_attention(q, k, v, scale: float, causal: bool, out=None, key_valid=Non
     the last dim must be contiguous.  ``key_valid`` (optional ``[B, S]`` bool):
     invalid keys are masked like future keys
     (src/torch_transformer_benchmark.py:105-108); a query row with no valid
-    key comes out non-finite, as the baseline's.
+    key comes out non-finite, as the baseline's.  ``batch_invariant``: a sequence's
+    bits do not depend on the batch (as in ``linear``).
     """
     _require_cuda(q, k, v)
     bsz, nh, s, hd = q.shape
@@ -282,7 +292,7 @@ def flash_attention(q, k, v, scale: float, causal: bool, out=None, key_valid=Non
             raise ValueError(f"key_valid must be [B, S] = {(bsz, s)}, got {tuple(key_valid.shape)}")
         kv = _row_mask(key_valid, bsz * s)
     _launch(
-        "flash_attn", "tk_flash_attn_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+        "flash_attn", _variant("tk_flash_attn_fwd", batch_invariant), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
         bsz, nh, s, hd, _lib.strides3(q.stride()[:3]), _lib.strides3(k.stride()[:3]),
         _lib.strides3(v.stride()[:3]), _lib.strides3(o_strides), float(scale), int(bool(causal)),
         kv.data_ptr() if kv is not None else None, s, _stream(q),

@@ -311,7 +311,7 @@ def qkv_attention(h, w_qkv, b_qkv, batch: int, seq: int, heads: int, head_dim: i
     ``h`` [batch*seq, d] fp16, ``w_qkv`` [3d, d] fp16 (q, k, v rows), ``b_qkv``
     [3d] fp32; returns the context ``[batch*seq, d]`` fp16 -- what
     ``linear`` into a q|k|v buffer followed by ``flash_attention`` on its
-    views gives (src/optimized.py:572-626), without the q|k|v buffer.
+    views, both ``batch_invariant``, gives (src/optimized.py:572-626), without the q|k|v buffer.
     """
     _require_cuda(h, w_qkv, b_qkv)
     _check_gemm_operands(h, w_qkv)

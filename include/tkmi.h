@@ -227,8 +227,7 @@ int tk_masked_softmax(const float *scores, tk_half *probs, int64_t groups,
  *   x += u.W_2^T + b_2
  * then out = LN_final(x), with the numerics of the layer-by-layer path
  * (fp16 operands, fp32 accumulation, residual and statistics).
- * x, out: [batch, seq, d_model] f32, or 16-bit as the flags say (out may not
- * alias x).
+ * x, out: [batch, seq, d_model] f32 (out may not alias x).
  * Weights stacked over the layers, each layer's block as the layer-by-layer
  * calls take it: w_qkv [L][3*heads*hd][d] f16 (head rows zero-padded to hd =
  * head_dim_padded), b_qkv [L][3*heads*hd] f32, w_o [L][d][heads*hd] f16,
@@ -407,8 +406,8 @@ typedef struct tk_model {
 
 enum tk_forward_flags {
   TK_FWD_FUSED_NORM = 1,    /* tk_narrow_qkv / tk_narrow_tail where they take the shape and every layer's
-                              packed weights are given, else residual + LayerNorm in the GEMM epilogues
-                              where tk_gemm_ln_supported */
+                              packed weights are given, else tk_gemm_bias_add_ln (with sum_out: a residual
+                              GEMM and a LayerNorm launch, timed as one step) where tk_gemm_ln_supported */
   TK_FWD_QKV_ATTENTION = 2, /* tk_qkv_attention where it takes the shape (dense inputs) */
   TK_FWD_BATCH_INVARIANT = 4, /* no kernel whose choice and order of sums depend on the batch size: a
                                  sequence's output bits are the same in every batch */

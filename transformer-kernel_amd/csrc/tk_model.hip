@@ -23,7 +23,7 @@ const char* const kStepNames[] = {"ln_in", "qkv", "flash_attn", "qkv_attn", "out
 
 struct Schedule {
   bool fused_qa;  // QKV projection and attention in one kernel
-  bool fuse;      // residual + LayerNorm in the GEMM epilogues
+  bool fuse;      // residual GEMM + LayerNorm as one step (tk_gemm_bias_add_ln)
   bool narrow;    // every row-local part of a block in one kernel
   int per_layer;
   int64_t layers;

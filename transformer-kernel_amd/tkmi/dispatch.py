@@ -7,7 +7,8 @@ run per shape, and write the winning settings to a table that
 
 The settings this build can vary per shape are the Python-level ones:
 ``graph`` (replay the forward from a HIP graph, tkmi.graphs) and
-``fused_norm`` (GEMM+LayerNorm epilogue vs residual GEMM + LayerNorm).
+``fused_norm`` (width 128: one kernel after attention; up to width 256 residual
+GEMM + LayerNorm as one operator; off: each as a launch of its own).
 Tile and wave-count choices are made per shape inside the kernels' own C
 dispatch and are not part of the table.
 

@@ -1,4 +1,9 @@
-"""Non-causal attention through the generated steady-state loops, and key masks whose tail is skipped."""
+"""Non-causal attention through the generated steady-state loops, and key masks whose tail is skipped.
+
+Every launch here is small enough for the default call to split its keys over a
+workgroup's waves (tests/test_gpu_attention_keysplit.py); batch_invariant rules
+that out, so that these reach the loops and the trimmed tile counts.
+"""
 
 from __future__ import annotations
 
@@ -26,7 +31,7 @@ def _reference(q, k, v, causal, valid):
 def _check(q, k, v, causal, valid=None):
     b, h, s, hd = q.shape
     got = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal,
-                              key_valid=None if valid is None else valid.to(DEV)).cpu()
+                              key_valid=None if valid is None else valid.to(DEV), batch_invariant=True).cpu()
     want = _reference(q, k, v, causal, valid)
     seen = torch.isfinite(want).all(-1)
     bad, err = or_rule_violations(got[seen], want[seen].float())
@@ -45,7 +50,28 @@ def test_full_attention_over_tile_counts(s, hd):
     _check(q, (k.float() + ramp * q.float().mean((0, 1, 2)).sign()).half(), v, False)
 
 
-@pytest.mark.parametrize("pattern", ["tail", "head", "holes", "one_batch_empty"])
+@pytest.mark.parametrize("masked", [False, True], ids=["dense", "masked"])
+@pytest.mark.parametrize("s", [448, 777, 1344])
+def test_full_loop_is_bit_identical(s, masked):
+    """head_dim 128: the loop does the compiled epochs' arithmetic in their order, also without the causal
+    mask.  K/V rows 4 MiB apart put the copies' span past 32-bit offsets, so the same values take the
+    compiled epochs."""
+    b, h, hd, rs = 2, 1, 128, 1 << 21
+    q, k, v = (seeded(b, h, s, hd, dtype=torch.float16, seed=90 + i).to(DEV) for i in range(3))
+    valid = None
+    if masked:
+        valid = torch.rand(b, s, generator=torch.Generator().manual_seed(5)) > 0.3
+        valid[1, s - 100:] = False
+        valid = valid.to(DEV)
+    wide = torch.zeros(2, b, s, rs, dtype=torch.float16, device=DEV)
+    wide[0, :, :, :hd], wide[1, :, :, :hd] = k[:, 0], v[:, 0]
+    kw, vw = wide[0, :, None, :, :hd], wide[1, :, None, :, :hd]
+    compact = ops.flash_attention(q, k, v, hd ** -0.5, False, key_valid=valid, batch_invariant=True)
+    spread = ops.flash_attention(q, kw, vw, hd ** -0.5, False, key_valid=valid, batch_invariant=True)
+    assert torch.equal(compact, spread)
+
+
+@pytest.mark.parametrize("pattern", ["tail", "short", "head", "holes", "one_batch_empty"])
 @pytest.mark.parametrize("causal", [False, True], ids=["full", "causal"])
 @pytest.mark.parametrize("hd", [32, 64, 128, 256, 80])
 def test_key_masks(hd, causal, pattern):
@@ -56,6 +82,10 @@ def test_key_masks(hd, causal, pattern):
         valid[0, 1:] = False
         valid[1, 512:] = False
         valid[2, 513:] = False
+    elif pattern == "short":  # one tile, a key past it, two tiles and a key
+        valid[0, 64:] = False
+        valid[1, 65:] = False
+        valid[2, 129:] = False
     elif pattern == "head":
         valid[:, :200] = False
     elif pattern == "holes":
@@ -71,6 +101,6 @@ def test_eight_byte_value_rows_keep_their_path():
     q, k, v = (seeded(b, h, s, hd, dtype=torch.float16, seed=80 + i) for i in range(3))
     wide = torch.zeros(b, h, s, hd + 4, dtype=torch.float16, device=DEV)
     wide[..., 4:] = v.to(DEV)
-    got = ops.flash_attention(q.to(DEV), k.to(DEV), wide[..., 4:], hd ** -0.5, False).cpu()
+    got = ops.flash_attention(q.to(DEV), k.to(DEV), wide[..., 4:], hd ** -0.5, False, batch_invariant=True).cpu()
     bad, err = or_rule_violations(got, _reference(q, k, v, False, None).float())
     assert bad == 0, err

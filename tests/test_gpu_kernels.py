@@ -325,11 +325,12 @@ def _qkv(shape, seed=1):
 def test_flash_attention_matches_reference(shape, causal):
     b, h, s, hd = shape
     q, k, v = _qkv(shape)
-    out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal)
     ref = ob.attention_ref(q, k, v, hd ** -0.5, causal)
-    assert out.shape == (b, s, h * hd)
-    bad, err = or_rule_violations(out, ref, atol=2e-3, rtol=2e-2)
-    assert bad == 0, err
+    for invariant in (False, True):  # the default splits the keys of most of these launches
+        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, batch_invariant=invariant)
+        assert out.shape == (b, s, h * hd)
+        bad, err = or_rule_violations(out, ref, atol=2e-3, rtol=2e-2)
+        assert bad == 0, (invariant, err)
 
 
 def test_flash_attention_strided_qkv_views():
@@ -357,20 +358,22 @@ def test_flash_attention_ragged_sequence_lengths(s):
     b, h, hd = 1, 2, 32
     q, k, v = _qkv((b, h, s, hd), seed=s)
     for causal in (True, False):
-        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal)
-        bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, causal))
-        assert bad == 0, (causal, err)
+        for invariant in (False, True):
+            out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, batch_invariant=invariant)
+            bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, causal))
+            assert bad == 0, (causal, invariant, err)
 
 
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("s", [512, 600, 777, 1000, 1300])
 def test_flash_attention_long_ragged(s, hd):
     """Long sequences (the two-group kernel): lengths off the 64-key tile and
-    256-row block grid, causal and full."""
+    256-row block grid, causal and full.  (batch_invariant here and below: the
+    default call splits the keys of launches as small as these.)"""
     b, h = 1, 2
     q, k, v = _qkv((b, h, s, hd), seed=s + hd)
     for causal in (True, False):
-        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal)
+        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, batch_invariant=True)
         bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, causal))
         assert bad == 0, (causal, err)
 
@@ -388,7 +391,7 @@ def test_flash_attention_epoch_loop_is_bit_identical(s, hd):
     b, h = 1, 1
     q, k, v = _qkv((b, h, s, hd), seed=s)
     qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
-    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True)
+    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True, batch_invariant=True)
     rs = 1 << 21  # fp16 elements between K (and V) rows
     wide_k = torch.zeros(s, rs, dtype=torch.float16, device=DEV)
     wide_v = torch.zeros(s, rs, dtype=torch.float16, device=DEV)
@@ -396,7 +399,7 @@ def test_flash_attention_epoch_loop_is_bit_identical(s, hd):
     wide_v[:, :hd] = vd[0, 0]
     kw, vw = wide_k[:, :hd][None, None], wide_v[:, :hd][None, None]
     assert kw.stride(2) == rs and torch.equal(kw, kd)
-    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True)
+    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True, batch_invariant=True)
     del wide_k, wide_v
     assert torch.equal(compact, spread)
     bad, err = or_rule_violations(compact, ob.attention_ref(q, k, v, hd ** -0.5, True))
@@ -412,7 +415,7 @@ def test_flash_attention_epoch_loop_boundaries(hd, s):
     min(q0/64, min(n_kt, S/64) - 2)), against the reference."""
     b, h = 1, 2
     q, k, v = _qkv((b, h, s, hd), seed=3 * s + hd)
-    out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, True)
+    out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, True, batch_invariant=True)
     bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, True))
     assert bad == 0, err
 
@@ -441,7 +444,7 @@ def test_flash_attention_long_strided_views(hd):
     q, k, v = qkv.to(DEV).permute(2, 0, 3, 1, 4).unbind(0)
     qc, kc, vc = qkv.permute(2, 0, 3, 1, 4).unbind(0)
     for causal in (True, False):
-        out = ops.flash_attention(q, k, v, hd ** -0.5, causal)
+        out = ops.flash_attention(q, k, v, hd ** -0.5, causal, batch_invariant=True)
         bad, err = or_rule_violations(out, ob.attention_ref(qc, kc, vc, hd ** -0.5, causal))
         assert bad == 0, (causal, err)
 
@@ -457,7 +460,7 @@ def test_flash_attention_large_logits(hd):
     q = (q.float() * ramp).half()
     k = (k.float() * 2.0).half()
     for causal in (True, False):
-        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal)
+        out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, batch_invariant=True)
         bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, causal))
         assert bad == 0, (causal, err)
 
@@ -486,10 +489,10 @@ def test_flash_attention_scores_rising_along_keys(hd, slope):
     assert torch.isfinite(k).all()
     qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
     for causal in (True, False):
-        out = ops.flash_attention(qd, kd, vd, hd ** -0.5, causal)
+        out = ops.flash_attention(qd, kd, vd, hd ** -0.5, causal, batch_invariant=True)
         bad, err = or_rule_violations(out, ob.attention_ref(q, k, v, hd ** -0.5, causal))
         assert bad == 0, (causal, err)
-    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True)
+    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True, batch_invariant=True)
     rs = 1 << 21
     wide_k = torch.zeros(b * h * s, rs, dtype=torch.float16, device=DEV)
     wide_v = torch.zeros(b * h * s, rs, dtype=torch.float16, device=DEV)
@@ -498,7 +501,7 @@ def test_flash_attention_scores_rising_along_keys(hd, slope):
     kw = wide_k.view(b, h, s, rs)[..., :hd]
     vw = wide_v.view(b, h, s, rs)[..., :hd]
     assert kw.stride(2) == rs and torch.equal(kw, kd)
-    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True)
+    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True, batch_invariant=True)
     del wide_k, wide_v
     assert torch.equal(compact, spread)
 
@@ -525,7 +528,8 @@ def test_flash_attention_key_mask(shape, causal):
     g = torch.Generator().manual_seed(s)
     kv = torch.rand(b, s, generator=g) < 0.7
     kv[0, s // 2:] = False  # a prefix mask in batch 0
-    out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, key_valid=kv.to(DEV)).cpu()
+    out = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), hd ** -0.5, causal, key_valid=kv.to(DEV),
+                              batch_invariant=True).cpu()
     ref = _attention_ref_keymask(q, k, v, hd ** -0.5, causal, kv)
     allowed = torch.ones(s, s, dtype=torch.bool).tril() if causal else torch.ones(s, s, dtype=torch.bool)
     seen = (kv[:, None, :] & allowed[None]).any(-1)  # [b, s]: query rows with a valid key
@@ -556,7 +560,7 @@ def test_flash_attention_key_masked_loop_is_bit_identical(pattern, hd):
     else:
         kv = torch.rand(b, s, generator=torch.Generator().manual_seed(5)) > 0.3
     qd, kd, vd, kvd = q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV)
-    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True, key_valid=kvd)
+    compact = ops.flash_attention(qd, kd, vd, hd ** -0.5, True, key_valid=kvd, batch_invariant=True)
     rs = 1 << 21
     wide_k = torch.zeros(b, s, rs, dtype=torch.float16, device=DEV)
     wide_v = torch.zeros(b, s, rs, dtype=torch.float16, device=DEV)
@@ -564,7 +568,7 @@ def test_flash_attention_key_masked_loop_is_bit_identical(pattern, hd):
     wide_v[:, :, :hd] = vd[:, 0]
     kw, vw = wide_k[:, :, :hd][:, None], wide_v[:, :, :hd][:, None]
     assert kw.stride(2) == rs and torch.equal(kw, kd)
-    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True, key_valid=kvd)
+    spread = ops.flash_attention(qd, kw, vw, hd ** -0.5, True, key_valid=kvd, batch_invariant=True)
     del wide_k, wide_v
     same = (compact == spread) | (torch.isnan(compact) & torch.isnan(spread))
     assert bool(same.all())

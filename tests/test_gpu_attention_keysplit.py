@@ -20,8 +20,8 @@ def _qkv(b, h, s, hd, seed):
 
 
 # One key past a tile, fewer tiles than waves, tiles of four and eight waves that end
-# unevenly, the last launch inside the rule (512 blocks of 32 rows) and the first past it
-# (for head_dim 256 that is the pipelined generic kernel).
+# unevenly, 512 blocks of 32 rows (the last launch inside the rule at most head dims) and
+# more (for head_dim 256 that is the pipelined generic kernel).
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "full"])
 @pytest.mark.parametrize("hd", [32, 64, 128, 256])
 @pytest.mark.parametrize("b,h,s", [(1, 1, 65), (2, 3, 127), (1, 5, 200), (1, 2, 513), (1, 2, 1057), (2, 1, 1990),
@@ -99,3 +99,17 @@ def test_batch_invariant_model():
     with torch.inference_mode():
         whole, alone = model(x), torch.cat([model(x[i:i + 1]) for i in range(24)])
     assert torch.equal(whole, alone)
+
+
+# Two workgroups per CU: one key tile too few, B*H off the XCD count, and the first inside each line.
+@pytest.mark.parametrize("b,s,hd,causal,split", [
+    (128, 128, 128, True, False), (128, 127, 128, False, False), (128, 128, 128, False, True),
+    (80, 160, 128, True, True), (72, 192, 256, False, False), (64, 256, 256, False, True),
+    (85, 192, 64, False, False), (80, 192, 64, False, True), (19, 512, 64, False, True), (170, 192, 32, True, False)])
+def test_rule_past_one_workgroup_per_cu(b, s, hd, causal, split):
+    q, k, v = (t.to(DEV) for t in _qkv(b, 1, s, hd, seed=s + hd))
+    out = ops.flash_attention(q, k, v, hd ** -0.5, causal)
+    assert torch.equal(out, ops.flash_attention(q, k, v, hd ** -0.5, causal, batch_invariant=True)) != split
+    few = slice(0, 4)
+    bad, err = or_rule_violations(out[few], ob.attention_ref(q[few].cpu(), k[few].cpu(), v[few].cpu(), hd ** -0.5, causal))
+    assert bad == 0, err

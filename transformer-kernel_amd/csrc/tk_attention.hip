@@ -1988,18 +1988,27 @@ __global__ __launch_bounds__(NW * 64, HD <= 64 ? 2 : 1) void flash_keysplit_kern
   keysplit_body<HD, NW, CAUSAL, KMASK>(p);
 }
 // Where the key-split kernel is taken: head dims 32, 64, 128 and 256, more than one key
-// tile, and at most two workgroups of it per CU (32 query rows each).  Measured on 87
-// launches, us (others -> key split): b1 h16 s512 causal, head_dim 64 10.1 -> 5.7,
-// 128 23.8 -> 8.9, 32 8.6 -> 4.7, 256 38.0 -> 16.9; b1 h4 s2048 23.1 -> 11.0 (eight waves); at 512
-// workgroups, b1 h16 s1024 without the causal mask 14.1 -> 11.8, 128 31.6 -> 25.3,
-// 32 12.8 -> 8.4, 256 66.3 -> 51.5.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs 12.6,
-// b1 h16 s2048 full 26.1 vs 35.5) except for head_dim 32 causal (b1 h16 s2048 24.5 ->
-// 18.3, b64 h4 s128 6.6 -> 6.4).  Eight waves: from 1024 keys, one workgroup per CU
-// (b1 h1 s4096 22.7 -> 17.7; b1 h16 s512 5.7 vs 5.9).
+// tile, few workgroups (32 query rows each).  Figures: us, others -> key split.
+// Up to one per CU it wins at every length: b1 h16 s512 causal, head_dim 64 10.1 -> 5.7,
+// 128 23.8 -> 8.9, 32 8.6 -> 4.7, 256 38.0 -> 16.9; b1 h4 s2048 23.1 -> 11.0 (eight waves:
+// past 1024 keys, one workgroup per CU; b1 h1 s4096 22.7 -> 17.7, b1 h16 s512 5.7 vs 5.9).
+// Up to two per CU (1024 workgroups at head_dim 32 causal) its 32-row blocks read K and V
+// from L2 twice as often, which pays where a head's blocks share an XCD (ids are dealt
+// round-robin over 8: B*H a multiple of 8) or the sequence is long: b64 h1 s256 head_dim
+// 64 full 7.0 -> 5.8, but b51 h1 s256 7.3 -> 7.5, b85 h1 s192 6.5 -> 7.5; b1 h16 s1024
+// full 14.1 -> 11.8, 128 31.6 -> 25.3.  At head_dim 128 and 256 a CU holds one workgroup,
+// so there are two rounds, which only longer chains repay: 128, b170 h1 s65 causal 8.5 vs
+// 10.8, b128 h1 s128 causal 10.1 vs 11.1, full 10.8 -> 10.0; 256 full, s192 1.08
+// times the other, s256 0.95.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs
+// 12.6, b1 h16 s2048 full 26.1 vs 35.5) except for head_dim 32 causal (b1 h16 s2048 24.5
+// -> 18.3, b64 h4 s128 6.6 -> 6.4).
 int64_t keysplit_blocks(int64_t bh, int64_t s) { return bh * ((s + 31) / 32); }
 bool keysplit_pays(int64_t bh, int64_t s, int64_t hd, bool causal) {
-  return (hd == 32 || hd == 64 || hd == 128 || hd == 256) && s > 64 &&
-         keysplit_blocks(bh, s) <= (hd == 32 && causal ? 1024 : 512);
+  if ((hd != 32 && hd != 64 && hd != 128 && hd != 256) || s <= 64) return false;
+  const int64_t blocks = keysplit_blocks(bh, s);
+  if (blocks <= 256) return true;
+  if (blocks > (hd == 32 && causal ? 1024 : 512) || (bh % 8 != 0 && s < 512)) return false;
+  return hd <= 64 || (hd == 128 ? s > (causal ? 128 : 127) : causal || s >= 256);
 }
 template <int HD, int NW>
 int launch_keysplit(const AttnArgs& p, bool causal, hipStream_t st) {

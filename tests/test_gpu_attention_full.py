@@ -104,3 +104,25 @@ def test_eight_byte_value_rows_keep_their_path():
     got = ops.flash_attention(q.to(DEV), k.to(DEV), wide[..., 4:], hd ** -0.5, False, batch_invariant=True).cpu()
     bad, err = or_rule_violations(got, _reference(q, k, v, False, None).float())
     assert bad == 0, err
+
+
+@pytest.mark.parametrize("hd", [16, 32, 64, 128, 256, 80])
+@pytest.mark.parametrize("s", [320, 321])
+def test_tail_skipping_around_its_line(s, hd):
+    """Key masks at the longest length without the scan for the last valid key and the shortest
+    with it, in launches of as many workgroups as CUs and of more (the scan's other condition);
+    batch_invariant launches take it at every batch, with the same bits."""
+    h = 64
+    valid = torch.ones(3, s, dtype=torch.bool)
+    valid[0, 1:] = False
+    valid[1, 200:] = False
+    q, k, v = (seeded(3, 1, s, hd, dtype=torch.float16, seed=60 + i).expand(3, h, s, hd).to(DEV) for i in range(3))
+    want = _reference(*(t[:, :1].cpu() for t in (q, k, v)), False, valid).float()
+    whole = ops.flash_attention(q, k, v, hd ** -0.5, False, key_valid=valid.to(DEV), batch_invariant=True)
+    for b in (1, 3):
+        got = ops.flash_attention(q[:b], k[:b], v[:b], hd ** -0.5, False, key_valid=valid[:b].to(DEV))
+        bad, err = or_rule_violations(got[..., -hd:], want[:b])
+        assert bad == 0, (b, err)
+        got = ops.flash_attention(q[:b], k[:b], v[:b], hd ** -0.5, False, key_valid=valid[:b].to(DEV),
+                                  batch_invariant=True)
+        assert torch.equal(got, whole[:b])

@@ -61,6 +61,8 @@ struct AttnArgs {
   int64_t kvs;
   int B, H, S;
   float scale_log2;  // scale * log2(e)
+  bool one_order;    // no choice that depends on B or H (TK_FWD_BATCH_INVARIANT)
+  bool trim;         // skip the key tiles after the last valid key (valid_tiles)
 };
 
 // ---- register-staged V (flash_vreg_body) ----
@@ -71,12 +73,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 // Position of key k (0..63 within the tile) in a V^T row: bits 2 and 3 swapped.
 __device__ __forceinline__ int vpos(int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); }
 
-// The bodies are __device__ functions (the __global__ wrapper below only
-// calls them): device-only builtins used directly in a kernel template's
-// lambdas would make the host-side instantiation, and with it the launch
-// stub, fail.  KMASK: the key-validity mask p.kv is applied (a separate
-// instantiation, so the unmasked kernels carry none of its registers or
-// loads).
 // Number of key tiles up to the last one with a valid key (at least 1): the tiles
 // after it change no row's max, sum or O, so a padded batch skips the tail of
 // its shorter sequences (b6 h12 s777 head_dim 64, lengths from 70 %: 28.5 ->
@@ -84,13 +80,13 @@ __device__ __forceinline__ int vpos(int k) { return (k & ~12) | ((k & 4) << 1) |
 // Not for causal launches: their query blocks end at the diagonal, only those past
 // the padding would gain, and the scan cost more (head_dim 256 s369 +4 %).
 template <bool TRIM>
-__device__ __forceinline__ int valid_tiles(const uint8_t* kvb, int n_kt, int S) {
-  if constexpr (!TRIM) return n_kt;
+__device__ __forceinline__ int valid_tiles(const AttnArgs& p, const uint8_t* kvb, int n_kt) {
+  if (!TRIM || !p.trim) return n_kt;
   const int lane = threadIdx.x & 63;
   for (int base = ((n_kt - 1) / 4) * 4; base >= 0; base -= 4) {
     uint8_t by[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) by[i] = kvb[min((base + i) * kBN + lane, S - 1)];
+    for (int i = 0; i < 4; ++i) by[i] = kvb[min((base + i) * kBN + lane, p.S - 1)];
 #pragma unroll
     for (int i = 3; i >= 0; --i)
       if (base + i < n_kt && __ballot(by[i] != 0) != 0ull) return __builtin_amdgcn_readfirstlane(base + i + 1);
@@ -98,7 +94,28 @@ __device__ __forceinline__ int valid_tiles(const uint8_t* kvb, int n_kt, int S) 
   return 1;
 }
 
-template <int HD, int NW, bool CAUSAL, bool KMASK>
+// Where it is asked for: the scan is a load latency ahead of everything else in a
+// workgroup, 0.2 to 0.4 us.  Up to five key tiles that is as much as a dropped tile gives (lengths
+// from 70 %: head_dim 32 b20 h16 s176 14.1 -> 14.9 us, 16 b7 h12 s320 9.7 -> 9.9, 128 b44
+// h16 s128 34.9 -> 36.7; from six on 64 b20 h12 s480 63.5 -> 52.5), and where every workgroup
+// has a CU the longest sequence sets the time (16 b3 h1 s640 14.3 -> 14.6).  (The scan
+// decides which steps the head_dim-64 loop covers, whose row sums round otherwise than the
+// compiled ones: one_order launches don't look at the number of blocks.)
+constexpr int kTrimFrom = 320;
+AttnArgs trimmed(AttnArgs p, bool causal, int64_t blocks) {
+  p.trim = p.kv != nullptr && !causal && p.S > kTrimFrom && (blocks > 256 || p.one_order);
+  return p;
+}
+
+// The bodies are __device__ functions (the __global__ wrapper below only
+// calls them): device-only builtins used directly in a kernel template's
+// lambdas would make the host-side instantiation, and with it the launch
+// stub, fail.  KMASK: the key-validity mask p.kv is applied (a separate
+// instantiation, so the unmasked kernels carry none of its registers or
+// loads).
+// LONG: with the generated loop (head_dim 64) and the scan of valid_tiles, whose code costs
+// the launches that take neither 2 to 5 % (flash_short_kernel).
+template <int HD, int NW, bool CAUSAL, bool KMASK, bool LONG = true>
 __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   constexpr int BM = 32 * NW;
   constexpr int RB = HD * 2;               // K / V tile row bytes
@@ -168,7 +185,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL && LONG>(p, kvb, (kv_end + kBN - 1) / kBN);
 
   // ---- copies: lane sources within a tile are fixed; a tile adds 64 rows ----
   // Lane l of wave copy ci writes physical chunk l % CPR of tile row
@@ -446,7 +463,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   // copies use 32-bit offsets from the K and V bases (span check) and the K read
   // addresses are formed by XOR on bits 5-6 of a 256-byte-aligned row offset.
   int groups = 0;
-  if constexpr (HD == 64 && (NW == 4 || NW == 8)) {
+  if constexpr (LONG && HD == 64 && (NW == 4 || NW == 8)) {
     int last = min(n_kt, p.S / kBN) - 3;
     if constexpr (CAUSAL) last = min(last, q0 / kBN - 1);
     const int64_t span =
@@ -466,7 +483,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
     // Two steps per iteration with no branch between them: the loop-carried
     // accumulators then keep one register assignment.
     int kt = 1;
-    if constexpr (HD == 64 && (NW == 4 || NW == 8)) {
+    if constexpr (LONG && HD == 64 && (NW == 4 || NW == 8)) {
       if (groups > 0) {
         // Pinned: O^T v[64:95], Q v[96:111], the scores of tile kt v[112:143] (s_b), P of
         // tile kt-1 v[144:159] (pf_a), m_run v161, l_run v162; v160 (mx_b, no longer read
@@ -642,7 +659,7 @@ __device__ __forceinline__ void flash_vreg_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  const int n_kt = (kv_end + kBN - 1) / kBN;  // (no valid_tiles: S <= 128, or V rows that nothing copies)
 
   // ---- K tile: direct copies; per-lane source offsets fixed, tile stride added ----
   int k_src_row[K_CPW], k_src_col[K_CPW];
@@ -968,7 +985,7 @@ __device__ __forceinline__ void flash_ring_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(p, kvb, (kv_end + kBN - 1) / kBN);
 
   // ---- copies (the layouts of flash_dma_body) ----
   int c_row[CPW], k_col[CPW], v_col[CPW];
@@ -1251,7 +1268,7 @@ __device__ __forceinline__ void flash_pair_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(p, kvb, (kv_end + kBN - 1) / kBN);
 
   // ---- copies (the layouts of flash_dma_body) ----
   int c_row[CPW];
@@ -1770,7 +1787,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
   const bool d_ok = HDP % 32 == 0 || (lane & 31) < HDP;
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(kvb, (kv_end + kBN - 1) / kBN, p.S);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL>(p, kvb, (kv_end + kBN - 1) / kBN);
   // VEC: one K and one V slot, filled by direct copies, 1 KB per wave and copy; the
   // next K tile is on its way from the moment that every wave has this one's
   // fragments, the next V tile from the end of P.V, so each crosses the other
@@ -1909,8 +1926,9 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
 }
 
 template <int HDP, bool VEC = false>
-int launch_generic(const AttnArgs& p, int hd, bool causal, hipStream_t st) {
-  const int64_t grid = (int64_t)((p.S + 127) / 128) * p.B * p.H;
+int launch_generic(const AttnArgs& args, int hd, bool causal, hipStream_t st) {
+  const int64_t grid = (int64_t)((args.S + 127) / 128) * args.B * args.H;
+  const AttnArgs p = trimmed(args, causal, grid);
   const dim3 g((unsigned)grid), blk(256);
   const bool km = p.kv != nullptr;
   if (causal && km)
@@ -1947,6 +1965,14 @@ __global__ __launch_bounds__(NW * 64, (NW <= 4 && HD <= 64) ? 2 : 1) void flash_
     flash_dma_body<HD, NW, CAUSAL, KMASK>(p);
   }
 }
+// Without the causal mask: head_dim 64 below the loop's first length, and 16 and 32 with a key
+// mask that is not scanned.  b54 h2 s80 d64 5.4 -> 5.2 us, b18 h8 s159 d64 masked 9.8 -> 9.3,
+// b20 h16 s176 d32 masked 14.9 -> 14.1.
+constexpr int kShortS = 320;  // five whole key tiles: one group of two steps
+template <int HD, int NW, bool KMASK>
+__global__ __launch_bounds__(NW * 64, 2) void flash_short_kernel(AttnArgs p) {
+  flash_dma_body<HD, NW, false, KMASK, false>(p);
+}
 // head_dim 128 without the causal mask, more than 128 keys, V rows 16-byte
 // vectors: the pair body too, whose asm loop then covers all but the first and the
 // last few key tiles.  Against the register body (kept for V rows of 8-byte
@@ -1958,8 +1984,10 @@ template <bool KMASK>
 __global__ __launch_bounds__(512, 1) void flash_full_kernel(AttnArgs p) {
   flash_pair_body<128, 8, false, KMASK>(p);
 }
-int launch_full128(const AttnArgs& p, hipStream_t st) {
-  const dim3 g((unsigned)((int64_t)((p.S + 255) / 256) * p.B * p.H)), blk(512);
+int launch_full128(const AttnArgs& args, hipStream_t st) {
+  const int64_t grid = (int64_t)((args.S + 255) / 256) * args.B * args.H;
+  const AttnArgs p = trimmed(args, false, grid);
+  const dim3 g((unsigned)grid), blk(512);
   if (p.kv) hipLaunchKernelGGL((flash_full_kernel<true>), g, blk, 0, st, p);
   else hipLaunchKernelGGL((flash_full_kernel<false>), g, blk, 0, st, p);
   return check_launch("tk_flash_attn_fwd");
@@ -2022,12 +2050,20 @@ int launch_keysplit(const AttnArgs& p, bool causal, hipStream_t st) {
 }
 
 template <int HD, int NW>
-int launch_flash(const AttnArgs& p, bool causal, hipStream_t st) {
+int launch_flash(const AttnArgs& args, bool causal, hipStream_t st) {
   constexpr int BM = 32 * NW;
-  const int64_t n_qt = (p.S + BM - 1) / BM;
-  const int64_t grid = n_qt * p.B * p.H;
+  const int64_t n_qt = (args.S + BM - 1) / BM;
+  const int64_t grid = n_qt * args.B * args.H;
+  const AttnArgs p = trimmed(args, causal, grid);
   const dim3 g((unsigned)grid), blk(NW * 64);
   const bool km = p.kv != nullptr;
+  if constexpr (HD <= 64 && NW == 4) {
+    if (!causal && (HD == 64 ? p.S < kShortS : km && !p.trim)) {
+      if (km) hipLaunchKernelGGL((flash_short_kernel<HD, NW, true>), g, blk, 0, st, p);
+      else hipLaunchKernelGGL((flash_short_kernel<HD, NW, false>), g, blk, 0, st, p);
+      return check_launch("tk_flash_attn_fwd");
+    }
+  }
   if (causal && km)
     hipLaunchKernelGGL((flash_fwd_kernel<HD, NW, true, true>), g, blk, 0, st, p);
   else if (causal)
@@ -2108,6 +2144,7 @@ int tk::flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half
   p.kvs = key_valid_stride;
   p.B = (int)batch; p.H = (int)heads; p.S = (int)seq;
   p.scale_log2 = scale * 1.4426950408889634f;
+  p.one_order = batch_invariant;
   hipStream_t st = as_stream(stream);
   const bool c = causal != 0;
   // Vector paths: q, k rows 16-byte vectors (register / LDS-DMA copies); v

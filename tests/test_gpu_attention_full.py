@@ -126,3 +126,12 @@ def test_tail_skipping_around_its_line(s, hd):
         got = ops.flash_attention(q[:b], k[:b], v[:b], hd ** -0.5, False, key_valid=valid[:b].to(DEV),
                                   batch_invariant=True)
         assert torch.equal(got, whole[:b])
+
+
+@pytest.mark.parametrize("b,s", [(65, 513), (89, 513), (90, 513), (65, 300)])
+def test_element_loads_around_one_workgroup_per_cu(b, s):
+    """Causal head_dim 100: 325 and 445 workgroups (one per CU), 450 and short sequences (two)."""
+    q, k, v = (seeded(b, 1, s, 100, dtype=torch.float16, seed=30 + i) for i in range(3))
+    got = ops.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), 0.1, True).cpu()
+    bad, err = or_rule_violations(got[-3:], _reference(q[-3:], k[-3:], v[-3:], True, None).float())
+    assert bad == 0, err

@@ -1720,8 +1720,11 @@ __device__ __forceinline__ void flash_single_body(const AttnArgs& p) {
 // instead of a load through registers between two barriers: b2 h8 s4096 causal
 // 481 -> 295 us, full 866 -> 504 (546 TFLOP/s), b4 h8 s1024 100 -> 69, b64 h4
 // s128 24.5 -> 21.6 (3.1 TB/s).
+// Waves per SIMD: at HDP 64 and 128 three and two, which keep the accumulators in VGPRs (an
+// AGPR move for each costs one wave per SIMD here): b60 h2 s700 d80 causal 137 -> 100 us, full 201 ->
+// 150, b1 h2 s1500 d80 132 -> 124, b300 h2 s300 d40 80 -> 67.
 template <int HDP, bool CAUSAL, bool KMASK, bool VEC>
-__global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) {
+__global__ __launch_bounds__(256, HDP == 128 ? 2 : HDP == 64 ? 3 : 1) void flash_generic_kernel(AttnArgs p, int hd) {
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
   constexpr int RB = HDP * 2;              // K / V tile row bytes
   constexpr int CPR = RB / 16;             // 16-byte chunks per row
@@ -1787,7 +1790,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
   const bool d_ok = HDP % 32 == 0 || (lane & 31) < HDP;
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL>(p, kvb, (kv_end + kBN - 1) / kBN);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL && VEC>(p, kvb, (kv_end + kBN - 1) / kBN);
   // VEC: one K and one V slot, filled by direct copies, 1 KB per wave and copy; the
   // next K tile is on its way from the moment that every wave has this one's
   // fragments, the next V tile from the end of P.V, so each crosses the other
@@ -1808,8 +1811,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
     copy(vb, p.vs[2], 0, v_lds, true);
   }
   for (int kt = 0; kt < n_kt; ++kt) {
-    const int k0 = kt * kBN;
-    const bool more = kt + 1 < n_kt;
+    const int k0 = kt * kBN;  // (no kt + 1 outside the VEC parts: it costs the others 2 to 5 %)
     if constexpr (!VEC) {
       __syncthreads();  // the previous tile's operands are no longer read
 #pragma unroll
@@ -1849,7 +1851,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
     if constexpr (VEC) {
       wait_lds_reads();  // this wave's K fragments are in registers
       lds_barrier();
-      if (more) copy(kb, p.ks[2], kt + 1, k_lds, false);
+      if (kt + 1 < n_kt) copy(kb, p.ks[2], kt + 1, k_lds, false);
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -1881,7 +1883,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
       l_run += (float)ph;
     }
     if constexpr (VEC) {
-      if (more) wait_vmcnt<CPW>();  // all but the next K's copies
+      if (kt + 1 < n_kt) wait_vmcnt<CPW>();  // all but the next K's copies
       else wait_vmcnt<0>();
       lds_barrier();
     }
@@ -1897,7 +1899,7 @@ __global__ __launch_bounds__(256) void flash_generic_kernel(AttnArgs p, int hd) 
       acc_o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[t], acc_o[d], 0, 0, 0);
     }
     if constexpr (VEC) {
-      if (more) {
+      if (kt + 1 < n_kt) {
         wait_lds_reads();
         lds_barrier();
         copy(vb, p.vs[2], kt + 1, v_lds, true);
@@ -1931,14 +1933,21 @@ int launch_generic(const AttnArgs& args, int hd, bool causal, hipStream_t st) {
   const AttnArgs p = trimmed(args, causal, grid);
   const dim3 g((unsigned)grid), blk(256);
   const bool km = p.kv != nullptr;
+  // Causal launches of few more workgroups than CUs: the first 256 (the longest) set the time, so
+  // one to a CU (unused LDS keeps a second away), as when there was no room for two (head_dim 100
+  // b30 h1 s1500, two per CU 160 us, one 147; b15 h1 s4000 418 vs 404; past 448, 512 if long, and
+  // for short sequences two win: b40 s1500 166 vs 166, b53 181 vs 234, b100 s300 43 vs 54).
+  const bool one_per_cu = !VEC && HDP == 128 && causal && p.S >= 512 && grid > 256 &&
+                          grid <= (p.S < 2048 ? 448 : 512);
+  const unsigned lds = one_per_cu ? 50u << 10 : 0u;
   if (causal && km)
-    hipLaunchKernelGGL((flash_generic_kernel<HDP, true, true, VEC>), g, blk, 0, st, p, hd);
+    hipLaunchKernelGGL((flash_generic_kernel<HDP, true, true, VEC>), g, blk, lds, st, p, hd);
   else if (causal)
-    hipLaunchKernelGGL((flash_generic_kernel<HDP, true, false, VEC>), g, blk, 0, st, p, hd);
+    hipLaunchKernelGGL((flash_generic_kernel<HDP, true, false, VEC>), g, blk, lds, st, p, hd);
   else if (km)
-    hipLaunchKernelGGL((flash_generic_kernel<HDP, false, true, VEC>), g, blk, 0, st, p, hd);
+    hipLaunchKernelGGL((flash_generic_kernel<HDP, false, true, VEC>), g, blk, lds, st, p, hd);
   else
-    hipLaunchKernelGGL((flash_generic_kernel<HDP, false, false, VEC>), g, blk, 0, st, p, hd);
+    hipLaunchKernelGGL((flash_generic_kernel<HDP, false, false, VEC>), g, blk, lds, st, p, hd);
   return check_launch("tk_flash_attn_fwd");
 }
 

@@ -22,13 +22,14 @@ SHAPES = {
     "tall_three_stages": (520, 2056, 192),   # 128 x 64, two K-tiles in flight
     "tall_two_stages": (777, 3080, 192),
     "mid_three_stages": (777, 3080, 2048),   # 128 x 128, 8 waves
-    "wide": (1500, 4104, 2048),              # 128 x 256
+    "mid_long_k": (1500, 4104, 2048),
     "tall_short_k": (1500, 3976, 192),
     "mid": (1500, 4104, 576),
     "two_stage_256": (4000, 2824, 576),      # 256 x 256, K an odd multiple of 64
-    "pingpong_one_round": (4001, 2312, 512),  # last tile row 161 rows, last column 8 columns
-    "pingpong_smallest": (4353, 2056, 512),  # one row and 8 columns past whole tiles
-    "pingpong_persistent": (8200, 2824, 512),
+    "pingpong_one_round": (4001, 3336, 512),  # last tile row 161 rows, last column 8 columns
+    "pingpong_smallest": (4353, 3080, 512),  # one row and 8 columns past whole tiles
+    "pingpong_persistent": (8200, 3592, 768),
+    "pingpong_short_k": (8200, 3592, 256),   # (residual epilogues: 128 x 128)
 }
 
 

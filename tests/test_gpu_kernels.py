@@ -154,19 +154,19 @@ def test_layernorm_model_widths_no_sum(cols):
 
 GEMM_SHAPES = [  # one or more per tile configuration of the dispatch, direct and K-tail paths
     (512, 384, 128),      # C1 QKV (reduced M): 64x64 tiles
-    (1024, 1536, 512),    # C2 QKV (reduced M)
-    (1024, 512, 2048),    # C2 FFN-down (reduced M)
-    (4096, 4096, 1024),   # 256x256 tiles
-    (8192, 4352, 384),    # 544 256x256 tiles: the persistent ping-pong kernel (bias, GELU and residual
+    (1024, 1536, 512),    # C2 QKV (reduced M): 128x64 tiles
+    (1024, 512, 2048),    # C2 FFN-down (reduced M): 32x64 tiles, four K groups
+    (4096, 4096, 1024),   # 256x256 ping-pong tiles, one round
+    (8192, 5888, 768),    # 736 256x256 tiles: the persistent ping-pong kernel (bias, GELU and residual
                           # epilogues; 2 or 3 tiles per workgroup, the next tile's first K-tile prefetched)
     (4096, 2048, 8192),   # C4 FFN-down (reduced M), long K: 128x128 tiles
-    (1000, 200, 72),      # ragged M, N, K
+    (1000, 200, 72),      # ragged M, N, K: operands through registers (K not a multiple of 64)
     (77, 300, 8),         # tiny K
     (130, 130, 136),
     (4000, 2100, 128),    # 128x128 tiles with M and N tails
-    (12800, 512, 2048),   # 256x128 tiles, three K stages
-    (13000, 500, 2056),   # 256x128 tiles, K tail, M and N tails
-    (4100, 4200, 1032),   # 256x256 tiles, K tail, M and N tails
+    (12800, 512, 2048),   # 128x128 tiles
+    (13000, 500, 2056),   # K tail, M and N tails, operands through registers
+    (4100, 4200, 1032),   # the same, 256x256 tiles
     (1, 384, 128),        # one row
     (300, 1, 64),         # one output column
     (200, 150, 100),      # K not a multiple of 8: element loads, zero fill past K
@@ -203,28 +203,30 @@ def test_gemm_residual_inplace(m, n, k):
     torch.testing.assert_close(out.cpu(), resid + ref, atol=5e-5, rtol=1e-5)
 
 
-# 256 x 256 tiles: launches of whole tiles (M, N multiples of 256, K of 128) run
-# the ping-pong K loop, others the two-stage loop (or 128 x 128 tiles); per
-# output element both accumulate the same MFMA k-steps in the same order, so
-# the first M rows of an (M + 8)-row launch equal the whole-tile launch bit for bit.
-@pytest.mark.parametrize("m,n,k", [(4096, 4096, 2048), (8192, 8192, 512), (8192, 2048, 4096)])
+# 256 x 256 tiles: launches whose output rows are 16-byte aligned run the ping-pong K
+# loop, others the two-stage loop; per output element both accumulate the same
+# MFMA k-steps in the same order, so the same product into a buffer one element off
+# equals it bit for bit.
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 2048), (8192, 8192, 768), (8192, 4096, 4096)])
 @pytest.mark.parametrize("epi", ["bias", "gelu", "resid"])
 def test_gemm_pingpong_matches_two_stage_loop(m, n, k, epi):
-    a, w, bias, ref = _gemm_inputs(m + 8, n, k, seed=31)
+    a, w, bias, ref = _gemm_inputs(m, n, k, seed=31)
     ag, wg, bg = a.to(DEV), w.to(DEV), bias.to(DEV)
     if epi == "resid":
-        resid = seeded(m + 8, n, seed=32).to(DEV)
-        whole = ops.linear_residual(ag[:m], wg, bg, resid[:m].contiguous())
-        ragged = ops.linear_residual(ag, wg, bg, resid)
+        resid = seeded(m, n, seed=32).to(DEV)
+        off = torch.empty(m, n + 1, device=DEV)[:, 1:]
+        pingpong = ops.linear_residual(ag, wg, bg, resid)
+        two_stage = ops.linear_residual(ag, wg, bg, resid, out=off)
         want = resid.cpu() + ref
         tol = dict(atol=5e-5, rtol=1e-5)
     else:
-        whole = ops.linear(ag[:m], wg, bg, gelu=epi == "gelu")
-        ragged = ops.linear(ag, wg, bg, gelu=epi == "gelu")
+        off = torch.empty(m, n + 1, dtype=torch.float16, device=DEV)[:, 1:]
+        pingpong = ops.linear(ag, wg, bg, gelu=epi == "gelu")
+        two_stage = ops.linear(ag, wg, bg, gelu=epi == "gelu", out=off)
         want = (ob.gelu_ref(ref) if epi == "gelu" else ref).half().float()
         tol = dict(atol=1e-3, rtol=1e-3)
-    assert torch.equal(whole, ragged[:m])
-    torch.testing.assert_close(ragged.cpu().float(), want, **tol)
+    assert torch.equal(pingpong, two_stage)
+    torch.testing.assert_close(pingpong.cpu().float(), want, **tol)
 
 
 @pytest.mark.parametrize("mode", ["keep", "zero"])
@@ -261,6 +263,10 @@ def test_gemm_add_layernorm_row_mask(mode):
     h = ops.linear_add_ln(a.to(DEV), w.to(DEV), bias.to(DEV), resid.to(DEV), lw.to(DEV), lb.to(DEV), 1e-5,
                           torch.float32, sum_out=sg, row_valid=valid.to(DEV), row_mode=code)
     torch.testing.assert_close(sg.cpu(), s_ref, atol=5e-5, rtol=1e-5)
+    torch.testing.assert_close(h.cpu(), h_ref, atol=1e-4, rtol=1e-4)
+    # without the sum: the full-row kernel
+    h = ops.linear_add_ln(a.to(DEV), w.to(DEV), bias.to(DEV), resid.to(DEV), lw.to(DEV), lb.to(DEV), 1e-5,
+                          torch.float32, row_valid=valid.to(DEV), row_mode=code)
     torch.testing.assert_close(h.cpu(), h_ref, atol=1e-4, rtol=1e-4)
 
 

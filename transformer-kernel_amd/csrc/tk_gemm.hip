@@ -11,7 +11,7 @@
 // vectors along the row.
 //
 // Block tile BM x BN (256x256 with 8 waves, 128x128 with 4 or 8, 128x64 with 8,
-// 64x64 with 4; gemm_dispatch picks), K-step BK with STAGES LDS buffers.  When K is a multiple of BK the K-tiles
+// 64x64 with 4, smaller in K groups; gemm_dispatch picks), K-step BK with STAGES LDS buffers.  When K is a multiple of BK the K-tiles
 // are copied global -> LDS with global_load_lds_dwordx4 (no register
 // staging), STAGES-1 tiles in flight, one vmcnt wait + barrier per K-step;
 // otherwise a register-staged path with zero fill handles the K tail.  LDS
@@ -19,8 +19,8 @@
 // the copies are bank-conflict free on gfx950's 64-bank LDS.  Block ids are
 // remapped so that the tiles of one XCD (workgroups are dealt round-robin
 // over the 8 XCDs) form a compact group of output tiles sharing A rows and
-// W rows in that XCD's L2.  256x256 tiles (M and N at least 256, K a multiple
-// of 128) run the ping-pong K loop instead (Mainloop::run_pingpong): the two
+// W rows in that XCD's L2.  256x256 tiles where they fill the chip (K a multiple of
+// 128; pingpong_pays) run the ping-pong K loop instead (Mainloop::run_pingpong): the two
 // waves of each SIMD alternate between a phase of LDS reads and copies and a
 // phase of MFMAs only, so one of them always feeds the matrix core.
 #include "tk_attn_tile.hpp"
@@ -1297,7 +1297,6 @@ using TileBig = Tile<256, 256, 4, 2, 64, 2>;   // 8 waves of 64 x 128
 using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop
 using TileMid = Tile<128, 128, 2, 2, 64, 2>;   // 4 waves of 64 x 64, 2 blocks per CU
 using TileMid3 = Tile<128, 128, 4, 2, 64, 3>;  // 8 waves of 32 x 64, 1 block per CU (96 KB LDS)
-using TileWide3 = Tile<128, 256, 2, 4, 64, 3>;  // 8 waves of 64 x 64, 1 block per CU (144 KB LDS)
 using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
 using TileTall3 = Tile<128, 64, 4, 2, 64, 3>;  // the same, two K-tiles in flight
 using TileSmall = Tile<64, 64, 2, 2, 64, 3>;   // 4 waves of 32 x 32, 3 blocks per CU
@@ -1321,11 +1320,37 @@ int launch_pingpong(const GemmArgs& p, int64_t tiles, hipStream_t st) {
   return launch_gemm<T, EPI, true>(p, st);
 }
 
-// Every figure: MI355X, us per launch, operands rotated through four buffers,
-// all tiles timed on 200 shapes (M 16 .. 30000, N 384 .. 6144, K 256 .. 4096,
-// the three epilogues).  Per accumulator the k order is the same for every
-// tile but the K-split ones, which one_order rules out: the choice then never
-// changes a result.
+// Every figure: MI355X, us per launch, operands rotated through two or four buffers,
+// all tiles and the dispatch before (256 x 256 and 128 x 128 tiles, one-wave 64 x 64
+// ones) timed in turn on 11392 shapes (M 300 .. 65536, N 256 .. 8192, K 256 .. 8192, the
+// four epilogues).  Per accumulator the k order is the same for every tile but the
+// K-split ones, which one_order rules out: the choice then never changes a result.
+
+// Whether the ping-pong loop on 256 x 256 tiles, one per CU and round, beats 128 x 128
+// tiles.  In several rounds the other takes as long as its CU with the most tiles, so each
+// ping-pong round is priced in 128 x 128 tiles: 2.6 to 4.1 of them, more at short K and with the
+// epilogues that keep the CU's one workgroup from its next tile (two rounds against 5 / 6 / 7
+// tiles, times the other's: bias K 512 1.06 / 0.95 / 0.86; residual K 1024 1.12 / 1.08 / 0.89,
+// K 512 1.17 / 1.12 / 0.99; with padded rows, K 512 1.10 / 1.07 / 0.93).  In one round the
+// share of the chip that it fills decides: at K 512 / 1024 GELU 0.62 1.12 / 1.00, 0.67 1.02 /
+// 0.95, 0.77 0.91 / 0.88, residual 0.52 1.06 / 0.96, 0.62 0.99 / 0.92; up to 512 tiles of
+// 128 x 128 are all resident, and it never does.
+template <int EPI>
+bool pingpong_pays(const GemmArgs& p, int64_t rounds, int64_t t128) {
+  constexpr bool kBias = EPI == TK_EPI_BIAS, kGelu = EPI == TK_EPI_BIAS_GELU;
+  if (p.K < (kBias || kGelu ? 256 : 512)) return false;  // residual, K 256, fill 0.92: 1.15 times the other
+  const double x = 512.0 / p.K;
+  if (rounds == 1) {
+    const double fill = (double)p.M * p.N / (65536.0 * 256.0);
+    return t128 > 512 && fill >= (kBias ? 0.46 + 0.12 * x : kGelu ? 0.46 + 0.31 * x : 0.44 + 0.16 * x);
+  }
+  const double round = kBias                   ? 0.64 + 0.055 * x
+                       : kGelu                 ? 0.67 + 0.07 * x
+                       : EPI == kEpiResidRows ? 0.712 + 0.1 * x
+                                               : 0.73 + 0.29 * x * x;
+  return 4.0 * round * (double)rounds <= (double)((t128 + 255) / 256);
+}
+
 template <int EPI>
 int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   const int64_t t256 = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
@@ -1340,17 +1365,12 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   const bool direct = p.K % 64 == 0 && p.kvec;
   // Ping-pong loop (256 x 256 tiles, K in pairs of 64, vector-aligned output
   // rows and bias; no row clamp, so M and N of at least a tile, edge tiles
-  // shifted, whose stores take 32-bit offsets).  Against the best two-stage
-  // tile: M4662 N3072 K1024 (fill 0.85) 33.8 vs 36.0, M4662 N2304 K768 (0.63)
-  // 25.1 vs 26.4, M3000 N3072 K1024 (0.55) 28.2 vs 31.0, M12000 N1024 K4096
-  // (0.73) 105 vs 125; at 0.5 and below it loses (M8192 N1024 K4096 92 vs 83).
-  // With two rounds it pays from two thirds (M4662 N6144 K2048, 0.85: 110 vs
-  // 126; M6000 N4096 K1024, 0.72: 65.5 vs 68.6; M6000 N3072 K1024, 0.55: 53.6
-  // vs 53.1).  Below K = 512 the smaller tiles are as fast.
+  // shifted, whose stores take 32-bit offsets): M43520 N768 K256 bias 41.2 on 128 x 128
+  // tiles -> 36.0, M46848 N1024 K256 GELU 64.0 -> 53.4, M7168 N3072 K1024 58.2 -> 55.9.
   const bool pp_fits = direct && p.K > 0 && p.K % 128 == 0 && p.vec && (p.bias == nullptr || p.bias16) &&
                        p.M >= 256 && p.N >= 256 && p.N % 8 == 0 && p.ldc < (1 << 19) && p.ldr < (1 << 19) &&
                        p.lda < (1 << 24) && p.ldw < (1 << 24);
-  if (pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.52 : 0.66)) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
+  if (pp_fits && pingpong_pays<EPI>(p, rounds, t128)) return launch_pingpong<TileBigPP, EPI>(p, t256, st);
   if (!direct) {  // register-staged operands
     const bool short_k = p.K <= 1024 && t256 <= 512;
     if (!short_k && t256 >= 256 && (t256 % 256 == 0 || t256 >= 512)) return launch_gemm<TileBig, EPI, false>(p, st);
@@ -1360,7 +1380,7 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   // Two-stage 256 x 256 tiles where the ping-pong loop cannot run (K an odd
   // multiple of 64): they win later than it does (M12000 N4096 K1024, fill
   // 0.98: 123.6 vs 133.6 on 128 x 128; M6000 N6144 K2048, 0.73: 171.6 vs 169.6).
-  if (p.K >= 512 && fill >= (rounds == 1 ? 0.62 : 0.8)) return launch_gemm<TileBig, EPI, true>(p, st);
+  if (!pp_fits && p.K >= 512 && fill >= (rounds == 1 ? 0.62 : 0.8)) return launch_gemm<TileBig, EPI, true>(p, st);
   // Up to one workgroup per CU the K loop is a chain of copy latencies: the
   // smallest tile that keeps every workgroup resident, more waves on each and
   // two K-tiles in flight.  From K = 768 the K loop is split over two or four
@@ -1390,13 +1410,13 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   // else two or three 128 x 64 tiles per CU, whose waves cover one another's
   // waits (M2048 N2048 K512 12.1 -> 11.1, M3000 N768 K768 13.4 -> 11.8).
   if (t128 <= 256) return p.K >= 2048 ? launch_gemm<TileMid3, EPI, true>(p, st) : launch_gemm<TileTall2, EPI, true>(p, st);
-  // Up to 512 of them: 128 x 256 tiles, one per CU, where a long K pays for
-  // the larger tile's epilogue (M16384 N512 K2048 54.0 -> 49.3, M6000 N1024
-  // K4096 75.8 -> 68.9); 128 x 64 ones where K is short and all are resident
-  // (M3000 N2048 K512 15.7 -> 14.8, M6000 N768 K256 10.0 -> 8.8; with more
-  // M16384 N512 K512 24.9 -> 27.6).  Everything else: 128 x 128.
-  if (t128 <= 512 && p.K >= 2048) return launch_gemm<TileWide3, EPI, true>(p, st);
-  if (tall <= 768 && p.K <= 512) return launch_gemm<TileTall2, EPI, true>(p, st);
+  // 128 x 64 ones also past that where K is short and all are resident, three to a CU, with room
+  // to spare (K 256 0.85 times 128 x 128, K 768 0.96; residual K 512 0.93, K 768 1.02; at 732 to
+  // 768 tiles 1.03 to 1.13, with more M16384 N512 K512 27.6 vs 24.9).  Everything else: 128 x 128.
+  // (128 x 256 tiles, one per CU, were 0.97 to 1.05 times those at K >= 2048, and 1.5 times
+  // where N's padding made more than 256 of them: M11312 N640 K2560 87.2 vs 54.3.)
+  constexpr bool kResid = EPI == TK_EPI_BIAS_RESID || EPI == kEpiResidRows;
+  if (tall <= (kResid ? 640 : 704) && p.K <= (kResid ? 512 : 768)) return launch_gemm<TileTall2, EPI, true>(p, st);
   return launch_gemm<TileMid, EPI, true>(p, st);
 }
 

@@ -53,3 +53,20 @@ def test_bad_calls_are_refused():
     assert lib.tk_small_pack(16, 16, 16, 16, 16, 0, None) == _lib.TK_ERR_ARG
     args = [16, 16, 1, 32, 4, 32, 1, 1, None] + [16] * 10 + [1e-5, 1e-5, 1e-5, 1.0, None]
     assert lib.tk_small_forward_packed(*args) == _lib.TK_ERR_ARG
+
+
+@pytest.mark.gpu
+def test_layers_share_the_whole_forward_fragments():
+    """Width 128 with ffn_dim 128: what the narrow kernels are given of the stacked fragments is the
+    fragment order of that layer's own weights (as the ffn_dim-256 model packs them one by one)."""
+    torch.manual_seed(83)
+    model = tkmi.OptimizedTransformer(tkmi.TransformerConfig(2, 200, 128, 4, 128, 3, True)).to(DEV).eval()
+    built, native = model._weights(), model._native_model()
+    packed = model._stacked["packed"]
+    for i, lw in enumerate(built):
+        for name in ("w_qkv", "w_o", "w_1", "w_2"):
+            w = getattr(lw, name)
+            assert torch.equal(model._stacked[name][i], w)
+            at = (getattr(native.layers[i], name + "_packed") - packed.data_ptr()) // 2
+            want = w.view(-1, 32, 8, 2, 8).permute(0, 2, 3, 1, 4)  # block, fragment, half, row, 8 columns
+            assert torch.equal(packed[at:at + w.numel()], want.flatten())

@@ -117,7 +117,8 @@ class _LayerWeights:
     b_1: torch.Tensor
     w_2: torch.Tensor  # [D, F]
     b_2: torch.Tensor
-    # The same in the narrow kernels' fragment order (width 128 only, else None).
+    # The same in the narrow kernels' fragment order (width 128 only, else None; with ffn_dim
+    # 128 they are parts of the whole-forward kernel's, OptimizedTransformer._stacked).
     w_qkv_packed: Optional[torch.Tensor] = None
     w_o_packed: Optional[torch.Tensor] = None
     w_1_packed: Optional[torch.Tensor] = None
@@ -129,6 +130,8 @@ def _fragments(w: torch.Tensor) -> torch.Tensor:
     n, k = w.shape
     return w.view(n // 32, 32, k // 128, 8, 2, 8).permute(2, 0, 3, 4, 1, 5).contiguous()
 
+
+_BLOCK_BYTES = 32 * 128 * 2  # 32 rows by 128 columns of a packed weight
 
 # Input dtypes that tk_forward takes, and returns, as they are.
 _IO_FLAGS = {torch.float16: TK_FWD_IO_F16, torch.bfloat16: TK_FWD_IO_BF16}
@@ -246,13 +249,16 @@ class OptimizedTransformer(BaselineTransformer):
                 for n in names:
                     setattr(lw, n + "_packed", _fragments(getattr(lw, n)))
             return None
-        stacked = {n: torch.stack([getattr(lw, n) for lw in built]).contiguous()
-                   for n in names + ("b_qkv", "b_o", "b_1", "b_2", "n1_w", "n1_b", "n2_w", "n2_b")}
+        # One copy per dtype: all layers' tensors of a name are a slice of it, in layer order.
+        stacked = {}
+        for group in (names, ("b_qkv", "b_o", "b_1", "b_2", "n1_w", "n1_b", "n2_w", "n2_b")):
+            flat = torch.cat([getattr(lw, n).reshape(-1) for n in group for lw in built])
+            at = 0
+            for n in group:
+                t = getattr(built[0], n)
+                stacked[n] = flat[at:at + len(built) * t.numel()].view(len(built), *t.shape)
+                at += len(built) * t.numel()
         stacked["packed"] = ops.small_pack(stacked)
-        # a layer's 12 + 4 + 4 + 4 blocks of 32 rows by 128 columns, in the order of `names`
-        for lw, blocks in zip(built, stacked["packed"].view(len(built), 24, -1)):
-            for n, part in zip(names, blocks.split((12, 4, 4, 4))):
-                setattr(lw, n + "_packed", part)
         return stacked
 
     def _native_model(self) -> _lib.Model:
@@ -264,18 +270,23 @@ class OptimizedTransformer(BaselineTransformer):
         now = (bool(self.config.causal), float(self.attn_scale))
         native = self._native
         if native is None or native.made_for != now:
+            stacked = self._stacked
             layers = (_lib.Layer * len(built))()
-            for dst, lw in zip(layers, built):
+            for i, (dst, lw) in enumerate(zip(layers, built)):
                 for name, _ in _lib.Layer._fields_:
                     val = getattr(lw, name)
                     setattr(dst, name, val.data_ptr() if isinstance(val, torch.Tensor) else val)
+                if stacked is not None:  # a layer's 12 + 4 + 4 + 4 blocks of 32 rows by 128 columns
+                    at = stacked["packed"].data_ptr() + i * 24 * _BLOCK_BYTES
+                    dst.w_qkv_packed, dst.w_o_packed = at, at + 12 * _BLOCK_BYTES
+                    dst.w_1_packed, dst.w_2_packed = at + 16 * _BLOCK_BYTES, at + 20 * _BLOCK_BYTES
             nf_w, nf_b, nf_eps = self._final
             native = _lib.Model(
                 d_model=self.d_model, heads=self.num_heads, head_dim=self.head_dim_padded,
                 ffn_dim=self.config.ffn_dim, num_layers=len(built), layers=layers, nf_w=nf_w.data_ptr(),
                 nf_b=nf_b.data_ptr(), nf_eps=nf_eps, scale=now[1], causal=int(now[0]))
             native.made_for = now
-            native.tensors = (built, self._final)
+            native.tensors = (built, stacked, self._final)
             self._native = native
         return native
 

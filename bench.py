@@ -107,8 +107,9 @@ def kernel_units(name: str, cfg) -> dict:
         return {"flop": 2.0 * m * n * k, "byte": 2.0 * (m * k + n * k) + 4.0 * n + float(ob) * m * n}
     if name == "ln_qkv":  # LayerNorm + QKV: fp32 x in, fp16 q|k|v out
         return {"flop": 2.0 * t * 3 * d * d, "byte": 10.0 * t * d + 2.0 * 3 * d * d}
-    if name == "block_tail":  # out-projection, FFN and both LayerNorms: ctx and x in, y out
-        return {"flop": 2.0 * t * (d * d + 2 * d * f), "byte": 10.0 * t * d + 2.0 * (d * d + 2 * d * f)}
+    if name == "block_tail":  # out-projection, FFN and both LayerNorms: ctx and x in; fp16 h and the sum out, last fp32 y
+        return {"flop": 2.0 * t * (d * d + 2 * d * f),
+                "byte": (12.0 - 2.0 / nl) * t * d + 2.0 * (d * d + 2 * d * f)}  # mean over the layers
     if name == "small_forward":  # the whole forward (every layer) in one launch
         per_layer = 2.0 * t * (3 * d * d + d * d + 2 * d * f) + 4.0 * b * d * pairs
         return {"flop": per_layer * nl}

@@ -258,6 +258,17 @@ def test_hot_kernels_use_no_scratch():
 
 # ---------------------------------------------------------------- tooling --
 
+def test_bench_block_tail_bytes():
+    """tk_narrow_tail reads ctx (2) and the residual (4) and writes fp32 y (4) in the last layer, the
+    sum (4) and fp16 h (2) in the others, per element: the mean over the layers, beside the weights."""
+    import bench
+
+    t, d, f = 4 * 200, 128, 256
+    weights = 2.0 * (d * d + 2 * d * f)
+    for layers, per in ((1, 10.0), (2, 11.0), (4, 11.5)):
+        assert bench.kernel_units("block_tail", (4, 200, d, 4, f, layers, True))["byte"] == per * t * d + weights
+
+
 def test_bench_parse_shape():
     import bench
 

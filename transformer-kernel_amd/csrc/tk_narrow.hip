@@ -7,9 +7,10 @@
 // At this width a block is bound by its rows' trips through HBM: launched
 // separately (LayerNorm, QKV, out-projection + LayerNorm, FFN-up, FFN-down +
 // LayerNorm) each of a row's 128 columns moves 44 bytes beside attention's, most
-// of them an intermediate written by one launch and read by the next.  Fused it
-// moves 4 + 6 (q|k|v) and 2 + 4 + 4 bytes.  65536 rows, F = 128: LN + QKV 32.5 ->
-// 19.8 us (4.2 TB/s), the rest 69.8 -> 25.2 us (3.3 TB/s; bound by its chain of
+// of them an intermediate written by one launch and read by the next.  Fused, a
+// one-layer model's moves 4 + 6 (q|k|v) and 2 + 4 + 4 bytes (a layer before the last: 2 + 4 in,
+// the sum 4 and h 2 out).  65536 rows, F = 128, one layer: LN + QKV 32.5 -> 19.8 us
+// (4.2 TB/s), the rest 69.8 -> 25.2 us (3.3 TB/s; bound by its chain of
 // hand-overs between the waves, two workgroups per CU).
 //
 // A workgroup of four waves takes 64 rows at a time.  As in the whole-forward

@@ -248,6 +248,11 @@ def test_hot_kernels_use_no_scratch():
     # head dims 16, 32, 64, 128: causal and not, and causal split (C1's listed above)
     assert len(small) == 11
     hot += small
+    # the same on weights in fragment order, and the blocks of width 128
+    packed = [k for k in usage if "small_packed_kernel" in k]
+    narrow = [k for k in usage if "narrow_qkv_kernel" in k or "narrow_tail_kernel" in k]
+    assert len(packed) == 12 and len(narrow) == 5
+    hot += packed + narrow
     missing = [k for k in hot if k not in usage]
     assert not missing, missing
     # the 256 x 256 ping-pong GEMM instantiations (direct path, every epilogue)

@@ -3,7 +3,7 @@
 // Per workgroup: BM = 32*NW query rows of one (batch, head), one wave per 32
 // rows, key/value tiles of 64 keys in LDS.
 //
-// Transposed formulation (both kernel bodies).  Each wave computes
+// Transposed formulation (every body).  Each wave computes
 // S^T = K . Q^T with v_mfma_f32_32x32x16_f16 (A operand = K rows from LDS,
 // B operand = the wave's Q rows, held in registers for the whole kernel).
 // In the 32x32 accumulator layout a lane then holds 16 keys of ONE query row
@@ -14,20 +14,20 @@
 //     directly the B operand of O^T = V^T . P^T; those 8 entries stand for
 //     the keys {16t + 8*e2 + 4g + e10} (g = lane >> 5).
 //
-// Two bodies, picked by head_dim at compile time:
+// Bodies, picked by head_dim, causality and length (dispatch_flash; few query blocks take
+// the key-split kernel, head_dim 256 and odd views flash_generic_kernel):
 //   flash_dma_body (head_dim <= 64): K and V tiles copied global -> LDS
 //     directly (global_load_lds_dwordx4, row-major); the V^T operand is two
 //     ds_read_b64_tr_b16 of the row-major V tile.  The O^T MFMAs of tile t-1
 //     are deferred into step t, so every MFMA of a step is independent of
 //     the step's exponentials and interleaves with them; the row max of the
 //     next tile is computed in the same pass.
-//   flash_vreg_body (head_dim 128): the deferred P needs 16 more registers
-//     than two waves per SIMD leave at head_dim 128, so tile t's O^T MFMAs
+//   flash_pair_body (head_dim 128 past 128 keys) and flash_ring_body (causal up
+//     to 128): K and V through LDS-DMA rings, P.V deferred one step.
+//   flash_vreg_body (head_dim 128 without the causal mask: up to 128 keys, or V
+//     rows that are 8-byte vectors only, which no DMA copies): tile t's O^T MFMAs
 //     follow its exponentials; V^T is written to LDS from registers with
 //     key bits 2 and 3 swapped so that each A operand is one 16-byte read.
-//   Measured on MI355X (C5 shape, head_dim 64): the DMA body 5.6-5.8 ms
-//   against 6.2-6.3 ms for the register body; at head_dim 128 (C4 shape)
-//   the register body 1.48 ms against 1.70 ms.
 //
 // Numerics (src/kernels.py:112-134, src/torch_transformer_benchmark.py:97-111):
 // fp32 scores, the scale applied in fp32 after Q.K^T (folded with log2(e)
@@ -1960,12 +1960,12 @@ int launch_generic(const AttnArgs& args, int hd, bool causal, hipStream_t st) {
 // causal 129 -> 118 us, b2 s32768 causal 5.81 -> 5.73 ms).
 template <int HD, int NW, bool CAUSAL, bool KMASK>
 __global__ __launch_bounds__(NW * 64, (NW <= 4 && HD <= 64) ? 2 : 1) void flash_fwd_kernel(AttnArgs p) {
-  // head_dim 128: causal launches take the DMA-ring body (C4 shape b4 s8192:
-  // 1263-1295 -> 1180-1199 us in alternating same-box runs); without the
-  // causal diagonal the register body stays (its ring build spills ~100 B
-  // there: b2 s4096 non-causal 318-340 vs 354 us).
+  // head_dim 128, causal: the pair body (C4 shape b4 s8192: register body 1263-1295, ring
+  // 1180-1199 us and, another day, ring 1268-1300, pair 1225-1263), up to 128 keys the ring.
+  // Without the causal mask this kernel keeps the register body (what flash_full_kernel
+  // does not take).
   if constexpr (HD == 128 && CAUSAL && NW == 8) {
-    flash_pair_body<HD, NW, CAUSAL, KMASK>(p);  // C4 b4 s8192: 1268-1300 -> 1225-1263 us against the ring body
+    flash_pair_body<HD, NW, CAUSAL, KMASK>(p);
   } else if constexpr (HD == 128 && CAUSAL) {
     flash_ring_body<HD, NW, CAUSAL, KMASK>(p);
   } else if constexpr (HD == 128) {

@@ -23,6 +23,8 @@ SHAPES = {
     "tall_two_stages": (777, 3080, 192),
     "mid_three_stages": (777, 3080, 2048),   # 128 x 128, 8 waves
     "mid_long_k": (1500, 4104, 2048),
+    "wide_one_to_a_row": (20993, 256, 2048),  # 128 x 256, last tile row one row
+    "wide_two_to_a_row": (14493, 512, 2048),
     "tall_short_k": (1500, 3976, 192),
     "mid": (1500, 4104, 576),
     "two_stage_256": (4000, 2824, 576),      # 256 x 256, K an odd multiple of 64

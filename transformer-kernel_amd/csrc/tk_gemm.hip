@@ -10,7 +10,7 @@
 // and LayerNorm epilogues then work on 16-byte (fp32) / 8-byte (fp16)
 // vectors along the row.
 //
-// Block tile BM x BN (256x256 with 8 waves, 128x128 with 4 or 8, 128x64 with 8,
+// Block tile BM x BN (256x256 with 8 waves, 128x256 with 8, 128x128 with 4 or 8, 128x64 with 8,
 // 64x64 with 4, smaller in K groups; gemm_dispatch picks), K-step BK with STAGES LDS buffers.  When K is a multiple of BK the K-tiles
 // are copied global -> LDS with global_load_lds_dwordx4 (no register
 // staging), STAGES-1 tiles in flight, one vmcnt wait + barrier per K-step;
@@ -1297,6 +1297,7 @@ using TileBig = Tile<256, 256, 4, 2, 64, 2>;   // 8 waves of 64 x 128
 using TileBigPP = Tile<256, 256, 4, 2, 64, 2, true>;  // the same, ping-pong K loop
 using TileMid = Tile<128, 128, 2, 2, 64, 2>;   // 4 waves of 64 x 64, 2 blocks per CU
 using TileMid3 = Tile<128, 128, 4, 2, 64, 3>;  // 8 waves of 32 x 64, 1 block per CU (96 KB LDS)
+using TileWide3 = Tile<128, 256, 2, 4, 64, 3>;  // 8 waves of 64 x 64, 1 block per CU (144 KB LDS)
 using TileTall2 = Tile<128, 64, 4, 2, 64, 2>;  // 8 waves of 32 x 32, 3 blocks per CU
 using TileTall3 = Tile<128, 64, 4, 2, 64, 3>;  // the same, two K-tiles in flight
 using TileSmall = Tile<64, 64, 2, 2, 64, 3>;   // 4 waves of 32 x 32, 3 blocks per CU
@@ -1410,13 +1411,19 @@ int gemm_dispatch(const GemmArgs& p, hipStream_t st) {
   // else two or three 128 x 64 tiles per CU, whose waves cover one another's
   // waits (M2048 N2048 K512 12.1 -> 11.1, M3000 N768 K768 13.4 -> 11.8).
   if (t128 <= 256) return p.K >= 2048 ? launch_gemm<TileMid3, EPI, true>(p, st) : launch_gemm<TileTall2, EPI, true>(p, st);
-  // 128 x 64 ones also past that where K is short and all are resident, three to a CU, with room
-  // to spare (K 256 0.85 times 128 x 128, K 768 0.96; residual K 512 0.93, K 768 1.02; at 732 to
-  // 768 tiles 1.03 to 1.13, with more M16384 N512 K512 27.6 vs 24.9).  Everything else: 128 x 128.
-  // (128 x 256 tiles, one per CU, were 0.97 to 1.05 times those at K >= 2048, and 1.5 times
-  // where N's padding made more than 256 of them: M11312 N640 K2560 87.2 vs 54.3.)
-  constexpr bool kResid = EPI == TK_EPI_BIAS_RESID || EPI == kEpiResidRows;
-  if (tall <= (kResid ? 640 : 704) && p.K <= (kResid ? 512 : 768)) return launch_gemm<TileTall2, EPI, true>(p, st);
+  // 128 x 64 ones also past that where K is short and all are resident, three to a CU: up to
+  // 768 tiles at K 256 0.86 to 0.90 times 128 x 128, K 768 0.94 to 0.97; residual K 512 0.93 to
+  // 0.98, K 640 and 768 0.95 to 1.05, with padded rows K 256 0.80 to 0.85, K 768 0.86 to 0.96
+  // (past them M16384 N512 K512 27.6 vs 24.9).
+  if (tall <= 768 && p.K <= (EPI == TK_EPI_BIAS_RESID ? 512 : 768)) return launch_gemm<TileTall2, EPI, true>(p, st);
+  // 128 x 256 ones, one per CU, where one or two of them span N and 128 x 128 tiles would be
+  // more than 40 or 56 per XCD: 0.81 to 0.93 times those at K 2048 and 4096, 0.87 to 0.98 at
+  // K 1024 (GELU, two to a row, 1.00 to 1.02); M16384 N512 K2048 residual in a block's forward
+  // 51.4 -> 48.9.  With fewer 0.94 to 1.04, at other N 0.99 to 1.05, and where they pad N
+  // M11312 N640 K2560 87.2 vs 54.3.  Everything else: 128 x 128.
+  if ((p.N == 256 || p.N == 512) && t128 <= 512 && t128 > (p.N == 256 ? 320 : 448) &&
+      p.K >= (EPI == TK_EPI_BIAS_GELU ? 2048 : 1024))
+    return launch_gemm<TileWide3, EPI, true>(p, st);
   return launch_gemm<TileMid, EPI, true>(p, st);
 }
 

@@ -102,14 +102,32 @@ def test_batch_invariant_model():
 
 
 # Two workgroups per CU: one key tile too few, B*H off the XCD count, and the first inside each line.
-@pytest.mark.parametrize("b,s,hd,causal,split", [
-    (128, 128, 128, True, False), (128, 127, 128, False, False), (128, 128, 128, False, True),
-    (80, 160, 128, True, True), (72, 192, 256, False, False), (64, 256, 256, False, True),
-    (85, 192, 64, False, False), (80, 192, 64, False, True), (19, 512, 64, False, True), (170, 192, 32, True, False)])
-def test_rule_past_one_workgroup_per_cu(b, s, hd, causal, split):
+@pytest.mark.parametrize("b,s,hd,causal,masked,split", [
+    (128, 128, 128, True, False, False), (128, 128, 128, True, True, True), (170, 96, 128, False, True, False),
+    (128, 96, 128, False, False, False), (128, 97, 128, False, False, True), (80, 160, 128, True, False, True),
+    (72, 192, 256, False, False, False), (64, 256, 256, False, False, True), (43, 320, 256, False, True, False),
+    (72, 192, 256, True, False, False), (73, 193, 256, True, False, True),
+    (85, 192, 64, False, False, False), (85, 192, 64, False, True, True), (80, 192, 64, False, False, True),
+    (52, 256, 64, True, False, True), (19, 512, 64, False, False, True),
+    (170, 192, 32, True, False, False), (170, 192, 32, True, True, True), (168, 192, 32, True, False, True),
+    (122, 96, 32, False, False, False)])
+def test_rule_past_one_workgroup_per_cu(b, s, hd, causal, masked, split):
     q, k, v = (t.to(DEV) for t in _qkv(b, 1, s, hd, seed=s + hd))
-    out = ops.flash_attention(q, k, v, hd ** -0.5, causal)
-    assert torch.equal(out, ops.flash_attention(q, k, v, hd ** -0.5, causal, batch_invariant=True)) != split
+    valid = None
+    if masked:
+        valid = torch.arange(s, device=DEV)[None] < torch.linspace(s - 40, s, b, device=DEV).long()[:, None]
+    out = ops.flash_attention(q, k, v, hd ** -0.5, causal, key_valid=valid)
+    other = ops.flash_attention(q, k, v, hd ** -0.5, causal, key_valid=valid, batch_invariant=True)
+    assert torch.equal(out, other) != split
     few = slice(0, 4)
-    bad, err = or_rule_violations(out[few], ob.attention_ref(q[few].cpu(), k[few].cpu(), v[few].cpu(), hd ** -0.5, causal))
+    qf, kf, vf = (t[few].cpu().float() for t in (q, k, v))
+    if not masked:
+        ref = ob.attention_ref(qf, kf, vf, hd ** -0.5, causal)
+    else:
+        gone = ~valid[few].cpu()[:, None, None, :].expand(4, 1, s, s).clone()
+        if causal:
+            gone |= torch.ones(s, s, dtype=torch.bool).triu(1)
+        scores = torch.matmul(qf, kf.transpose(-2, -1).contiguous()) * hd ** -0.5
+        ref = torch.matmul(scores.masked_fill(gone, float("-inf")).softmax(-1), vf)[:, 0]
+    bad, err = or_rule_violations(out[few], ref)
     assert bad == 0, err

@@ -2029,23 +2029,39 @@ __global__ __launch_bounds__(NW * 64, HD <= 64 ? 2 : 1) void flash_keysplit_kern
 // Up to one per CU it wins at every length: b1 h16 s512 causal, head_dim 64 10.1 -> 5.7,
 // 128 23.8 -> 8.9, 32 8.6 -> 4.7, 256 38.0 -> 16.9; b1 h4 s2048 23.1 -> 11.0 (eight waves:
 // past 1024 keys, one workgroup per CU; b1 h1 s4096 22.7 -> 17.7, b1 h16 s512 5.7 vs 5.9).
-// Up to two per CU (1024 workgroups at head_dim 32 causal) its 32-row blocks read K and V
-// from L2 twice as often, which pays where a head's blocks share an XCD (ids are dealt
-// round-robin over 8: B*H a multiple of 8) or the sequence is long: b64 h1 s256 head_dim
-// 64 full 7.0 -> 5.8, but b51 h1 s256 7.3 -> 7.5, b85 h1 s192 6.5 -> 7.5; b1 h16 s1024
-// full 14.1 -> 11.8, 128 31.6 -> 25.3.  At head_dim 128 and 256 a CU holds one workgroup,
-// so there are two rounds, which only longer chains repay: 128, b170 h1 s65 causal 8.5 vs
-// 10.8, b128 h1 s128 causal 10.1 vs 11.1, full 10.8 -> 10.0; 256 full, s192 1.08
-// times the other, s256 0.95.  At 1024 the larger query tiles win (b4 h16 s512 11.6 vs
-// 12.6, b1 h16 s2048 full 26.1 vs 35.5) except for head_dim 32 causal (b1 h16 s2048 24.5
-// -> 18.3, b64 h4 s128 6.6 -> 6.4).
+// Up to two per CU (four at head_dim 32 causal) its 32-row blocks read K and V from L2 two or
+// four times as often.  That is cheap where a head's blocks share an XCD (ids are dealt
+// round-robin over 8), dear where B*H is odd and every XCD reads every head, and always repaid
+// by long chains.  Times the others' (50000 launches, 257 blocks on), medians: causal, 64 0.62 to
+// 0.94, 128 past 128 keys 0.43 to 0.91, 256 0.39 to 0.97 but 129 to 192 keys 0.98 to 1.09 past 384
+// blocks, 32 0.43 to 0.95, past 512 blocks 0.96 to 1.13 at 97 to 384 keys unless B*H is a
+// multiple of 8 (0.7 to 0.95).  128 up to 128 keys: causal 1.09 to 1.23, full 1.03 to 1.12, from 97
+// on with B*H a multiple of 8 0.95; 256 full up to 192 keys 1.04 to 1.27.  Full with B*H a
+// multiple of 4 0.68 to 0.98; with an even one 0.77 to 1.0; odd ones at 449 to 512 blocks
+// and 129 to 384 keys 1.00 to 1.05, 256 1.20.  A key mask, which costs the others a second
+// pass over each score, moves all but 256: causal 0.57 to 0.91 everywhere, 128 up to 128 keys too
+// (0.69 to 0.73), full past 128 keys 0.80 to 0.99.  b26 h2 s256 d64 causal masked 12.5 -> 6.6 us.
 int64_t keysplit_blocks(int64_t bh, int64_t s) { return bh * ((s + 31) / 32); }
-bool keysplit_pays(int64_t bh, int64_t s, int64_t hd, bool causal) {
+// The most workgroups that it is taken for.
+int64_t keysplit_limit(int64_t bh, int64_t s, int64_t hd, bool causal, bool masked) {
+  if (causal) {
+    if (hd == 128) return s > 128 || masked ? 512 : 256;
+    if (hd == 256) return s > 128 && s <= 192 ? 384 : 512;
+    if (hd == 64) return 512;
+    return masked || bh % 8 == 0 || s > 384 || s <= 96 ? 1024 : s > 192 ? 768 : 512;
+  }
+  if (s > (hd <= 64 ? 384 : 768)) return 512;
+  if (hd == 128 && s <= (bh % 8 == 0 ? 96 : 128)) return 256;
+  if (hd == 256 && s <= 192) return 256;
+  if (bh % 4 == 0 || (masked && hd <= 128 && s > 128)) return 512;
+  if (hd == 256 && s <= 384) return 256;
+  if (hd <= 64 && s <= 128) return 320;
+  return bh % 2 == 0 ? 512 : hd == 256 ? 384 : 416;
+}
+bool keysplit_pays(int64_t bh, int64_t s, int64_t hd, bool causal, bool masked) {
   if ((hd != 32 && hd != 64 && hd != 128 && hd != 256) || s <= 64) return false;
   const int64_t blocks = keysplit_blocks(bh, s);
-  if (blocks <= 256) return true;
-  if (blocks > (hd == 32 && causal ? 1024 : 512) || (bh % 8 != 0 && s < 512)) return false;
-  return hd <= 64 || (hd == 128 ? s > (causal ? 128 : 127) : causal || s >= 256);
+  return blocks <= 256 || blocks <= keysplit_limit(bh, s, hd, causal, masked);
 }
 template <int HD, int NW>
 int launch_keysplit(const AttnArgs& p, bool causal, hipStream_t st) {
@@ -2167,7 +2183,7 @@ int tk::flash_attn(const tk_half* q, const tk_half* k, const tk_half* v, tk_half
           o_strides[i] % 4 == 0;
   if (vec) {
     const bool v16 = al(v, 16) && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0 && v_strides[2] % 8 == 0;
-    if (v16 && !batch_invariant && keysplit_pays(batch * heads, seq, head_dim, c)) {
+    if (v16 && !batch_invariant && keysplit_pays(batch * heads, seq, head_dim, c, p.kv != nullptr)) {
       const bool w8 = keysplit_blocks(batch * heads, seq) <= 256 && seq > 1024;
       if (head_dim == 32) return w8 ? launch_keysplit<32, 8>(p, c, st) : launch_keysplit<32, 4>(p, c, st);
       if (head_dim == 64) return w8 ? launch_keysplit<64, 8>(p, c, st) : launch_keysplit<64, 4>(p, c, st);

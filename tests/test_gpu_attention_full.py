@@ -107,12 +107,12 @@ def test_eight_byte_value_rows_keep_their_path():
 
 
 @pytest.mark.parametrize("hd", [16, 32, 64, 128, 256, 80])
-@pytest.mark.parametrize("s", [320, 321])
+@pytest.mark.parametrize("s", [85, 86, 170, 171, 192, 193, 321])
 def test_tail_skipping_around_its_line(s, hd):
-    """Key masks at the longest length without the scan for the last valid key and the shortest
-    with it, in launches of as many workgroups as CUs and of more (the scan's other condition);
+    """Key masks at lengths with the scan for the last valid key and their neighbours without it,
+    in launches of up to as many workgroups as CUs and of more (the scan's other condition);
     batch_invariant launches take it at every batch, with the same bits."""
-    h = 64
+    h = 96
     valid = torch.ones(3, s, dtype=torch.bool)
     valid[0, 1:] = False
     valid[1, 200:] = False

@@ -95,15 +95,17 @@ __device__ __forceinline__ int valid_tiles(const AttnArgs& p, const uint8_t* kvb
 }
 
 // Where it is asked for: the scan is a load latency ahead of everything else in a
-// workgroup, 0.2 to 0.4 us.  Up to five key tiles that is as much as a dropped tile gives (lengths
-// from 70 %: head_dim 32 b20 h16 s176 14.1 -> 14.9 us, 16 b7 h12 s320 9.7 -> 9.9, 128 b44
-// h16 s128 34.9 -> 36.7; from six on 64 b20 h12 s480 63.5 -> 52.5), and where every workgroup
-// has a CU the longest sequence sets the time (16 b3 h1 s640 14.3 -> 14.6).  (The scan
-// decides which steps the head_dim-64 loop covers, whose row sums round otherwise than the
-// compiled ones: one_order launches don't look at the number of blocks.)
-constexpr int kTrimFrom = 320;
+// workgroup, 0.2 to 0.4 us, which pays where sequences end before the last key tile: not with 86
+// to 128 and 171 to 192 keys, whose last tile holds more than a quarter of them
+// (lengths from 70 %: head_dim 32 b20 h16 s176 14.1 -> 14.9 us, 128 b44 h16 s128 34.9 ->
+// 36.7; the others 256 b300 h2 s65 41.4 -> 30.7, 64 b118 h12 s206 66.0 -> 60.5, 64 b20 h12 s480
+// 63.5 -> 52.5), and not where every workgroup has a CU, since the longest sequence sets the
+// time there (16 b3 h1 s640 14.3 -> 14.6).  (The scan decides which steps the head_dim-64 loop
+// covers, whose row sums round otherwise than the compiled ones: one_order launches don't
+// look at the number of blocks.)
 AttnArgs trimmed(AttnArgs p, bool causal, int64_t blocks) {
-  p.trim = p.kv != nullptr && !causal && p.S > kTrimFrom && (blocks > 256 || p.one_order);
+  const bool ends_early = p.S > kBN && 4 * ((p.S - 1) % kBN + 1) <= p.S;
+  p.trim = p.kv != nullptr && !causal && ends_early && (blocks > 256 || p.one_order);
   return p;
 }
 
@@ -597,7 +599,7 @@ __device__ __forceinline__ void flash_dma_body(const AttnArgs& p) {
   }
 }
 
-template <int HD, int NW, bool CAUSAL, bool KMASK>
+template <int HD, int NW, bool CAUSAL, bool KMASK, bool TRIM>
 __device__ __forceinline__ void flash_vreg_body(const AttnArgs& p) {
   constexpr int BM = 32 * NW;
   constexpr int NT = NW * 64;
@@ -659,7 +661,7 @@ __device__ __forceinline__ void flash_vreg_body(const AttnArgs& p) {
   float l_run = 0.f;        // lane-partial running sum (this lane's keys)
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = (kv_end + kBN - 1) / kBN;  // (no valid_tiles: S <= 128, or V rows that nothing copies)
+  const int n_kt = valid_tiles<KMASK && !CAUSAL && TRIM>(p, kvb, (kv_end + kBN - 1) / kBN);
 
   // ---- K tile: direct copies; per-lane source offsets fixed, tile stride added ----
   int k_src_row[K_CPW], k_src_col[K_CPW];
@@ -1723,8 +1725,8 @@ __device__ __forceinline__ void flash_single_body(const AttnArgs& p) {
 // Waves per SIMD: at HDP 64 and 128 three and two, which keep the accumulators in VGPRs (an
 // AGPR move for each costs one wave per SIMD here): b60 h2 s700 d80 causal 137 -> 100 us, full 201 ->
 // 150, b1 h2 s1500 d80 132 -> 124, b300 h2 s300 d40 80 -> 67.
-template <int HDP, bool CAUSAL, bool KMASK, bool VEC>
-__global__ __launch_bounds__(256, HDP == 128 ? 2 : HDP == 64 ? 3 : 1) void flash_generic_kernel(AttnArgs p, int hd) {
+template <int HDP, bool CAUSAL, bool KMASK, bool VEC, bool TRIM = VEC>
+__global__ __launch_bounds__(256, HDP == 128 ? 2 : HDP == 64 ? 3 : HDP <= 32 ? 4 : 0) void flash_generic_kernel(AttnArgs p, int hd) {
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
   constexpr int RB = HDP * 2;              // K / V tile row bytes
   constexpr int CPR = RB / 16;             // 16-byte chunks per row
@@ -1790,7 +1792,7 @@ __global__ __launch_bounds__(256, HDP == 128 ? 2 : HDP == 64 ? 3 : 1) void flash
   const bool d_ok = HDP % 32 == 0 || (lane & 31) < HDP;
 
   const int kv_end = CAUSAL ? min(p.S, q0 + BM) : p.S;
-  const int n_kt = valid_tiles<KMASK && !CAUSAL && VEC>(p, kvb, (kv_end + kBN - 1) / kBN);
+  const int n_kt = valid_tiles<KMASK && !CAUSAL && TRIM>(p, kvb, (kv_end + kBN - 1) / kBN);
   // VEC: one K and one V slot, filled by direct copies, 1 KB per wave and copy; the
   // next K tile is on its way from the moment that every wave has this one's
   // fragments, the next V tile from the end of P.V, so each crosses the other
@@ -1944,6 +1946,8 @@ int launch_generic(const AttnArgs& args, int hd, bool causal, hipStream_t st) {
     hipLaunchKernelGGL((flash_generic_kernel<HDP, true, true, VEC>), g, blk, lds, st, p, hd);
   else if (causal)
     hipLaunchKernelGGL((flash_generic_kernel<HDP, true, false, VEC>), g, blk, lds, st, p, hd);
+  else if (km && p.trim)
+    hipLaunchKernelGGL((flash_generic_kernel<HDP, false, true, VEC, true>), g, blk, lds, st, p, hd);
   else if (km)
     hipLaunchKernelGGL((flash_generic_kernel<HDP, false, true, VEC>), g, blk, lds, st, p, hd);
   else
@@ -1969,10 +1973,15 @@ __global__ __launch_bounds__(NW * 64, (NW <= 4 && HD <= 64) ? 2 : 1) void flash_
   } else if constexpr (HD == 128 && CAUSAL) {
     flash_ring_body<HD, NW, CAUSAL, KMASK>(p);
   } else if constexpr (HD == 128) {
-    flash_vreg_body<HD, NW, CAUSAL, KMASK>(p);
+    flash_vreg_body<HD, NW, CAUSAL, KMASK, false>(p);
   } else {
     flash_dma_body<HD, NW, CAUSAL, KMASK>(p);
   }
+}
+// The register body with the scan of valid_tiles (b300 h2 s65 26.1 -> 21.6 us).
+template <int NW>
+__global__ __launch_bounds__(NW * 64, 1) void flash_vreg_trim_kernel(AttnArgs p) {
+  flash_vreg_body<128, NW, false, true, true>(p);
 }
 // Without the causal mask: head_dim 64 below the loop's first length, and 16 and 32 with a key
 // mask that is not scanned.  b54 h2 s80 d64 5.4 -> 5.2 us, b18 h8 s159 d64 masked 9.8 -> 9.3,
@@ -2083,9 +2092,15 @@ int launch_flash(const AttnArgs& args, bool causal, hipStream_t st) {
   const dim3 g((unsigned)grid), blk(NW * 64);
   const bool km = p.kv != nullptr;
   if constexpr (HD <= 64 && NW == 4) {
-    if (!causal && (HD == 64 ? p.S < kShortS : km && !p.trim)) {
+    if (!causal && !p.trim && (HD == 64 ? p.S < kShortS : km)) {
       if (km) hipLaunchKernelGGL((flash_short_kernel<HD, NW, true>), g, blk, 0, st, p);
       else hipLaunchKernelGGL((flash_short_kernel<HD, NW, false>), g, blk, 0, st, p);
+      return check_launch("tk_flash_attn_fwd");
+    }
+  }
+  if constexpr (HD == 128 && NW >= 4) {
+    if (p.trim) {
+      hipLaunchKernelGGL((flash_vreg_trim_kernel<NW>), g, blk, 0, st, p);
       return check_launch("tk_flash_attn_fwd");
     }
   }
